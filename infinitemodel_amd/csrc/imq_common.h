@@ -227,6 +227,19 @@ IMQ_DEV void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::
 
 static inline int64_t imq_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// n / d for n < 2^31 without a division: mul = floor(2^(31 + l) / d) + 1 with l = ceil(log2 d), so
+// n mul >> (31 + l) is the exact quotient (d = 1 passes n through).
+struct FastDiv {
+  uint32_t d, mul, sh;
+};
+inline FastDiv fast_div(uint32_t d) {
+  if (d <= 1) return FastDiv{1, 0, 0};
+  uint32_t l = 0;
+  while ((1ull << l) < d) ++l;
+  return FastDiv{d, (uint32_t)((1ull << (31 + l)) / d) + 1, l - 1};
+}
+IMQ_DEV uint32_t div_fast(uint32_t n, const FastDiv& f) { return f.d == 1 ? n : __umulhi(n, f.mul) >> f.sh; }
+
 // Host-side launch error check: hipGetLastError after a launch, mapped to an int status.
 #define IMQ_LAUNCH_CHECK()                                   \
   do {                                                       \

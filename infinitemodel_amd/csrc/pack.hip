@@ -13,114 +13,290 @@
 // Per-row symmetric (int8), in W's own dtype: scale = max(dt(amax|w| / 127), dt(1e-8)),
 // q = clamp(rint(dt(w / scale)), -127, 127) -- the quotient is rounded to dt before rint.
 #include <algorithm>
+#include <type_traits>
 
 #include "imq_common.h"
 
 namespace {
 
+// 8 consecutive elements of a weight row as fp32 (exact widening): two 16-byte loads for fp32, one for
+// the 16-bit types.
 template <int DT>
-IMQ_DEV float load_w(const void* p, int64_t idx) { return load_as_f32<DT>(p, idx); }
-
-// One wave per (row, group) item, grid-strided; a lane holds EPL = G / 64 consecutive columns.
-template <int BITS, int DT, int EPL>
-__global__ __launch_bounds__(256) void pack_g_kernel(const void* __restrict__ W, int64_t sw, int64_t N,
-                                                     int64_t in_f, int ng, uint8_t* __restrict__ q, int64_t sq,
-                                                     void* __restrict__ sc, void* __restrict__ zr, int64_t ssn) {
-  constexpr int G = 64 * EPL;
-  constexpr float QMAX = (float)((1 << BITS) - 1);
-  constexpr int CPB = 8 / BITS;                        // codes per byte
-  __shared__ uint8_t codes[4][G];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t items = N * ng;
-  for (int64_t it = (int64_t)blockIdx.x * 4 + wave; it < items; it += (int64_t)gridDim.x * 4) {
-    const int64_t n = it / ng;
-    const int g = (int)(it - n * ng);
-    const int64_t k0 = (int64_t)g * G + lane * EPL;
-    float v[EPL];
-    float lo = 0.f, hi = 0.f;
+struct Raw8 {
+  u32x4_t d[DT == IMQ_DT_FP32 ? 2 : 1];
+};
+template <int DT>
+IMQ_DEV void load8(Raw8<DT>& r, const void* p, int64_t idx) {
+  const u32x4_t* s = (const u32x4_t*)((const char*)p + idx * (DT == IMQ_DT_FP32 ? 4 : 2));
+  r.d[0] = s[0];
+  if constexpr (DT == IMQ_DT_FP32) r.d[1] = s[1];
+}
+template <int DT>
+IMQ_DEV float get8(const Raw8<DT>& r, int e) {
+  if constexpr (DT == IMQ_DT_FP32) {
+    const uint32_t w = r.d[e >> 2][e & 3];
+    return __uint_as_float(w);
+  } else {
+    const uint32_t w = r.d[0][e >> 1];
+    return raw_bits_to_f32<DT>((e & 1) ? (w >> 16) : (w & 0xffffu));
+  }
+}
+// The row's elements [k, k + 8), zero past `end`; vec: the row is 16-byte aligned (k a multiple of 8).
+template <int DT>
+IMQ_DEV void load8_row(Raw8<DT>& r, const void* W, int64_t row, int64_t k, int64_t end, bool vec) {
+  if (vec && k + 8 <= end) {
+    load8<DT>(r, W, row + k);
+    return;
+  }
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      v[e] = (k0 + e < in_f) ? load_w<DT>(W, n * sw + k0 + e) : 0.f;
-      lo = e == 0 ? v[e] : fminf(lo, v[e]);
-      hi = e == 0 ? v[e] : fmaxf(hi, v[e]);
+  for (int i = 0; i < (DT == IMQ_DT_FP32 ? 8 : 4); ++i) {
+    uint32_t w = 0;
+    if constexpr (DT == IMQ_DT_FP32) {
+      if (k + i < end) w = load_raw_bits<DT>(W, row + k + i);
+    } else {
+      if (k + 2 * i < end) w = load_raw_bits<DT>(W, row + k + 2 * i);
+      if (k + 2 * i + 1 < end) w |= load_raw_bits<DT>(W, row + k + 2 * i + 1) << 16;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      lo = fminf(lo, __shfl_xor(lo, off, 64));
-      hi = fmaxf(hi, __shfl_xor(hi, off, 64));
-    }
-    float s = (hi - lo) / QMAX;
-    s = s < 1e-8f ? 1e-8f : s;
-    float z = rintf(-lo / s);
-    z = z < 0.f ? 0.f : z;
-    z = z > QMAX ? QMAX : z;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      float t = rintf(v[e] / s + z);
-      t = t < 0.f ? 0.f : t;
-      t = t > QMAX ? QMAX : t;
-      codes[wave][lane * EPL + e] = (uint8_t)(int)t;
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // codes visible to the wave's lanes
-    constexpr int NB = G / CPB;                               // packed bytes of the group
-    for (int b = lane; b < NB; b += 64) {
-      uint32_t byte = 0;
-#pragma unroll
-      for (int j = 0; j < CPB; ++j) byte |= (uint32_t)codes[wave][b * CPB + j] << (BITS * j);
-      q[n * sq + (int64_t)g * NB + b] = (uint8_t)byte;
-    }
-    if (lane == 0) {
-      store_from_f32<DT>(sc, n * ssn + g, s);
-      store_from_f32<DT>(zr, n * ssn + g, z);
-    }
-    __builtin_amdgcn_wave_barrier();                          // codes reused by the next item
+    r.d[i >> 2][i & 3] = w;
   }
 }
 
-// One wave per row: |w| max over the row, then the codes.
-template <int DT>
+// Correctly rounded v / s from r = the correctly rounded 1 / s (Markstein's division: one Newton step
+// makes v r a faithful quotient, and the exact remainder of a faithful quotient rounds it correctly):
+// 5 VALU operations against the ~10 of the IEEE division sequence, whose reciprocal and scaling a
+// group's elements share. Exact for s in [2^-60, 2^60] and |v| <= 2^60 (no step overflows; where a tiny
+// v lets the remainder underflow the quotient is below 2^-30, which neither the add of the integer
+// zero point nor the rint that follow can see); other groups take the IEEE division.
+IMQ_DEV float div_by(float v, float s, float r) {
+  float q = v * r;
+  q = fmaf(fmaf(-q, s, v), r, q);
+  return fmaf(fmaf(-q, s, v), r, q);
+}
+IMQ_DEV bool div_by_exact(float s, float vmax) {
+  return s >= 0x1p-60f && s <= 0x1p60f && vmax <= 0x1p60f;   // false for NaN
+}
+
+// A lane holds 16 consecutive columns of one group, G / 16 neighbouring lanes a whole group, a wave
+// 1024 / G groups in row-major group order (so short rows leave no lane idle). HBM-bound by design:
+// two 16-byte loads and one 8- or 4-byte packed store per lane, min / max by lane exchanges inside the
+// group, two divisions per group and 5 operations per element instead of an IEEE division for each
+// (the kernel that gave a wave one group, two elements a lane through LDS, was bound by those
+// divisions and by its 4-byte loads). 4096 -> 28672 bf16 int4: 272 -> 64 us, 4.6 TB/s of reads and
+// writes (a plain device copy: 4.8).
+template <int BITS, int DT, int G>
+__global__ __launch_bounds__(256) void pack_g_kernel(const void* __restrict__ W, int64_t sw, uint32_t groups,
+                                                     int64_t in_f, FastDiv ngd, uint8_t* __restrict__ q, int64_t sq,
+                                                     void* __restrict__ sc, void* __restrict__ zr, int64_t ssn,
+                                                     bool wvec, bool qvec) {
+  constexpr float QMAX = (float)((1 << BITS) - 1);
+  constexpr int LPG = G / 16;                          // lanes of a group
+  constexpr int NB = G * BITS / 8;                     // packed bytes of a group
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t gid0 = t / LPG;
+  const int part = (int)(t % LPG);
+  const bool live = gid0 < groups;
+  const uint32_t gid = live ? gid0 : groups - 1;       // past the end: repeats the last group, stores nothing
+  const uint32_t n = div_fast(gid, ngd);
+  const uint32_t g = gid - n * ngd.d;
+  const int64_t row = (int64_t)n * sw;
+  const int64_t k0 = (int64_t)g * G + part * 16;
+  Raw8<DT> raw[2];
+  load8_row<DT>(raw[0], W, row, k0, in_f, wvec);
+  load8_row<DT>(raw[1], W, row, k0 + 8, in_f, wvec);
+  float v[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) v[e] = get8<DT>(raw[e >> 3], e & 7);
+  float lo = v[0], hi = v[0];
+#pragma unroll
+  for (int e = 1; e < 16; ++e) {
+    lo = fminf(lo, v[e]);
+    hi = fmaxf(hi, v[e]);
+  }
+#pragma unroll
+  for (int off = LPG / 2; off > 0; off >>= 1) {
+    lo = fminf(lo, __shfl_xor(lo, off, 64));
+    hi = fmaxf(hi, __shfl_xor(hi, off, 64));
+  }
+  float s = (hi - lo) / QMAX;
+  s = s < 1e-8f ? 1e-8f : s;
+  const float r = 1.f / s;
+  const bool fast = div_by_exact(s, fmaxf(fabsf(lo), fabsf(hi)));
+  float z = rintf(-lo / s);                            // IEEE: keeps the -0.0 of a group whose least value is 0
+  z = z < 0.f ? 0.f : z;
+  z = z > QMAX ? QMAX : z;
+  if (!fast) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = v[e] / s;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = div_by(v[e], s, r);
+  }
+  // clamp(rint(t)) == rint(clamp(t)) for the integer bounds; adding 2^23 rounds to an integer (half to
+  // even) and leaves it in the low mantissa bits. A NaN becomes code 0 (fmaxf returns the other operand).
+  uint32_t d[BITS / 2] = {};                           // 16 codes: 2 dwords of int4, 1 of int2
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const float c = fminf(fmaxf(v[e] + z, 0.f), QMAX) + 0x1p23f;
+    d[e * BITS / 32] |= (__float_as_uint(c) & ((1u << BITS) - 1u)) << (e * BITS & 31);
+  }
+  if (!live) return;
+  uint8_t* dst = q + (int64_t)n * sq + (int64_t)g * NB + part * (2 * BITS);
+  if (qvec) {
+    if constexpr (BITS == 4) *(u32x2_t*)dst = u32x2_t{d[0], d[1]};
+    else *(uint32_t*)dst = d[0];
+  } else {
+#pragma unroll
+    for (int b = 0; b < 2 * BITS; ++b) dst[b] = (uint8_t)(d[b >> 2] >> (8 * (b & 3)));
+  }
+  if (part == 0) {
+    store_from_f32<DT>(sc, (int64_t)n * ssn + g, s);
+    store_from_f32<DT>(zr, (int64_t)n * ssn + g, z);
+  }
+}
+
+// WPR waves per row (1 or 4), 8 columns per lane and pass: the row's |w| max, then the codes. The
+// first NV passes keep the row in registers, so rows up to 512 NV WPR columns are read once (longer
+// ones re-read their tail); divisions as in pack_g_kernel, one shared reciprocal per row. 4096 -> 14336 bf16:
+// 39 us, 4.5 TB/s (one wave per row with 2-byte loads and a division per element: 118 us).
+template <int DT, int WPR, int NV>
 __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W, int64_t sw, int64_t N,
                                                       int64_t K, int8_t* __restrict__ q, int64_t sq,
-                                                      void* __restrict__ sc, int64_t ssn) {
+                                                      void* __restrict__ sc, int64_t ssn, bool wvec, bool qvec) {
+  constexpr int64_t STEP = 512 * WPR;                  // columns of a pass
+  __shared__ float part[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int64_t n = (int64_t)blockIdx.x * 4 + wave; n < N; n += (int64_t)gridDim.x * 4) {
-    float amax = 0.f;
-    for (int64_t k = lane; k < K; k += 64) amax = fmaxf(amax, fabsf(load_w<DT>(W, n * sw + k)));
+  const int64_t n0 = WPR == 1 ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
+  const bool live = n0 < N;
+  const int64_t n = live ? n0 : N - 1;
+  const int64_t row = n * sw, kl = 8 * (WPR == 1 ? lane : (int)threadIdx.x);
+  Raw8<DT> raw[NV];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    float s = round_to<DT>(amax / 127.f);
-    const float smin = round_to<DT>(1e-8f);
-    s = s < smin ? smin : s;
-    for (int64_t k = lane; k < K; k += 64) {
-      float t = rintf(round_to<DT>(load_w<DT>(W, n * sw + k) / s));
-      t = t < -127.f ? -127.f : t;                   // NaN (0 / 0 at an fp16 zero row) stays NaN
-      t = t > 127.f ? 127.f : t;
-      q[n * sq + k] = (int8_t)(t == t ? (int)t : 0);  // and converts to 0, as the host cast does
-    }
-    if (lane == 0) store_from_f32<DT>(sc, n * ssn, s);
+  for (int i = 0; i < NV; ++i) load8_row<DT>(raw[i], W, row, kl + i * STEP, K, wvec);
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(get8<DT>(raw[i], e)));
+  for (int64_t k = kl + NV * STEP; k < K; k += STEP) {
+    Raw8<DT> t;
+    load8_row<DT>(t, W, row, k, K, wvec);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(get8<DT>(t, e)));
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+  if constexpr (WPR == 4) {
+    if (lane == 0) part[wave] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  }
+  float s = round_to<DT>(amax / 127.f);
+  const float smin = round_to<DT>(1e-8f);
+  s = s < smin ? smin : s;
+  const float r = 1.f / s;
+  const bool fast = div_by_exact(s, amax);
+  auto emit = [&](auto fastc, const Raw8<DT>& w, int64_t k) {
+    constexpr bool FAST = decltype(fastc)::value;
+    if (k >= K || !live) return;
+    uint32_t d[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float v = get8<DT>(w, e);
+      float t = FAST ? div_by(v, s, r) : v / s;
+      if constexpr (DT == IMQ_DT_BF16) t = round_bf16_hw(t);
+      else t = round_to<DT>(t);
+      // the conversion saturates and takes a NaN (0 / 0 at an fp16 zero row) to 0, as the host cast does
+      int ci = __float2int_rn(t);
+      ci = ci < -127 ? -127 : ci > 127 ? 127 : ci;
+      d[e >> 2] |= ((uint32_t)ci & 0xffu) << (8 * (e & 3));
+    }
+    int8_t* dst = q + n * sq + k;
+    if (qvec && k + 8 <= K) {
+      *(u32x2_t*)dst = u32x2_t{d[0], d[1]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (k + e < K) dst[e] = (int8_t)(d[e >> 2] >> (8 * (e & 3)));
+    }
+  };
+  auto codes = [&](auto fastc) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) emit(fastc, raw[i], kl + i * STEP);
+    for (int64_t k = kl + NV * STEP; k < K; k += STEP) {
+      Raw8<DT> t;
+      load8_row<DT>(t, W, row, k, K, wvec);
+      emit(fastc, t, k);
+    }
+  };
+  if (fast) codes(std::true_type{});
+  else codes(std::false_type{});
+  if (live && lane == 0 && (WPR == 1 || wave == 0)) store_from_f32<DT>(sc, n * ssn, s);
 }
 
 bool dt_ok(int d) { return d == IMQ_DT_BF16 || d == IMQ_DT_FP16 || d == IMQ_DT_FP32; }
 
-unsigned grid_for(int64_t items) {
-  const int64_t b = (items + 3) / 4;
-  return (unsigned)(b < 65536 ? (b > 0 ? b : 1) : 65536);
+// Rows a launch covers so that its group ids (rows * ng) and threads stay below 2^31.
+int64_t rows_per_launch(int64_t per_row) {
+  const int64_t r = 0x7fffff00ll / per_row;
+  return r > 0 ? r : 1;
+}
+
+template <int BITS, int DT, int G>
+int launch_gg(const void* W, int64_t sw, int64_t N, int64_t in_f, uint8_t* q, int64_t sq, void* sc, void* zr,
+              int64_t ssn, hipStream_t st) {
+  constexpr int ES = DT == IMQ_DT_FP32 ? 4 : 2, LPG = G / 16;
+  const int64_t ng = (in_f + G - 1) / G;
+  if (ng * LPG > 0x7fffff00ll) return IMQ_ERR_UNSUPPORTED;
+  const bool wvec = ((uintptr_t)W & 15) == 0 && ((sw * ES) & 15) == 0;
+  const bool qvec = ((uintptr_t)q & (2 * BITS - 1)) == 0 && (sq & (2 * BITS - 1)) == 0;
+  const FastDiv ngd = fast_div((uint32_t)ng);
+  const int64_t step = rows_per_launch(ng * LPG);
+  for (int64_t n = 0; n < N; n += step) {
+    const int64_t rows = std::min(step, N - n);
+    const unsigned grid = (unsigned)((rows * ng * LPG + 255) / 256);
+    pack_g_kernel<BITS, DT, G><<<grid, 256, 0, st>>>((const char*)W + n * sw * ES, sw, (uint32_t)(rows * ng), in_f, ngd,
+                                                    q + n * sq, sq, (char*)sc + n * ssn * ES, (char*)zr + n * ssn * ES,
+                                                    ssn, wvec, qvec);
+    IMQ_LAUNCH_CHECK();
+  }
+  return IMQ_OK;
 }
 
 template <int BITS, int DT>
 int launch_g(const void* W, int64_t sw, int64_t N, int64_t in_f, int64_t G, uint8_t* q, int64_t sq, void* sc,
              void* zr, int64_t ssn, hipStream_t st) {
-  const int ng = (int)((in_f + G - 1) / G);
-  const unsigned grid = grid_for(N * ng);
   switch (G) {
-    case 64: pack_g_kernel<BITS, DT, 1><<<grid, 256, 0, st>>>(W, sw, N, in_f, ng, q, sq, sc, zr, ssn); break;
-    case 128: pack_g_kernel<BITS, DT, 2><<<grid, 256, 0, st>>>(W, sw, N, in_f, ng, q, sq, sc, zr, ssn); break;
-    case 256: pack_g_kernel<BITS, DT, 4><<<grid, 256, 0, st>>>(W, sw, N, in_f, ng, q, sq, sc, zr, ssn); break;
-    default: return IMQ_ERR_UNSUPPORTED;
+    case 64: return launch_gg<BITS, DT, 64>(W, sw, N, in_f, q, sq, sc, zr, ssn, st);
+    case 128: return launch_gg<BITS, DT, 128>(W, sw, N, in_f, q, sq, sc, zr, ssn, st);
+    case 256: return launch_gg<BITS, DT, 256>(W, sw, N, in_f, q, sq, sc, zr, ssn, st);
   }
-  IMQ_LAUNCH_CHECK();
+  return IMQ_ERR_UNSUPPORTED;
+}
+
+// A wave per row while the row fits one wave's registers (4096 columns), else four; NV passes cover
+// the row where they can.
+template <int DT>
+int launch_w8(const void* W, int64_t sw, int64_t N, int64_t K, int8_t* q, int64_t sq, void* sc, int64_t ssn,
+              hipStream_t st) {
+  constexpr int ES = DT == IMQ_DT_FP32 ? 4 : 2;
+  const bool wvec = ((uintptr_t)W & 15) == 0 && ((sw * ES) & 15) == 0;
+  const bool qvec = ((uintptr_t)q & 7) == 0 && (sq & 7) == 0;
+  const int64_t step = 1 << 22;                        // rows a launch: its threads stay below 2^31
+  for (int64_t n = 0; n < N; n += step) {
+    const int64_t rows = std::min(step, N - n);
+    const dim3 g((unsigned)(K <= 4096 ? (rows + 3) / 4 : rows)), b(256);
+    const void* Wn = (const char*)W + n * sw * ES;
+    void* scn = (char*)sc + n * ssn * ES;
+    int8_t* qn = q + n * sq;
+#define IMQ_P8(W_, V_) pack_w8_kernel<DT, W_, V_><<<g, b, 0, st>>>(Wn, sw, rows, K, qn, sq, scn, ssn, wvec, qvec)
+    if (K <= 1024) IMQ_P8(1, 2);
+    else if (K <= 2048) IMQ_P8(1, 4);
+    else if (K <= 4096) IMQ_P8(1, 8);
+    else if (K <= 8192) IMQ_P8(4, 4);
+    else IMQ_P8(4, 8);
+#undef IMQ_P8
+    IMQ_LAUNCH_CHECK();
+  }
   return IMQ_OK;
 }
 
@@ -233,13 +409,11 @@ extern "C" int imq_pack_w8(const void* W, int64_t w_row_stride, int w_dtype, int
   if (N < 0 || K <= 0 || w_row_stride < K || q_row_stride < K || s_stride_n < 1) return IMQ_ERR_INVALID;
   if (N == 0) return IMQ_OK;
   hipStream_t st = (hipStream_t)stream;
-  const unsigned grid = grid_for(N);
   int8_t* qb = (int8_t*)qweight;
   switch (w_dtype) {
-    case IMQ_DT_BF16: pack_w8_kernel<IMQ_DT_BF16><<<grid, 256, 0, st>>>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n); break;
-    case IMQ_DT_FP16: pack_w8_kernel<IMQ_DT_FP16><<<grid, 256, 0, st>>>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n); break;
-    case IMQ_DT_FP32: pack_w8_kernel<IMQ_DT_FP32><<<grid, 256, 0, st>>>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n); break;
+    case IMQ_DT_BF16: return launch_w8<IMQ_DT_BF16>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n, st);
+    case IMQ_DT_FP16: return launch_w8<IMQ_DT_FP16>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n, st);
+    case IMQ_DT_FP32: return launch_w8<IMQ_DT_FP32>(W, w_row_stride, N, K, qb, q_row_stride, scale, s_stride_n, st);
   }
-  IMQ_LAUNCH_CHECK();
-  return IMQ_OK;
+  return IMQ_ERR_INVALID;
 }
