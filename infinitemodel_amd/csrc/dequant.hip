@@ -3,73 +3,156 @@
 // These reproduce `_dequant(dtype)` of the reference modules exactly, rounding after every
 // elementwise op in the output dtype (worker_quant.py:638-648, 1652-1664, 439). They serve the
 // module's `_dequant` on the GPU (the naive path and the self-checks) and are the unit the
-// bit-exact parity tests pin. HBM-bound: each thread reads one packed word, writes 8 values.
+// bit-exact parity tests pin. HBM-bound (2 to 4 bytes written per code): a thread takes 8 codes, one
+// 2- to 8-byte load and one or two 16-byte stores, rows and groups found by multiplication instead
+// of 64-bit division, two codes rounded per v_cvt_pk_bf16_f32. 4096 -> 28672 int4 to bf16: 149
+// (byte loads, element stores, two 64-bit divisions per thread) -> 57 us, 5.2 TB/s.
+#include <algorithm>
+
 #include "imq_common.h"
 
 namespace {
 
-template <int BITS, int SDT, int ZDT, int ODT>
-__global__ __launch_bounds__(256) void dequant_g_kernel(
-    const uint8_t* __restrict__ q, int64_t sq, const void* __restrict__ sc, int64_t ssn, int64_t ssg,
-    const void* __restrict__ zr, int64_t szn, int64_t szg, int64_t N, int64_t in_f, int64_t G,
-    void* __restrict__ out, int64_t so, int64_t chunks_per_row) {
-  constexpr int CODES_PER_BYTE = 8 / BITS;
-  constexpr int BYTES_PER_CHUNK = 8 / CODES_PER_BYTE;   // 8 codes per thread
-  const int64_t total = N * chunks_per_row;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t n = t / chunks_per_row;
-    const int64_t c = t - n * chunks_per_row;
-    const int64_t k0 = c * 8;
-    const uint8_t* qp = q + n * sq + c * BYTES_PER_CHUNK;
-    uint32_t bits = 0;
+// fp32 values -> ODT, two per dword for the 16-bit types, round to nearest even. HW: the hardware pack
+// (bit-equal to store_from_f32 for every non-NaN value).
+template <int ODT, bool HW>
+IMQ_DEV uint32_t pack2(float a, float b) {
+  static_assert(ODT != IMQ_DT_FP32, "16-bit types");
+  if constexpr (ODT == IMQ_DT_FP16) return f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16);
+  else if constexpr (HW) return cvt_pk_bf16(a, b);
+  else return f32_to_bf16_bits(a) | (f32_to_bf16_bits(b) << 16);
+}
+
+// 8 results: d[i] = ODT(ODT(c[i] - z) * s) (ZERO) or ODT(c[i] * s), as the dwords of the row.
+template <int ODT, bool ZERO, bool HW>
+IMQ_DEV void dequant_values(const float* c, float s, float z, uint32_t* o) {
 #pragma unroll
-    for (int b = 0; b < BYTES_PER_CHUNK; ++b) bits |= (uint32_t)qp[b] << (8 * b);
-    // All 8 codes of a chunk share one group when G % 8 == 0 (always true: G is a multiple
-    // of the 8-code chunk for every format this library accepts; checked on the host).
-    const int64_t g = k0 / G;
-    const float z = round_to<ODT>(load_as_f32<ZDT>(zr, n * szn + g * szg));
-    const float s = round_to<ODT>(load_as_f32<SDT>(sc, n * ssn + g * ssg));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int64_t k = k0 + i;
-      if (k < in_f) {
-        const float code = (float)((bits >> (BITS * i)) & ((1u << BITS) - 1u));
-        const float d = round_to<ODT>(code - z);
-        const float w = round_to<ODT>(d * s);
-        store_from_f32<ODT>(out, n * so + k, w);
+  for (int i = 0; i < 8; i += 2) {
+    float a = c[i], b = c[i + 1];
+    if constexpr (ZERO) {
+      a -= z;
+      b -= z;
+      if constexpr (ODT != IMQ_DT_FP32) {
+        const uint32_t p = pack2<ODT, HW>(a, b);
+        a = raw_bits_to_f32<ODT>(p & 0xffffu);
+        b = raw_bits_to_f32<ODT>(p >> 16);
       }
+    }
+    if constexpr (ODT == IMQ_DT_FP32) {
+      o[i] = __float_as_uint(a * s);
+      o[i + 1] = __float_as_uint(b * s);
+    } else {
+      o[i / 2] = pack2<ODT, HW>(a * s, b * s);
     }
   }
 }
 
-template <int SDT, int ODT>
-__global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restrict__ q, int64_t sq,
-                                                         const void* __restrict__ sc, int64_t ssn,
-                                                         int64_t N, int64_t K, void* __restrict__ out,
-                                                         int64_t so) {
-  const int64_t total = N * K;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t n = t / K;
-    const int64_t k = t - n * K;
-    const float s = load_as_f32<SDT>(sc, n * ssn);
-    // q.to(x_dtype) is exact for |q| <= 127; one fp32 product, one rounding to the result dtype.
-    store_from_f32<ODT>(out, n * so + k, round_to<ODT>((float)q[n * sq + k] * s));
+// The 8 results at column k of an output row (elements past `end` are not written); vec: 16-byte
+// aligned rows.
+template <int ODT>
+IMQ_DEV void store8(void* out, int64_t row, int64_t k, int64_t end, const uint32_t* o, bool vec) {
+  if (vec && k + 8 <= end) {
+    u32x4_t* d = (u32x4_t*)((char*)out + (row + k) * (ODT == IMQ_DT_FP32 ? 4 : 2));
+    d[0] = u32x4_t{o[0], o[1], o[2], o[3]};
+    if constexpr (ODT == IMQ_DT_FP32) d[1] = u32x4_t{o[4], o[5], o[6], o[7]};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if (k + i >= end) break;
+    if constexpr (ODT == IMQ_DT_FP32) ((uint32_t*)out)[row + k + i] = o[i];
+    else ((uint16_t*)out)[row + k + i] = (uint16_t)(o[i >> 1] >> (16 * (i & 1)));
   }
 }
+
+// Thread t: codes [8 c, 8 c + 8) of row n, t = n * chunks + c. All 8 share one group (G is a
+// multiple of 8 for every format the library accepts; checked on the host).
+template <int BITS, int SDT, int ZDT, int ODT>
+__global__ __launch_bounds__(256) void dequant_g_kernel(
+    const uint8_t* __restrict__ q, int64_t sq, const void* __restrict__ sc, int64_t ssn, int64_t ssg,
+    const void* __restrict__ zr, int64_t szn, int64_t szg, uint32_t total, int64_t in_f, FastDiv chd, FastDiv gd,
+    void* __restrict__ out, int64_t so, bool qvec, bool ovec) {
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  if (t >= total) return;
+  const uint32_t n = div_fast(t, chd), c = t - n * chd.d, g = div_fast(c, gd);
+  const uint8_t* qp = q + (int64_t)n * sq + (int64_t)c * BITS;
+  uint32_t bits = 0;
+  if (qvec) {
+    if constexpr (BITS == 4) bits = *(const uint32_t*)qp;
+    else bits = *(const uint16_t*)qp;
+  } else {
+#pragma unroll
+    for (int b = 0; b < BITS; ++b) bits |= (uint32_t)qp[b] << (8 * b);
+  }
+  const float z = round_to<ODT>(load_as_f32<ZDT>(zr, (int64_t)n * szn + (int64_t)g * szg));
+  const float s = round_to<ODT>(load_as_f32<SDT>(sc, (int64_t)n * ssn + (int64_t)g * ssg));
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = (float)((bits >> (BITS * i)) & ((1u << BITS) - 1u));
+  uint32_t o[ODT == IMQ_DT_FP32 ? 8 : 4];
+  // finite scale and zero give no NaN (only overflow to infinity), which the two packs treat alike
+  if (__builtin_isfinite(s) && __builtin_isfinite(z)) dequant_values<ODT, true, true>(v, s, z, o);
+  else dequant_values<ODT, true, false>(v, s, z, o);
+  store8<ODT>(out, (int64_t)n * so, 8ll * c, in_f, o, ovec);
+}
+
+template <int SDT, int ODT>
+__global__ __launch_bounds__(256) void dequant_w8_kernel(const int8_t* __restrict__ q, int64_t sq,
+                                                         const void* __restrict__ sc, int64_t ssn, uint32_t total,
+                                                         int64_t K, FastDiv chd, void* __restrict__ out, int64_t so,
+                                                         bool qvec, bool ovec) {
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  if (t >= total) return;
+  const uint32_t n = div_fast(t, chd), c = t - n * chd.d;
+  const int8_t* qp = q + (int64_t)n * sq + 8ll * c;
+  uint32_t w[2] = {0u, 0u};
+  if (qvec && 8ll * c + 8 <= K) {
+    const u32x2_t p = *(const u32x2_t*)qp;
+    w[0] = p[0];
+    w[1] = p[1];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (8ll * c + i < K) w[i >> 2] |= (uint32_t)(uint8_t)qp[i] << (8 * (i & 3));
+  }
+  const float s = load_as_f32<SDT>(sc, (int64_t)n * ssn);
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = (float)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
+  uint32_t o[ODT == IMQ_DT_FP32 ? 8 : 4];
+  // q.to(x_dtype) is exact for |q| <= 127; one fp32 product, one rounding to the result dtype.
+  if (__builtin_isfinite(s)) dequant_values<ODT, false, true>(v, s, 0.f, o);
+  else dequant_values<ODT, false, false>(v, s, 0.f, o);
+  store8<ODT>(out, (int64_t)n * so, 8ll * c, K, o, ovec);
+}
+
+// Rows of `chunks` threads one launch covers (its threads stay below 2^31).
+inline int64_t rows_per_launch(int64_t chunks) { return std::max<int64_t>(1, 0x7fffff00ll / chunks); }
+
+template <int DT>
+constexpr int esize() { return DT == IMQ_DT_FP32 ? 4 : 2; }
 
 template <int BITS, int SDT, int ZDT, int ODT>
 int launch_g(const void* q, int64_t sq, const void* sc, int64_t ssn, int64_t ssg, const void* zr,
              int64_t szn, int64_t szg, int64_t N, int64_t in_f, int64_t G, void* out, int64_t so,
              hipStream_t st) {
-  const int64_t kpad_chunks = imq_cdiv(in_f, 8);
-  const int64_t total = N * kpad_chunks;
-  if (total == 0) return IMQ_OK;
-  const int64_t blocks = imq_cdiv(total, 256) < 65536 ? imq_cdiv(total, 256) : 65536;
-  dequant_g_kernel<BITS, SDT, ZDT, ODT><<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
-      (const uint8_t*)q, sq, sc, ssn, ssg, zr, szn, szg, N, in_f, G, out, so, kpad_chunks);
-  IMQ_LAUNCH_CHECK();
+  const int64_t chunks = imq_cdiv(in_f, 8);
+  if (N == 0 || chunks == 0) return IMQ_OK;
+  if (chunks > 0x7fffff00ll) return IMQ_ERR_UNSUPPORTED;
+  constexpr int OES = esize<ODT>(), QA = BITS == 4 ? 4 : 2;
+  const bool qvec = ((uintptr_t)q % QA) == 0 && sq % QA == 0;
+  const bool ovec = ((uintptr_t)out & 15) == 0 && ((so * OES) & 15) == 0;
+  const FastDiv chd = fast_div((uint32_t)chunks), gd = fast_div((uint32_t)std::min<int64_t>(G / 8, 0x7fffffff));
+  const int64_t step = rows_per_launch(chunks);
+  for (int64_t n = 0; n < N; n += step) {
+    const int64_t rows = std::min(step, N - n);
+    const uint32_t total = (uint32_t)(rows * chunks);
+    dequant_g_kernel<BITS, SDT, ZDT, ODT><<<dim3((total + 255u) / 256u), dim3(256), 0, st>>>(
+        (const uint8_t*)q + n * sq, sq, (const char*)sc + n * ssn * esize<SDT>(), ssn, ssg,
+        (const char*)zr + n * szn * esize<ZDT>(), szn, szg, total, in_f, chd, gd, (char*)out + n * so * OES, so, qvec,
+        ovec);
+    IMQ_LAUNCH_CHECK();
+  }
   return IMQ_OK;
 }
 
@@ -112,27 +195,38 @@ int dequant_g(const void* q, int64_t sq, const void* sc, int64_t ssn, int64_t ss
   return IMQ_ERR_INVALID;
 }
 
+template <int SDT, int ODT>
+int launch_w8(const int8_t* q, int64_t sq, const void* sc, int64_t ssn, int64_t N, int64_t K, void* out, int64_t so,
+              hipStream_t st) {
+  const int64_t chunks = imq_cdiv(K, 8);
+  if (N == 0 || chunks == 0) return IMQ_OK;
+  if (chunks > 0x7fffff00ll) return IMQ_ERR_UNSUPPORTED;
+  constexpr int OES = esize<ODT>();
+  const bool qvec = ((uintptr_t)q & 7) == 0 && (sq & 7) == 0;
+  const bool ovec = ((uintptr_t)out & 15) == 0 && ((so * OES) & 15) == 0;
+  const FastDiv chd = fast_div((uint32_t)chunks);
+  const int64_t step = rows_per_launch(chunks);
+  for (int64_t n = 0; n < N; n += step) {
+    const int64_t rows = std::min(step, N - n);
+    const uint32_t total = (uint32_t)(rows * chunks);
+    dequant_w8_kernel<SDT, ODT><<<dim3((total + 255u) / 256u), dim3(256), 0, st>>>(
+        q + n * sq, sq, (const char*)sc + n * ssn * esize<SDT>(), ssn, total, K, chd, (char*)out + n * so * OES, so,
+        qvec, ovec);
+    IMQ_LAUNCH_CHECK();
+  }
+  return IMQ_OK;
+}
+
 template <int SDT>
 int dequant8_out(int odt, const void* q, int64_t sq, const void* sc, int64_t ssn, int64_t N, int64_t K,
                  void* out, int64_t so, hipStream_t st) {
-  const int64_t total = N * K;
-  if (total == 0) return IMQ_OK;
-  const int64_t blocks = imq_cdiv(total, 256) < 65536 ? imq_cdiv(total, 256) : 65536;
+  const int8_t* qb = (const int8_t*)q;
   switch (odt) {
-    case IMQ_DT_BF16:
-      dequant_w8_kernel<SDT, IMQ_DT_BF16><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const int8_t*)q, sq, sc, ssn, N, K, out, so);
-      break;
-    case IMQ_DT_FP16:
-      dequant_w8_kernel<SDT, IMQ_DT_FP16><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const int8_t*)q, sq, sc, ssn, N, K, out, so);
-      break;
-    case IMQ_DT_FP32:
-      dequant_w8_kernel<SDT, IMQ_DT_FP32><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const int8_t*)q, sq, sc, ssn, N, K, out, so);
-      break;
-    default:
-      return IMQ_ERR_INVALID;
+    case IMQ_DT_BF16: return launch_w8<SDT, IMQ_DT_BF16>(qb, sq, sc, ssn, N, K, out, so, st);
+    case IMQ_DT_FP16: return launch_w8<SDT, IMQ_DT_FP16>(qb, sq, sc, ssn, N, K, out, so, st);
+    case IMQ_DT_FP32: return launch_w8<SDT, IMQ_DT_FP32>(qb, sq, sc, ssn, N, K, out, so, st);
   }
-  IMQ_LAUNCH_CHECK();
-  return IMQ_OK;
+  return IMQ_ERR_INVALID;
 }
 
 }  // namespace
