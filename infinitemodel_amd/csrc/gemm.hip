@@ -102,32 +102,6 @@ IMQ_DEV int swz(int row, int c) {
   return (row * C::CH + (c ^ ((row >> C::SH) & (C::CH - 1)))) * 8;
 }
 
-// 8 codes (BITS 4: nibbles of a dword; BITS 2: crumbs in the low 16 bits) -> 4 dwords of bf16
-// (c - z) * s in K order.
-template <int BITS>
-IMQ_DEV u32x4_t dequant8(uint32_t w, float s, float nzs) {
-  u32x4_t r;
-  if constexpr (BITS == 4) {
-    // even codes in the bytes of lo, odd codes in the bytes of hi: each code is then one
-    // v_cvt_f32_ubyteN away from fp32
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float c0 = (float)((lo >> (8 * i)) & 0xffu);
-      const float c1 = (float)((hi >> (8 * i)) & 0xffu);
-      r[i] = cvt_pk_bf16(fmaf(c0, s, nzs), fmaf(c1, s, nzs));
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float c0 = (float)((w >> (4 * i)) & 3u);
-      const float c1 = (float)((w >> (4 * i + 2)) & 3u);
-      r[i] = cvt_pk_bf16(fmaf(c0, s, nzs), fmaf(c1, s, nzs));
-    }
-  }
-  return r;
-}
-
 // 8 int8 codes (two dwords) -> 4 dwords of bf16, exact.
 IMQ_DEV u32x4_t convert8_i8(uint32_t lo, uint32_t hi) {
   u32x4_t r;
@@ -175,9 +149,9 @@ IMQ_DEV void load_w(WRegs<BITS, WC>& r, const uint8_t* p) {
 template <int BITS, int WC>
 IMQ_DEV u32x4_t weight_chunk(const WRegs<BITS, WC>& r, int c, float s, float nzs) {
   if constexpr (BITS == 4) {
-    return dequant8<4>(r.d[c], s, nzs);
+    return dequant8_bf16<4>(r.d[c], 0, s, nzs);
   } else if constexpr (BITS == 2) {
-    return dequant8<2>(r.d[c >> 1] >> (16 * (c & 1)), s, nzs);
+    return dequant8_bf16<2>(r.d[c >> 1], c & 1, s, nzs);
   } else {
     return convert8_i8(r.d[2 * c], r.d[2 * c + 1]);
   }

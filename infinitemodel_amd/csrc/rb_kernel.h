@@ -36,9 +36,11 @@ namespace {
 constexpr int RB_GROUP_M = 8;
 constexpr int RB_BK = 64;
 // VALU instructions the scheduler places after each MFMA (int4 dequant / int8 conversion work):
-// chosen per format as the pattern that keeps the 256-row variants within the register file.
+// chosen per format as the pattern that keeps the 256-row variants within the register file and
+// spreads a slice's work (about 2.7 per MFMA for int4) evenly. int4 4096 <-> 14336 at M = 2048, both
+// linears: 488 / 486 / 478 / 489 us at 5 / 4 / 3 / 2; 535 with v_cvt_f32_ubyteN at 5.
 #ifndef RB_VALU_PER_MFMA_4
-#define RB_VALU_PER_MFMA_4 5
+#define RB_VALU_PER_MFMA_4 3
 #endif
 #ifndef RB_VALU_PER_MFMA_8
 #define RB_VALU_PER_MFMA_8 3
@@ -127,30 +129,6 @@ template <int DT>
 IMQ_DEV uint32_t rb_bload_raw(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   if constexpr (DT == IMQ_DT_FP32) return __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0);
   else return __builtin_amdgcn_raw_buffer_load_b16(r, (int)voff, (int)soff, 0);
-}
-
-// w & m computed in a register the compiler cannot see through, so the byte extractions below
-// stay single v_cvt_f32_ubyteN instructions instead of being re-folded into per-nibble bit-field
-// extracts (the result only feeds VALU conversions, never an MFMA operand directly).
-IMQ_DEV uint32_t rb_and(uint32_t w, uint32_t m) {
-  uint32_t r;
-  asm("v_and_b32 %0, %1, %2" : "=v"(r) : "v"(w), "v"(m));
-  return r;
-}
-
-// 8 int4 codes of one dword (code i at bits 4i) -> 4 dwords of bf16 (c - z) s in K order: the
-// even codes sit in the bytes of lo, the odd ones in the bytes of hi, each one v_cvt_f32_ubyteN
-// from fp32; fma(c, s, -z s) is the exact (c - z) s, rounded once by the pack.
-IMQ_DEV u32x4_t rb_dequant4(uint32_t w, float s, float nzs) {
-  const uint32_t lo = rb_and(w, 0x0F0F0F0Fu), hi = rb_and(w >> 4, 0x0F0F0F0Fu);
-  u32x4_t r;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float c0 = (float)((lo >> (8 * i)) & 0xffu);
-    const float c1 = (float)((hi >> (8 * i)) & 0xffu);
-    r[i] = cvt_pk_bf16(fmaf(c0, s, nzs), fmaf(c1, s, nzs));
-  }
-  return r;
 }
 
 // 8 int8 codes (two dwords) -> 4 dwords of bf16, exact.
@@ -298,7 +276,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
   const uint8_t* qb[2];
   int64_t sb[2], zb[2];
   uint32_t qvo[2], svo[2], zvo[2];                  // BUF: byte offsets from the tile's rows
-  uint32_t qto[2][2] = {{0u, 0u}, {0u, 0u}};        // line-tiled weights: lane offsets by (kt / 2) & 1
+  uint32_t qto[2] = {0u, 0u};                       // line-tiled weights: lane offsets at sel 0
   constexpr int SES = SDT == IMQ_DT_FP32 ? 4 : 2, ZES = ZDT == IMQ_DT_FP32 ? 4 : 2;
   const int gh = (32 * h) >> a.gsh;                 // the lane half's group within a step (groups < 64)
 #pragma unroll
@@ -316,11 +294,11 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
       // rr / 16, half hr = (rr / 8) & 1, slot (rr & 7) + 8 (sel ^ hr) + 16 (piece & 3) of the
       // step's line-step. int4 (16 bytes at 32 kt + 16 h): line-step kt / 4, piece 2 (kt & 1) + h,
       // sel = (kt / 2) & 1; int8 (two pieces at 64 kt + 32 h + 16 v): line-step kt / 2, piece 2 h
-      // + v, sel = kt & 1. A lane offset per value of sel plus the step's uniform part (rb_tl_step).
+      // + v, sel = kt & 1. sel moves the slot by 8, bit 7 of the byte offset (nothing else reaches that
+      // bit: 16 rows are a multiple of 2048 bytes), so a lane keeps one offset and xors sel << 7 into it.
       const int rr = n - n0, hr = (rr >> 3) & 1;
       const uint32_t tb = (uint32_t)((rr >> 4) * 16 * (int)a.sqn + 1024 * hr + 16 * (rr & 7) + (BITS == 8 ? 512 : 256) * h);
-      qto[j][0] = tb + 128 * hr;
-      qto[j][1] = tb + 128 * (1 - hr);
+      qto[j] = tb + 128 * hr;
     }
   }
   // (built unconditionally; the forms that do not use them drop them)
@@ -482,10 +460,10 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if constexpr (TL) {
-          const int sel = BITS == 8 ? (kt & 1) : ((kt >> 1) & 1);
+          const uint32_t sx = (BITS == 8 ? (kt & 1) : ((kt >> 1) & 1)) << 7;
           const uint32_t so = BITS == 8 ? 2048 * (kt >> 1) : 2048 * (kt >> 2) + 512 * (kt & 1);
 #pragma unroll
-          for (int v = 0; v < QV; ++v) qr[set][j][v] = rb_bload128(qrs, (sel ? qto[j][1] : qto[j][0]) + 256 * v, so);
+          for (int v = 0; v < QV; ++v) qr[set][j][v] = rb_bload128(qrs, (qto[j] ^ sx) + 256 * v, so);
         } else {
 #pragma unroll
           for (int v = 0; v < QV; ++v) qr[set][j][v] = rb_bload128(qrs, qvo[j] + 16 * v, kt * (BK * BITS / 8));
@@ -500,11 +478,11 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if constexpr (TL) {
-        const int sel = BITS == 8 ? (kt & 1) : ((kt >> 1) & 1);
+        const uint32_t sx = (BITS == 8 ? (kt & 1) : ((kt >> 1) & 1)) << 7;
         const uint32_t so = BITS == 8 ? 2048 * (kt >> 1) : 2048 * (kt >> 2) + 512 * (kt & 1);
 #pragma unroll
         for (int v = 0; v < QV; ++v)
-          qr[set][j][v] = *(const u32x4_t*)(a.q + (int64_t)n0 * a.sqn + (sel ? qto[j][1] : qto[j][0]) + 256 * v + so);
+          qr[set][j][v] = *(const u32x4_t*)(a.q + (int64_t)n0 * a.sqn + (qto[j] ^ sx) + 256 * v + so);
       } else {
 #pragma unroll
         for (int v = 0; v < QV; ++v) qr[set][j][v] = *(const u32x4_t*)(qb[j] + kt * (BK * BITS / 8) + 16 * v);
@@ -584,7 +562,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
     if constexpr (FOLD) return unpack_nib8_bf16(qr[bs][j][0][s], magic);
     u32x4_t d;
     if constexpr (BITS == 8) d = rb_convert8(qr[bs][j][s >> 1][2 * (s & 1)], qr[bs][j][s >> 1][2 * (s & 1) + 1]);
-    else d = rb_dequant4(qr[bs][j][0][s], sv, nz);
+    else d = dequant8_bf16<4>(qr[bs][j][0][s], 0, sv, nz);
     return __builtin_bit_cast(bf16x8_t, d);
   };
 
