@@ -318,6 +318,8 @@ int imq_gptq_int2_solve(float* W, int64_t ldw, int64_t out, int64_t in_f, const 
  *     IMQ_PLAN_GEMM       LDS-dequant GEMM: p1 tile rows, p2 tile columns, p3 K splits
  *     IMQ_PLAN_GEMM_RB    register-B GEMM (int4 with group_size, int8 when it is 0):
  *                         p1 32-row blocks per wave, p2 K splits
+ *     IMQ_PLAN_GEMM_WK    short-batch GEMM (16 < M <= 64; the format by q_row_stride, dense rows):
+ *                         p1 32-column blocks per workgroup, p2 K ranges
  * Returns IMQ_OK, or IMQ_ERR_INVALID for an unknown kind or a null pointer. */
 #define IMQ_PLAN_W4_LINE 1
 #define IMQ_PLAN_W4_KSPLIT 2
@@ -328,6 +330,7 @@ int imq_gptq_int2_solve(float* W, int64_t ldw, int64_t out, int64_t in_f, const 
 #define IMQ_PLAN_W8_LINE 7
 #define IMQ_PLAN_GEMM 8
 #define IMQ_PLAN_GEMM_RB 9
+#define IMQ_PLAN_GEMM_WK 10
 int imq_launch_plan(int kind, const int64_t* in, int64_t* out);
 
 #ifdef __cplusplus

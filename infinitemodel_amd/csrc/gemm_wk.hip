@@ -1,0 +1,103 @@
+// The short-batch GEMM (gemm_wk.h): plan and dispatch.
+#include "gemm_wk.h"
+#include "splitk_sum.h"
+
+#include <algorithm>
+
+namespace imq {
+
+int wk_run4(const WkArgs& a, int jb, bool tiled, hipStream_t st);
+int wk_run2(const WkArgs& a, int jb, bool tiled, hipStream_t st);
+int wk_run8(const WkArgs& a, int jb, bool tiled, hipStream_t st);
+
+namespace {
+
+// The scale groups are powers of two >= 32 codes (int8: one per row, no shift).
+int wk_gsh(int bits, int64_t G) {
+  int gsh = 0;
+  if (bits != 8)
+    while ((1ll << gsh) < G) ++gsh;
+  return gsh;
+}
+
+// Column blocks and K ranges of a call, the cheapest by a model fitted to a sweep of both over int4 / int8 /
+// int2 linears of 2944 to 28672 columns and 768 to 28672 codes (it picks the measured best or one within
+// 4% of it): a wave's steps cost 0.8 / 1.4 / 2.4 us at 1 / 2 / 4 column blocks (32 rows; 1.35 / 2.1 at 64)
+// while the workgroups fit the CUs and in proportion to their number past that; a split costs the
+// sum's launch (4.5 us with its gap) and its fp32 planes (written and read). 4096 -> 28672: 4 blocks, whole K; 14336 ->
+// 4096: 2 blocks, 4 ranges (16.8 us against 18.7 for 1 block in 2); 4096 -> 4096: 1 block, whole K.
+bool wk_plan(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int max_splits, WkPlan* p) {
+  const int ib = M <= 32 ? 1 : 2, KT = (int)(K / RB_BK), gsh = wk_gsh(bits, G);
+  double best = 0;
+  p->splits = 0;
+  for (int jb = 1; jb <= (ib == 1 && bits != 8 ? 4 : 2); jb *= 2) {
+    const int64_t T = imq_cdiv(N, 32 * jb);
+    for (int s = 1; s <= max_splits; ++s) {
+      const int kps = (KT + s - 1) / s;
+      if (s > 1 && ((s - 1) * kps >= KT || kps < 2 * WK_WAVES || T * s > 2 * cus)) break;
+      if (wk_lds_bytes(bits, ib, jb, kps, gsh) > (size_t)max_lds) continue;
+      const double per = ib == 1 ? (jb == 1 ? 0.8 : jb == 2 ? 1.4 : 2.4) : (jb == 1 ? 1.35 : 2.1);
+      const double fill = (double)(T * s) / cus;
+      const double us = (fill > 1 ? fill : 1) * ((kps + WK_WAVES - 1) / WK_WAVES) * per +
+                        (s > 1 ? 4.5 + 8e-6 / 4 * s * M * N : 0);
+      if (p->splits == 0 || us < best) {
+        best = us;
+        *p = WkPlan{jb, s};
+      }
+    }
+  }
+  return p->splits != 0;
+}
+
+}  // namespace
+
+// The short-batch GEMM's plan of an M x N x K call (int8 when G is 0) on a device of `cus` CUs, without a
+// device: out = {takes the call, 32-column blocks per workgroup, K ranges}.
+void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out) {
+  WkPlan p{0, 0};
+  const bool takes = M > 16 && M <= 64 && K % RB_BK == 0 && wk_plan(bits, M, N, K, G, cus, max_lds, 8, &p);
+  out[0] = takes ? 1 : 0;
+  out[1] = p.jb;
+  out[2] = p.splits;
+}
+
+// Bytes of split-K planes a call of this shape may use: no plan has more than 8 ranges, nor more than two
+// workgroups per CU when it splits (of at least N / 128 column tiles).
+int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+  if (M <= 16 || M > 64 || N <= 0 || K % RB_BK != 0) return 0;
+  const int64_t s = std::min<int64_t>(8, 2 * (int64_t)cus / imq_cdiv(N, 128));
+  return s > 1 ? s * M * N * 4 : 0;
+}
+
+// 16 < M <= 64, K a multiple of 64; groups and strides checked by the caller (gemm_wq_any). Scale and
+// zero of any dtype. IMQ_ERR_UNSUPPORTED for offsets beyond 32 bits or tiles no LDS holds: the
+// LDS-dequant GEMM takes those. Without a large enough workspace K is not split.
+int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+            const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+            int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled) {
+  if (M <= 16 || M > 64) return IMQ_ERR_UNSUPPORTED;
+  if ((64 * sxm + K) * 2 > 0x7fffffff || 128 * sqn + K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
+  const DevInfo d = device_info();
+  WkPlan p;
+  if (!wk_plan(bits, M, N, K, G, d.cus, d.max_lds, 8, &p)) return IMQ_ERR_UNSUPPORTED;
+  if (p.splits > 1 && (!ws || wsb < (int64_t)p.splits * M * N * 4 || ((uintptr_t)ws & 15)))
+    if (!wk_plan(bits, M, N, K, G, d.cus, d.max_lds, 1, &p)) return IMQ_ERR_UNSUPPORTED;
+  const int KT = (int)(K / RB_BK), kps = (KT + p.splits - 1) / p.splits;
+  const int64_t T = imq_cdiv(N, 32 * p.jb);
+  if (T * p.splits > 0x7fffff) return IMQ_ERR_UNSUPPORTED;
+  WkArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, sdt, zdt, (int)N, wk_gsh(bits, G), y, sym,
+           (int)T, p.splits, kps, p.splits > 1 ? (float*)ws : nullptr};
+  const int rc = bits == 4   ? wk_run4(a, p.jb, tiled, st)
+                 : bits == 2 ? wk_run2(a, p.jb, tiled, st)
+                             : wk_run8(a, p.jb, tiled, st);
+  if (rc != IMQ_OK || p.splits == 1) return rc;
+  if (bits != 8) return splitk_sum<4, IMQ_DT_BF16>(a.part, p.splits, a.M, a.N, sc, ssn, y, sym, st);
+  switch (sdt) {   // int8: the row scale multiplies the sum
+    case IMQ_DT_BF16: return splitk_sum<8, IMQ_DT_BF16>(a.part, p.splits, a.M, a.N, sc, ssn, y, sym, st);
+    case IMQ_DT_FP16: return splitk_sum<8, IMQ_DT_FP16>(a.part, p.splits, a.M, a.N, sc, ssn, y, sym, st);
+    case IMQ_DT_FP32: return splitk_sum<8, IMQ_DT_FP32>(a.part, p.splits, a.M, a.N, sc, ssn, y, sym, st);
+  }
+  return IMQ_ERR_INVALID;
+}
+
+}  // namespace imq

@@ -1,0 +1,8 @@
+// The int2 short-batch GEMM (gemm_wk.h).
+#include "gemm_wk.h"
+
+namespace imq {
+int wk_run2(const WkArgs& a, int jb, bool tiled, hipStream_t st) {
+  return tiled ? wk_shape<2, true>(a, jb, st) : wk_shape<2, false>(a, jb, st);
+}
+}  // namespace imq

@@ -31,31 +31,6 @@
 #include <type_traits>
 
 namespace imq {
-namespace {
-
-constexpr int RB_GROUP_M = 8;
-constexpr int RB_BK = 64;
-// VALU instructions the scheduler places after each MFMA (int4 dequant / int8 conversion work):
-// chosen per format as the pattern that keeps the 256-row variants within the register file and
-// spreads a slice's work (about 2.7 per MFMA for int4) evenly. int4 4096 <-> 14336 at M = 2048, both
-// linears: 488 / 486 / 478 / 489 us at 5 / 4 / 3 / 2; 535 with v_cvt_f32_ubyteN at 5.
-#ifndef RB_VALU_PER_MFMA_4
-#define RB_VALU_PER_MFMA_4 3
-#endif
-#ifndef RB_VALU_PER_MFMA_8
-#define RB_VALU_PER_MFMA_8 3
-#endif
-#ifndef RB_VALU_PER_MFMA_FOLD
-#define RB_VALU_PER_MFMA_FOLD 4
-#endif
-// FOLD: 1 unpacks a step's four B slices at its top (step_fold), 0 one slice ahead (step)
-#ifndef RB_FOLD_EARLY_UNPACK
-#define RB_FOLD_EARLY_UNPACK 1
-#endif
-// Dense form: 1 loads activations, weights and scale / zero through buffer resources (see the kernel)
-#ifndef IMQ_RB_BUF
-#define IMQ_RB_BUF 1
-#endif
 
 struct RbArgs {
   const uint16_t* x;
@@ -100,6 +75,31 @@ struct RbArgs {
   int xk = 0;
 };
 
+namespace {
+
+constexpr int RB_GROUP_M = 8;
+constexpr int RB_BK = 64;
+// VALU instructions the scheduler places after each MFMA (int4 dequant / int8 conversion work):
+// chosen per format as the pattern that keeps the 256-row variants within the register file and
+// spreads a slice's work (about 2.7 per MFMA for int4) evenly. int4 4096 <-> 14336 at M = 2048, both
+// linears: 488 / 486 / 478 / 489 us at 5 / 4 / 3 / 2; 535 with v_cvt_f32_ubyteN at 5.
+#ifndef RB_VALU_PER_MFMA_4
+#define RB_VALU_PER_MFMA_4 3
+#endif
+#ifndef RB_VALU_PER_MFMA_2
+#define RB_VALU_PER_MFMA_2 3
+#endif
+#ifndef RB_VALU_PER_MFMA_8
+#define RB_VALU_PER_MFMA_8 3
+#endif
+#ifndef RB_VALU_PER_MFMA_FOLD
+#define RB_VALU_PER_MFMA_FOLD 4
+#endif
+// FOLD: 1 unpacks a step's four B slices at its top (step_fold), 0 one slice ahead (step)
+#ifndef RB_FOLD_EARLY_UNPACK
+#define RB_FOLD_EARLY_UNPACK 1
+#endif
+
 // Bias element i as the raw aligned dword holding it (which lies in the element's page), read
 // without a branch so it can go out with the first loads (a null bias reads `fb`'s first word);
 // rb_bias_of converts it where it is used.
@@ -124,6 +124,9 @@ IMQ_DEV __amdgpu_buffer_rsrc_t rb_rsrc(const void* base) {
 }
 IMQ_DEV u32x4_t rb_bload128(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
+IMQ_DEV u32x2_t rb_bload64(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
 }
 template <int DT>
 IMQ_DEV uint32_t rb_bload_raw(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
@@ -163,14 +166,18 @@ IMQ_DEV u32x4_t rb_convert8(uint32_t lo, uint32_t hi) {
 // (q - z) s products (the dequantizing form rounds each weight to bf16 first).
 // TL: the dense int4 form on weights in the line-tiled layout (16-byte pieces permuted within
 // 16-row tiles), a separate instantiation so the row-layout loop is unchanged.
-template <int BITS, int SDT, int ZDT, int IB, int NW, int MOE = 0, int PD = 2, bool FOLD = false, bool TL = false>
-__global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
+// MINW: waves per SIMD the registers are bounded for.
+template <int BITS, int SDT, int ZDT, int IB, int NW, int MOE = 0, int PD = 2, bool FOLD = false, bool TL = false,
+          int MINW = 1>
+__global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
+  static_assert(BITS != 2 || MOE == 0, "int2: the dense forms");
   static_assert(!FOLD || (MOE != 0 && BITS == 4 && PD % 2 == 0), "the folded form: int4 MoE, even pipeline depth");
   static_assert(!TL || MOE == 0, "line-tiled weights: the dense forms");
   constexpr int BM = 32 * IB, BN = 64 * NW, BK = RB_BK, NTHR = 64 * NW;
   constexpr int A_EL = BM * BK;                    // bf16 elements of one LDS buffer
   constexpr int XC = BM * 8 / NTHR;                // 16-byte activation chunks per thread per step
-  constexpr int QV = BITS == 8 ? 2 : 1;            // 16-byte weight loads per lane per column block
+  constexpr int QV = BITS == 8 ? 2 : 1;            // weight loads per lane per column block (16 bytes, int2: 8)
+  constexpr int QB = 4 * BITS;                     // packed bytes of a lane's 32 codes
   static_assert((BM * 8) % NTHR == 0, "activation chunks must divide evenly");
   extern __shared__ __align__(16) uint16_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -235,7 +242,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
   // into it is fixed for the whole K loop and the step's offset is a scalar operand, so a step's
   // loads cost no vector address arithmetic (64-bit per-lane addresses were a fifth of the loop's
   // VALU instructions). gemm_rb keeps every offset below 2^31.
-  constexpr bool BUF = MOE == 0 && IMQ_RB_BUF;
+  constexpr bool BUF = MOE == 0;
   const uint16_t* xtile = a.x + (int64_t)m0 * a.sxm;
   int xo[XC], xl[XC];
   // MoE forms: the block's routed rows RID[row] = perm[prow0 + row] (0 past cnt), staged in LDS by
@@ -283,10 +290,10 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
   for (int j = 0; j < 2; ++j) {
     int n = MOE == 1 ? (j ? a.I : 0) + tn * (32 * NW) + 32 * wave + c : n0 + 64 * wave + 32 * j + c;
     n = n < a.N ? n : a.N - 1;
-    qb[j] = a.q + (int64_t)e * a.sqe + (int64_t)n * a.sqn + (BITS == 8 ? 32 : 16) * h;
+    qb[j] = a.q + (int64_t)e * a.sqe + (int64_t)n * a.sqn + QB * h;
     sb[j] = (int64_t)e * a.sse + (int64_t)n * a.ssn;
     zb[j] = (int64_t)e * a.sse + (int64_t)n * a.szn;
-    qvo[j] = (uint32_t)((n - n0) * (int)a.sqn + (BITS == 8 ? 32 : 16) * h);
+    qvo[j] = (uint32_t)((n - n0) * (int)a.sqn + QB * h);
     svo[j] = (uint32_t)(((n - n0) * (int)a.ssn + gh * (int)a.ssg) * SES);
     zvo[j] = (uint32_t)(((n - n0) * (int)a.szn + gh * (int)a.szg) * ZES);
     if constexpr (TL) {
@@ -294,10 +301,11 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
       // rr / 16, half hr = (rr / 8) & 1, slot (rr & 7) + 8 (sel ^ hr) + 16 (piece & 3) of the
       // step's line-step. int4 (16 bytes at 32 kt + 16 h): line-step kt / 4, piece 2 (kt & 1) + h,
       // sel = (kt / 2) & 1; int8 (two pieces at 64 kt + 32 h + 16 v): line-step kt / 2, piece 2 h
-      // + v, sel = kt & 1. sel moves the slot by 8, bit 7 of the byte offset (nothing else reaches that
+      // + v, sel = kt & 1; int2 (8 bytes at 16 kt + 8 h, half of a piece): line-step kt / 8, piece
+      // kt & 7, sel = (kt / 4) & 1. sel moves the slot by 8, bit 7 of the byte offset (nothing else reaches that
       // bit: 16 rows are a multiple of 2048 bytes), so a lane keeps one offset and xors sel << 7 into it.
       const int rr = n - n0, hr = (rr >> 3) & 1;
-      const uint32_t tb = (uint32_t)((rr >> 4) * 16 * (int)a.sqn + 1024 * hr + 16 * (rr & 7) + (BITS == 8 ? 512 : 256) * h);
+      const uint32_t tb = (uint32_t)((rr >> 4) * 16 * (int)a.sqn + 1024 * hr + 16 * (rr & 7) + (BITS == 8 ? 512 : BITS == 4 ? 256 : 8) * h);
       qto[j] = tb + 128 * hr;
     }
   }
@@ -437,7 +445,12 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
 
   static_assert(PD >= 2 && PD <= 4, "pipeline depth 2..4");
   u32x4_t xr[PD][XC];
-  u32x4_t qr[PD][2][QV];
+  using QT = std::conditional_t<BITS == 2, u32x2_t, u32x4_t>;
+  QT qr[PD][2][QV];
+  auto bload_q = [&](uint32_t voff, uint32_t soff) -> QT {
+    if constexpr (BITS == 2) return rb_bload64(qrs, voff, soff);
+    else return rb_bload128(qrs, voff, soff);
+  };
   uint32_t sr[PD][2], zr[PD][2];
   const int kt0 = split * a.kps;
   const int KS = ((MOE != 0 && a.xk > 0) ? a.xk : a.K) / BK;   // K steps with nonzero activations
@@ -460,13 +473,14 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if constexpr (TL) {
-          const uint32_t sx = (BITS == 8 ? (kt & 1) : ((kt >> 1) & 1)) << 7;
-          const uint32_t so = BITS == 8 ? 2048 * (kt >> 1) : 2048 * (kt >> 2) + 512 * (kt & 1);
+          const uint32_t sx = ((BITS == 8 ? kt : BITS == 4 ? (kt >> 1) : (kt >> 2)) & 1) << 7;
+          const uint32_t so = BITS == 8 ? 2048 * (kt >> 1) : BITS == 4 ? 2048 * (kt >> 2) + 512 * (kt & 1)
+                                                                       : 2048 * (kt >> 3) + 256 * (kt & 3);
 #pragma unroll
-          for (int v = 0; v < QV; ++v) qr[set][j][v] = rb_bload128(qrs, (qto[j] ^ sx) + 256 * v, so);
+          for (int v = 0; v < QV; ++v) qr[set][j][v] = bload_q((qto[j] ^ sx) + 256 * v, so);
         } else {
 #pragma unroll
-          for (int v = 0; v < QV; ++v) qr[set][j][v] = rb_bload128(qrs, qvo[j] + 16 * v, kt * (BK * BITS / 8));
+          for (int v = 0; v < QV; ++v) qr[set][j][v] = bload_q(qvo[j] + 16 * v, kt * (BK * BITS / 8));
         }
         if constexpr (BITS != 8) {
           sr[set][j] = rb_bload_raw<SDT>(srs, svo[j], gs * (uint32_t)a.ssg * SES);
@@ -475,23 +489,11 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
       }
       return;
     }
+    if constexpr (MOE != 0) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      if constexpr (TL) {
-        const uint32_t sx = (BITS == 8 ? (kt & 1) : ((kt >> 1) & 1)) << 7;
-        const uint32_t so = BITS == 8 ? 2048 * (kt >> 1) : 2048 * (kt >> 2) + 512 * (kt & 1);
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int v = 0; v < QV; ++v)
-          qr[set][j][v] = *(const u32x4_t*)(a.q + (int64_t)n0 * a.sqn + (qto[j] ^ sx) + 256 * v + so);
-      } else {
-#pragma unroll
-        for (int v = 0; v < QV; ++v) qr[set][j][v] = *(const u32x4_t*)(qb[j] + kt * (BK * BITS / 8) + 16 * v);
-      }
-      if constexpr (MOE == 0 && BITS != 8) {
-        const int g = (kt * BK + 32 * h) >> a.gsh;
-        sr[set][j] = load_raw_bits<SDT>(a.sc, sb[j] + (int64_t)g * a.ssg);
-        zr[set][j] = load_raw_bits<ZDT>(a.zr, zb[j] + (int64_t)g * a.szg);
-      }
+        for (int v = 0; v < QV; ++v) qr[set][j][v] = *(const QT*)(qb[j] + kt * (BK * BITS / 8) + 16 * v);
     }
   };
   // MoE forms: the scale / zero pair of a weight set, from the staged LDS copy
@@ -562,10 +564,13 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
     if constexpr (FOLD) return unpack_nib8_bf16(qr[bs][j][0][s], magic);
     u32x4_t d;
     if constexpr (BITS == 8) d = rb_convert8(qr[bs][j][s >> 1][2 * (s & 1)], qr[bs][j][s >> 1][2 * (s & 1) + 1]);
+    else if constexpr (BITS == 2) d = dequant8_bf16<2>(qr[bs][j][0][s >> 1], s & 1, sv, nz);
     else d = dequant8_bf16<4>(qr[bs][j][0][s], 0, sv, nz);
     return __builtin_bit_cast(bf16x8_t, d);
   };
 
+  constexpr int VPM = FOLD ? RB_VALU_PER_MFMA_FOLD : BITS == 8 ? RB_VALU_PER_MFMA_8 : BITS == 4 ? RB_VALU_PER_MFMA_4
+                                                                                             : RB_VALU_PER_MFMA_2;
   // LDS: three buffers of BM x 64 activations; step kt reads buffer kt % 3 and writes A(kt+1) into
   // buffer (kt+1) % 3, whose last reads (steps kt-2 and the slice-0 prefetch at the end of kt-3)
   // all precede the barrier of step kt-1 -- so one barrier per step suffices, placed after
@@ -645,7 +650,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_rb_kernel(RbArgs a) {
 #pragma unroll
       for (int k = 0; k < 2 * IB; ++k) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, FOLD ? RB_VALU_PER_MFMA_FOLD : BITS == 8 ? RB_VALU_PER_MFMA_8 : RB_VALU_PER_MFMA_4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
     }

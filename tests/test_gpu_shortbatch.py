@@ -1,0 +1,104 @@
+"""The short-batch GEMM (16 < M <= 64) where it can go wrong: the first and last row counts of each row
+block, ragged column tiles, K of one step and of fewer steps than waves, K ranges that end inside a
+scale group, every group size, dtype pair and layout it takes, strided operands, and the plan without a
+workspace. Against the oracle's product of the once-rounded bf16 weights, per element."""
+import numpy as np
+import pytest
+
+from oracle import quant as oq
+from tests import _cases as C
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(y, x, w, acc_scale=1e-5):
+    """bf16 result of an fp32 sum: half an ulp of bf16 plus the sum's own rounding."""
+    exact = oq.linear_ref(x, w)
+    tol = 2.0 ** -8 * np.abs(exact) + acc_scale * np.abs(exact).max()
+    bad = np.abs(C.t2np(y) - exact) > tol
+    assert not bad.any(), (int(bad.sum()), np.argwhere(bad)[:4].tolist())
+
+
+def _group_case(dev, bits, N, K, G, sdt, zdt, seed):
+    r = C.rng(seed)
+    ng = K // G
+    codes = r.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    q = np.zeros((N, K * bits // 8), np.uint8)
+    for i in range(8 // bits):
+        q |= codes[:, i::8 // bits] << (bits * i)
+    s = oq.round_to(r.uniform(0.005, 0.05, (N, ng)).astype(np.float32), sdt)
+    z = oq.round_to(r.uniform(0, (1 << bits) - 1, (N, ng)).astype(np.float32), zdt)
+    w = oq.round_to(oq.dequant_exact(codes, s, z, G, K).astype(np.float32), "bf16")
+    return C.u8(q, dev), C.to_torch(s, sdt, dev), C.to_torch(z, zdt, dev), w
+
+
+CASES = [
+    # M, N, K, bits, G, scale dtype, zero dtype
+    (17, 37, 64, 4, 64, "bf16", "bf16"), (32, 100, 448, 4, 64, "fp16", "bf16"), (33, 33, 576, 4, 32, "bf16", "fp32"),
+    (64, 2944, 768, 4, 128, "fp32", "fp32"), (48, 4096, 4096, 4, 128, "bf16", "bf16"), (31, 257, 14336, 4, 256, "fp16", "fp16"),
+    (20, 30000, 512, 4, 128, "bf16", "bf16"), (17, 96, 448, 2, 64, "fp16", "fp16"), (64, 1000, 8192, 2, 64, "fp16", "fp16"),
+    (32, 16400, 1024, 2, 32, "bf16", "fp16"), (40, 300, 28672, 2, 128, "fp32", "bf16"),
+]
+
+
+@pytest.mark.parametrize("M,N,K,bits,G,sdt,zdt", CASES)
+def test_group_formats_match_the_oracle(dev, M, N, K, bits, G, sdt, zdt):
+    import torch
+    from infinitemodel_amd import ops
+    q, s, z, w = _group_case(dev, bits, N, K, G, sdt, zdt, seed=M + N + K)
+    x = C.bf16_normal(C.rng(M), (M, K))
+    op = ops.linear_w4 if bits == 4 else ops.linear_w2
+    y = op(C.to_torch(x, "bf16", dev), q, G, (s, z))
+    _check(y, x, w)
+    # strided operands: padded activation and weight rows, column-major scales, padded output rows
+    xw = torch.zeros(M, K + 24, dtype=torch.bfloat16, device=dev)
+    xw[:, 8:8 + K] = C.to_torch(x, "bf16", dev)
+    qw = torch.zeros(N, q.shape[1] + 64, dtype=torch.uint8, device=dev)
+    qw[:, :q.shape[1]] = q
+    out = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device=dev)
+    op(xw[:, 8:8 + K], qw[:, :q.shape[1]], G, (s.t().contiguous().t(), z.t().contiguous().t()), out=out[:, :N])
+    assert torch.equal(out[:, :N], y) and bool((out[:, N:] == 7).all())
+    if N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == (128 if bits == 4 else 64) and sdt == zdt:
+        tiled = ops.linear_w4_tiled if bits == 4 else ops.linear_w2_tiled
+        assert torch.equal(tiled(C.to_torch(x, "bf16", dev), ops.line_tile(q), G, (s, z)), y)
+
+
+@pytest.mark.parametrize("M,N,K,sdt", [(17, 40, 64, "bf16"), (33, 272, 1152, "fp16"), (64, 1008, 14336, "fp32"),
+                                       (32, 14336, 4096, "fp16")])
+def test_int8_matches_the_oracle(dev, M, N, K, sdt):
+    import torch
+    from infinitemodel_amd import ops
+    r = C.rng(N + K)
+    q = r.integers(-127, 128, (N, K), dtype=np.int8)
+    s = oq.round_to(r.uniform(1e-4, 1e-3, (N, 1)).astype(np.float32), sdt)
+    x = C.bf16_normal(C.rng(M), (M, K))
+    qt, st, xt = torch.from_numpy(q).to(dev), C.to_torch(s, sdt, dev), C.to_torch(x, "bf16", dev)
+    y = ops.linear_w8(xt, qt, st)
+    _check(y, x, q.astype(np.float64) * s)
+    if N % 16 == 0 and K % 128 == 0:
+        assert torch.equal(ops.linear_w8_tiled(xt, ops.line_tile(qt), st), y)
+
+
+def test_without_a_workspace_and_repeated(dev):
+    """A shape whose plan splits K: the same call without a workspace runs unsplit, and repeats and graph
+    replays of the split call agree bit for bit."""
+    import torch
+    from infinitemodel_amd import _lib, ops
+    M, N, K = 24, 256, 8192
+    assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, 128, N, sqn=K // 2)[1] > 1
+    q, s, z, w = _group_case(dev, 4, N, K, 128, "bf16", "bf16", seed=5)
+    x = C.bf16_normal(C.rng(M), (M, K))
+    xt = C.to_torch(x, "bf16", dev)
+    y = ops.linear_w4(xt, q, 128, (s, z))
+    _check(y, x, w)
+    y0 = torch.empty_like(y)
+    _lib.call("imq_linear_w4", xt.data_ptr(), K, M, K, q.data_ptr(), K // 2, s.data_ptr(), s.stride(0), 1, 0, z.data_ptr(),
+              z.stride(0), 1, 0, N, 128, y0.data_ptr(), N, None, 0, torch.cuda.current_stream(dev).cuda_stream)
+    _check(y0, x, w)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        yg = ops.linear_w4(xt, q, 128, (s, z))
+    for _ in range(3):
+        yg.zero_()
+        g.replay()
+        assert torch.equal(yg, y) and torch.equal(ops.linear_w4(xt, q, 128, (s, z)), y)

@@ -1,0 +1,95 @@
+"""The short-batch GEMM's plan and address arithmetic (csrc/gemm_wk.h), restated: every K step is taken by
+one wave of one range, every operand read lies inside its buffer, the line-tiled offsets are the
+layout's definition, the staged scale groups cover the steps that use them, and the LDS regions fit."""
+import numpy as np
+import pytest
+
+from infinitemodel_amd import _lib
+from tests import _cases as C
+
+WAVES, BK = 8, 64
+
+
+def _plan(bits, M, N, K, G, cus=256, lds=160 * 1024):
+    got = _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, G, N, sqn=K * bits // 8, max_lds=lds, cus=cus)
+    return got and got[:2]
+
+
+def _szs(jb):
+    return 32 * jb + {1: 4, 2: 8, 4: 16}[jb]
+
+
+CASES = [(4, 17, 28672, 4096, 128), (4, 64, 28672, 4096, 128), (4, 32, 4096, 14336, 128), (4, 20, 37, 64, 64),
+         (4, 33, 1008, 448, 32), (2, 64, 8192, 28672, 64), (2, 17, 96, 448, 64), (8, 40, 4096, 14336, 0),
+         (8, 17, 40, 64, 0), (4, 24, 256, 8192, 128), (4, 17, 151936, 3584, 128)]
+
+
+@pytest.mark.parametrize("bits,M,N,K,G", CASES)
+@pytest.mark.parametrize("cus,lds", [(256, 160 * 1024), (32, 64 * 1024)])
+def test_plan_and_addresses(bits, M, N, K, G, cus, lds):
+    p = _plan(bits, M, N, K, G, cus, lds)
+    if p is None:
+        assert lds < 160 * 1024          # only a small LDS refuses a shape
+        return
+    jb, splits = p
+    ib, KT_all = (1 if M <= 32 else 2), K // BK
+    kps = -(-KT_all // splits)
+    rj = 2 if ib == 1 and jb > 1 else 1
+    gsh = G.bit_length() - 1 if G else 0
+    groups_alloc = 0 if bits == 8 else ((kps * BK) >> gsh) + 2
+    region = WAVES * ib * rj * 4096
+    assert region + groups_alloc * _szs(jb) * 4 <= lds
+    taken = np.zeros(KT_all, int)
+    for split in range(splits):
+        kt0 = split * kps
+        KT = min(KT_all - kt0, kps)
+        assert KT >= 1
+        g_lo, g_hi = (kt0 * BK) >> gsh, ((kt0 + KT) * BK - 1) >> gsh
+        assert bits == 8 or g_hi - g_lo + 1 <= groups_alloc
+        for wave in range(WAVES):
+            steps = (KT - wave + WAVES - 1) // WAVES if KT > wave else 0
+            for i in range(steps + 2):                       # loads run up to two steps ahead, clamped
+                kt = kt0 + min(wave, KT - 1) + WAVES * max(min(i, steps - 1), 0)
+                assert kt0 <= kt < kt0 + KT
+                if i < steps:
+                    taken[kt] += 1
+                    if bits != 8:
+                        for h in range(2):
+                            assert g_lo <= (kt * BK + 32 * h) >> gsh <= g_hi
+    assert (taken == 1).all()
+    # activation rows and chunks of a step: 32 ib rows of 8 chunks, each LDS slot once
+    slots = set()
+    for j in range(4 * ib):
+        for lane in range(64):
+            row, ch = 8 * j + (lane >> 3), lane & 7
+            slots.add((row * 8 + (ch ^ ((row >> 1) & 7))) * 16)
+            assert min(row, M - 1) * K + ch * 8 + (KT_all - 1) * BK + 8 <= M * K
+    assert slots == set(range(0, ib * 4096, 16))
+    # the sums' quads fill the same regions
+    assert max(((u * ib + b) * 4 + r4) * 64 + lane for u in range(rj) for b in range(ib) for r4 in range(4)
+               for lane in (63,)) * 16 + 16 == ib * rj * 4096
+
+
+@pytest.mark.parametrize("bits,K", [(4, 512), (2, 1024), (8, 256)])
+def test_tiled_offsets_are_the_layout(bits, K):
+    """Lane (column c, half h) at K step kt reads, at its tiled offset, the bytes [QB (2 kt + h), + QB) of
+    its row (QB = 4 bits), int8 in two 16-byte pieces 256 bytes apart."""
+    N = 48
+    q = np.random.default_rng(bits).integers(0, 256, (N, K * bits // 8), dtype=np.uint8)
+    flat, sqn, QB = C.line_tile_np(q).reshape(-1), K * bits // 8, 4 * bits
+    for rr in range(N):
+        for h in range(2):
+            hr = (rr >> 3) & 1
+            qo = (rr >> 4) * 16 * sqn + 1152 * hr + 16 * (rr & 7) + {8: 512, 4: 256, 2: 8}[bits] * h
+            for kt in range(K // BK):
+                sel = {8: kt, 4: kt >> 1, 2: kt >> 2}[bits] & 1
+                so = {8: 2048 * (kt >> 1), 4: 2048 * (kt >> 2) + 512 * (kt & 1),
+                      2: 2048 * (kt >> 3) + 256 * (kt & 3)}[bits]
+                at = (qo ^ (sel << 7)) + so
+                got = np.concatenate([flat[at + 256 * v: at + 256 * v + min(QB, 16)] for v in range(2 if bits == 8 else 1)])
+                assert np.array_equal(got, q[rr, QB * (2 * kt + h): QB * (2 * kt + h) + QB])
+
+
+def test_small_devices_and_other_rows_decline():
+    assert _plan(4, 16, 4096, 4096, 128) is None and _plan(4, 65, 4096, 4096, 128) is None
+    assert _plan(4, 17, 4096, 4096 + 32, 128) is None
