@@ -94,7 +94,7 @@ SIGNATURES = {
 
 IMQ_PLAN_W4_LINE, IMQ_PLAN_W4_KSPLIT, IMQ_PLAN_W4_WSPLIT, IMQ_PLAN_W4_SKINNY = 1, 2, 3, 4
 IMQ_PLAN_W2_LINE, IMQ_PLAN_W2_KSPLIT, IMQ_PLAN_W8_LINE, IMQ_PLAN_GEMM, IMQ_PLAN_GEMM_RB = 5, 6, 7, 8, 9
-IMQ_PLAN_GEMM_WK = 10
+IMQ_PLAN_GEMM_WK, IMQ_PLAN_GEMM_RBM = 10, 11
 
 
 class ImqUnavailable(RuntimeError):

@@ -23,6 +23,7 @@
 #include "imq_common.h"
 #include "splitk_sum.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace imq {
@@ -36,6 +37,10 @@ int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus);
 int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled);
+int64_t rbm_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus);
+int gemm_rbm(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled);
 
 namespace {
 
@@ -654,8 +659,8 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   const int64_t lds = use_big(M) ? split_bytes<CfgBig>(M, N, K, cus) : split_bytes<CfgSmall>(M, N, K, cus);
   const int64_t rb = rb_workspace_bytes(4, M, N, K, cus);
   const int64_t wk = wk_workspace_bytes(M, N, K, cus);
-  const int64_t m = lds > rb ? lds : rb;
-  return m > wk ? m : wk;
+  const int64_t rbm = rbm_workspace_bytes(M, N, K, cus);
+  return std::max(std::max(lds, rb), std::max(wk, rbm));
 }
 
 namespace {
@@ -751,9 +756,9 @@ int gemm_wq_any(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, 
   // widest weight load of either tile configuration: 16 B (int4, int8 as 2 x 16 B), 8 B (int2)
   const int wbytes = bits == 2 ? 8 : 16;
   if (((uintptr_t)q % wbytes) || (sqn % wbytes)) return IMQ_ERR_UNSUPPORTED;
-  if (M <= 64) {
-    const int rc = gemm_wk(bits, x, sxm, M, K, q, sqn, sc, ssn, ssg, sdt, zr, szn, szg, zdt, N, G, y, sym, ws, wsb, st,
-                           tiled);
+  {
+    const auto gemm = M <= 64 ? gemm_wk : gemm_rbm;
+    const int rc = gemm(bits, x, sxm, M, K, q, sqn, sc, ssn, ssg, sdt, zr, szn, szg, zdt, N, G, y, sym, ws, wsb, st, tiled);
     if (rc != IMQ_ERR_UNSUPPORTED) return rc;
   }
   if (rb_takes(bits, M, N, K, G)) {

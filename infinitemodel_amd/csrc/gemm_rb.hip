@@ -1,5 +1,6 @@
 // Prefill-regime fused dequant GEMM with the weights dequantized straight into MFMA B operands
-// ("register-B" form): the dense launchers (tile plan, split-K partials and their reduction).
+// ("register-B" form) at two tile heights, for scale / zero dtype pairs other than the two 16-bit
+// types alike (those run at any height, gemm_rbm.hip): tile plan, split-K partials and their reduction.
 // The kernel and its structure are described in rb_kernel.h.
 #include "rb_kernel.h"
 #include "splitk_sum.h"
@@ -66,18 +67,15 @@ int rb_ib_dispatch(const RbArgs& a, void* ws, int64_t wsb, hipStream_t st) {
   return rb_launch<BITS, SDT, ZDT, 4, TL>(a, ws, wsb, st);
 }
 
-template <int BITS, int SDT>
+// The dtype pairs gemm_rbm (one 16-bit dtype for both) does not take; int8: an fp32 scale.
+template <int SDT>
 int rb_z(const RbArgs& a, int zdt, void* ws, int64_t wsb, hipStream_t st) {
-  if constexpr (BITS == 8) {
-    return rb_ib_dispatch<8, SDT, SDT>(a, ws, wsb, st);
-  } else {
-    switch (zdt) {
-      case IMQ_DT_BF16: return rb_ib_dispatch<BITS, SDT, IMQ_DT_BF16>(a, ws, wsb, st);
-      case IMQ_DT_FP16: return rb_ib_dispatch<BITS, SDT, IMQ_DT_FP16>(a, ws, wsb, st);
-      case IMQ_DT_FP32: return rb_ib_dispatch<BITS, SDT, IMQ_DT_FP32>(a, ws, wsb, st);
-    }
-    return IMQ_ERR_INVALID;
-  }
+  if constexpr (SDT != IMQ_DT_BF16)
+    if (zdt == IMQ_DT_BF16) return rb_ib_dispatch<4, SDT, IMQ_DT_BF16>(a, ws, wsb, st);
+  if constexpr (SDT != IMQ_DT_FP16)
+    if (zdt == IMQ_DT_FP16) return rb_ib_dispatch<4, SDT, IMQ_DT_FP16>(a, ws, wsb, st);
+  if (zdt == IMQ_DT_FP32) return rb_ib_dispatch<4, SDT, IMQ_DT_FP32>(a, ws, wsb, st);
+  return IMQ_ERR_UNSUPPORTED;
 }
 
 }  // namespace
@@ -128,25 +126,18 @@ int gemm_rb(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, cons
     if ((256 * ssn + ng * ssg) * 4 > 0x7fffffff || (256 * szn + ng * szg) * 4 > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
   }
   RbArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, (int)N, gsh, y, sym, 0, 0, 1, 0, nullptr};
-  if (tiled) {   // line-tiled weights: int4 with scale and zero of one dtype, or int8
-    if (bits == 4 && sdt != zdt) return IMQ_ERR_UNSUPPORTED;
-    switch (sdt) {
-      case IMQ_DT_BF16:
-        return bits == 8 ? rb_ib_dispatch<8, IMQ_DT_BF16, IMQ_DT_BF16, true>(a, ws, wsb, st)
-                         : rb_ib_dispatch<4, IMQ_DT_BF16, IMQ_DT_BF16, true>(a, ws, wsb, st);
-      case IMQ_DT_FP16:
-        return bits == 8 ? rb_ib_dispatch<8, IMQ_DT_FP16, IMQ_DT_FP16, true>(a, ws, wsb, st)
-                         : rb_ib_dispatch<4, IMQ_DT_FP16, IMQ_DT_FP16, true>(a, ws, wsb, st);
-      case IMQ_DT_FP32:
-        return bits == 8 ? rb_ib_dispatch<8, IMQ_DT_FP32, IMQ_DT_FP32, true>(a, ws, wsb, st)
-                         : rb_ib_dispatch<4, IMQ_DT_FP32, IMQ_DT_FP32, true>(a, ws, wsb, st);
-    }
-    return IMQ_ERR_INVALID;
+  if (bits == 8) {
+    if (sdt != IMQ_DT_FP32) return IMQ_ERR_UNSUPPORTED;
+    return tiled ? rb_ib_dispatch<8, IMQ_DT_FP32, IMQ_DT_FP32, true>(a, ws, wsb, st)
+                 : rb_ib_dispatch<8, IMQ_DT_FP32, IMQ_DT_FP32>(a, ws, wsb, st);
   }
+  if (tiled)   // line-tiled weights carry scale and zero of one dtype
+    return sdt == IMQ_DT_FP32 && zdt == IMQ_DT_FP32 ? rb_ib_dispatch<4, IMQ_DT_FP32, IMQ_DT_FP32, true>(a, ws, wsb, st)
+                                                    : IMQ_ERR_UNSUPPORTED;
   switch (sdt) {
-    case IMQ_DT_BF16: return bits == 8 ? rb_z<8, IMQ_DT_BF16>(a, zdt, ws, wsb, st) : rb_z<4, IMQ_DT_BF16>(a, zdt, ws, wsb, st);
-    case IMQ_DT_FP16: return bits == 8 ? rb_z<8, IMQ_DT_FP16>(a, zdt, ws, wsb, st) : rb_z<4, IMQ_DT_FP16>(a, zdt, ws, wsb, st);
-    case IMQ_DT_FP32: return bits == 8 ? rb_z<8, IMQ_DT_FP32>(a, zdt, ws, wsb, st) : rb_z<4, IMQ_DT_FP32>(a, zdt, ws, wsb, st);
+    case IMQ_DT_BF16: return rb_z<IMQ_DT_BF16>(a, zdt, ws, wsb, st);
+    case IMQ_DT_FP16: return rb_z<IMQ_DT_FP16>(a, zdt, ws, wsb, st);
+    case IMQ_DT_FP32: return rb_z<IMQ_DT_FP32>(a, zdt, ws, wsb, st);
   }
   return IMQ_ERR_INVALID;
 }

@@ -1,0 +1,118 @@
+// Register-B GEMM (rb_kernel.h) at any tile height of 96 to 256 rows, scale and zero both bf16 or both fp16:
+// plan and dispatch. M > 64.
+#include "rbm_launch.h"
+
+namespace imq {
+
+int rbm_run4(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStream_t st);
+int rbm_run2(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStream_t st);
+int rbm_run8(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStream_t st);
+void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out);
+
+namespace {
+
+// Bytes of split-K planes a plan may use. Up to 512 rows, where the LDS-dequant GEMM is the alternative, the
+// planes of a good plan stay in the last-level cache beside the operands (int8 14336 -> 4096 at M = 512 in 8
+// planes of 8 MiB: 73.5 us against 70.3); larger batches compare with unsplit tiles on half the CUs.
+constexpr int64_t rbm_max_planes(int64_t M) { return (M <= 512 ? 48ll : 64ll) << 20; }
+
+// us of `splits` fp32 planes: the sum's launch with its gap, the planes written and read (mostly from cache).
+double planes_us(int s, int64_t M, int64_t N) { return s > 1 ? 4.5 + 1e-6 * s * M * N : 0; }
+
+// The tile plan, the cheapest by a model fitted to sweeps of heights and splits over 4096 x 4096 .. 28672 at
+// M 96 .. 2048 (it picks the measured best or one within 5%): a 64-code step of an ib x 32 row, 256-column
+// tile takes 0.55 + 0.17 ib us (int8 0.45 + 0.15 ib); heights up to 128 rows keep two workgroups on a CU,
+// whose steps then overlap to 0.89 of that each. Row blocks are spread evenly over the row tiles (777 rows:
+// 4 tiles of 7 blocks, not 4 of 8). Returns the modelled us.
+double rbm_plan(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes, RbmPlan* p) {
+  const int KT = (int)(K / RB_BK);
+  const int64_t blocks = imq_cdiv(M, 32), cols = imq_cdiv(N, 256);
+  double best = -1;
+  const int64_t rt0 = imq_cdiv(blocks, 8);
+  for (int64_t rt = rt0; rt <= 3 * rt0; ++rt) {
+    const int ib = (int)imq_cdiv(blocks, rt);
+    if (ib < 3) break;
+    if (rt > rt0 && ib == (int)imq_cdiv(blocks, rt - 1)) continue;   // the same height with idle tiles
+    const double t = bits == 8 ? 0.45 + 0.15 * ib : 0.55 + 0.17 * ib;
+    for (int s = 1; s <= (planes ? 8 : 1); ++s) {
+      const int kps = (KT + s - 1) / s;
+      const int64_t W = rt * cols * s;
+      if (s > 1 && ((s - 1) * kps >= KT || kps < 8 || W > 2 * (int64_t)cus || 4ll * s * M * N > rbm_max_planes(M))) break;
+      double us;
+      if (W <= cus) us = kps * t;
+      else if (ib <= 4) us = (double)((W + 2 * cus - 1) / (2 * cus)) * kps * 2 * 0.89 * t;
+      else us = (double)((W + cus - 1) / cus) * kps * t;
+      us += 3 + planes_us(s, M, N);
+      if (best < 0 || us < best) {
+        best = us;
+        *p = RbmPlan{ib, s};
+      }
+    }
+  }
+  return best;
+}
+
+// The LDS-dequant GEMM's modelled us on the same call (its plan as gemm_plan_query gives it).
+double lds_us(int64_t M, int64_t N, int64_t K, int cus, bool planes) {
+  int64_t out[5] = {};
+  gemm_plan_query(M, N, K, cus, out);
+  const int64_t s = planes ? out[3] : 1, W = imq_cdiv(M, out[1]) * imq_cdiv(N, out[2]) * s;
+  return 3 + (double)imq_cdiv(W, cus) * imq_cdiv(K / RB_BK, s) * (out[1] == 256 ? 1.1 : 0.87) + planes_us((int)s, M, N);
+}
+
+bool rbm_takes(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, bool planes, RbmPlan* p) {
+  if (M <= 64 || N <= 0 || K <= 0 || K % RB_BK != 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return false;
+  if (bits != 8 && (G < 32 || (G & (G - 1)) != 0)) return false;
+  const double us = rbm_plan(bits, M, N, K, cus, planes, p);
+  // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within 7% (its own spread)
+  return us > 0 && (M > 512 || us < 0.93 * lds_us(M, N, K, cus, planes));
+}
+
+}  // namespace
+
+// The plan of a call without a device (workspace given): out = {takes the call, 32-row blocks per tile, K splits}.
+void rbm_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int64_t* out) {
+  RbmPlan p{0, 0};
+  const bool takes = rbm_takes(bits, M, N, K, G, cus, true, &p);
+  out[0] = takes ? 1 : 0;
+  out[1] = takes ? p.ib : 0;
+  out[2] = takes ? p.splits : 0;
+}
+
+int64_t rbm_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
+  int64_t need = 0;
+  for (int bits : {4, 8}) {                        // int2 plans as int4
+    RbmPlan p;
+    if (rbm_takes(bits, M, N, K, 128, cus, true, &p) && p.splits > 1) need = 4 * p.splits * M * N > need ? 4 * p.splits * M * N : need;
+  }
+  return need;
+}
+
+// Operands as gemm_wq_any checked them. IMQ_ERR_UNSUPPORTED: another GEMM is as fast or the layout is not
+// covered (other dtype pairs, offsets beyond 32 bits).
+int gemm_rbm(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled) {
+  if (sdt != IMQ_DT_BF16 && sdt != IMQ_DT_FP16) return IMQ_ERR_UNSUPPORTED;
+  if (bits != 8 && sdt != zdt) return IMQ_ERR_UNSUPPORTED;
+  // the kernel's buffer offsets from a tile's first row (activations, weights, scale / zero)
+  if ((256 * sxm + K) * 2 > 0x7fffffff || 256 * sqn + K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
+  int gsh = 0;
+  if (bits != 8) {
+    while ((1ll << gsh) < G) ++gsh;
+    if (ssg < 0 || szg < 0 || ssn < 0 || szn < 0) return IMQ_ERR_UNSUPPORTED;
+    const int64_t ng = K / G + 1;
+    if ((256 * ssn + ng * ssg) * 4 > 0x7fffffff || (256 * szn + ng * szg) * 4 > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
+  }
+  const int cus = device_info().cus;
+  RbmPlan p;
+  if (!rbm_takes(bits, M, N, K, G, cus, true, &p)) return IMQ_ERR_UNSUPPORTED;
+  if (p.splits > 1 && (!ws || wsb < 4 * p.splits * M * N || ((uintptr_t)ws & 15)))
+    if (!rbm_takes(bits, M, N, K, G, cus, false, &p)) return IMQ_ERR_UNSUPPORTED;
+  RbArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, (int)N, gsh, y, sym, 0, 0, 1, 0, nullptr};
+  if (bits == 4) return rbm_run4(a, p, sdt, tiled, ws, st);
+  if (bits == 2) return rbm_run2(a, p, sdt, tiled, ws, st);
+  return rbm_run8(a, p, sdt, tiled, ws, st);
+}
+
+}  // namespace imq

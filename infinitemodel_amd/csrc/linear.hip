@@ -36,6 +36,7 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int decode_plan_query(int kind, const int64_t* in, int64_t* out);
 void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out);
 void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out);
+void rbm_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int64_t* out);
 void rb_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int64_t* out);
 template <int BITS>
 int generic_gemv(const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
@@ -98,9 +99,13 @@ extern "C" int imq_launch_plan(int kind, const int64_t* in, int64_t* out) {
     imq::rb_plan_query(G == 0 ? 8 : 4, M, N, K, G == 0 ? 128 : G, cus, out);
     return IMQ_OK;
   }
-  if (kind == IMQ_PLAN_GEMM_WK) {
+  if (kind == IMQ_PLAN_GEMM_WK || kind == IMQ_PLAN_GEMM_RBM) {
     const int64_t bits = K > 0 ? in[4] * 8 / K : 0;
     if (cus <= 0 || N <= 0 || K <= 0 || (bits != 2 && bits != 4 && bits != 8)) return IMQ_OK;
+    if (kind == IMQ_PLAN_GEMM_RBM) {
+      imq::rbm_plan_query((int)bits, M, N, K, G, cus, out);
+      return IMQ_OK;
+    }
     imq::wk_plan_query((int)bits, M, N, K, G, cus, (int)in[8], out);
     return IMQ_OK;
   }

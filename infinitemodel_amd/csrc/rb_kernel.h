@@ -1,6 +1,6 @@
-// The register-B GEMM kernel (weights dequantized straight into MFMA B operands) for int4
-// group-wise and int8 per-row weights on gfx950, shared by the dense launchers (gemm_rb.hip)
-// and the grouped MoE launchers (moe_rb.hip).
+// The register-B GEMM kernel (weights dequantized straight into MFMA B operands) for int4 / int2
+// group-wise and int8 per-row weights on gfx950, shared by the dense launchers (gemm_rbm.hip,
+// gemm_rb.hip) and the grouped MoE launchers (moe_rb.hip).
 //
 // y[M, N] = x[M, K] . dequant(W[N, K])^T, bf16 activations, fp32 accumulation, bf16 output: the
 // contract of the reference's `_k` / `_k8` GEMM kernels (worker_quant.py:1098-1126, 953-980).

@@ -1,0 +1,50 @@
+"""The register-B GEMM at every tile height it is built for (3 to 8 blocks of 32 rows), with and without K
+splits, ragged rows and columns, each weight format and layout: against the oracle's product of the
+once-rounded bf16 weights per element (int8: the exact integers), tiled against rows bit for bit."""
+import numpy as np
+import pytest
+
+from oracle import quant as oq
+from infinitemodel_amd import _lib
+from tests import _cases as C
+from tests.test_gpu_shortbatch import _check, _group_case
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K, bits, G, dtype: on 256 CUs each pair (height, splits) below comes up
+CASES = [(513, 1008, 1024, 4, 128, "bf16"), (777, 8200, 256, 4, 64, "fp16"), (1010, 1000, 4096, 4, 32, "bf16"),
+         (513, 4096, 2048, 4, 128, "fp16"), (500, 16400, 256, 4, 128, "bf16"), (777, 14336, 256, 4, 128, "bf16"),
+         (1010, 14336, 256, 4, 256, "fp16"), (601, 1000, 256, 2, 64, "fp16"), (777, 2000, 2048, 2, 64, "bf16"),
+         (1010, 8200, 512, 2, 32, "fp16"), (601, 16400, 512, 2, 64, "bf16"), (150, 1008, 1024, 8, 0, "fp16"),
+         (1010, 14336, 256, 8, 0, "bf16")]
+
+
+@pytest.mark.parametrize("M,N,K,bits,G,dt", CASES)
+def test_tile_heights(dev, M, N, K, bits, G, dt):
+    import torch
+    from infinitemodel_amd import ops
+    plan = _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, G, N, sqn=K * bits // 8)
+    assert plan is not None and 3 <= plan[0] <= 8, plan
+    x = C.bf16_normal(C.rng(M), (M, K))
+    xt = C.to_torch(x, "bf16", dev)
+    if bits == 8:
+        r = C.rng(N)
+        q = r.integers(-127, 128, (N, K), dtype=np.int8)
+        s = oq.round_to(r.uniform(1e-4, 1e-3, (N, 1)).astype(np.float32), dt)
+        qt, st = torch.from_numpy(q).to(dev), C.to_torch(s, dt, dev)
+        y = ops.linear_w8(xt, qt, st)
+        _check(y, x, q.astype(np.float64) * s)
+        if N % 16 == 0 and K % 128 == 0:
+            assert torch.equal(ops.linear_w8_tiled(xt, ops.line_tile(qt), st), y)
+        return
+    q, s, z, w = _group_case(dev, bits, N, K, G, dt, dt, seed=N + K)
+    y = (ops.linear_w4 if bits == 4 else ops.linear_w2)(xt, q, G, (s, z))
+    _check(y, x, w)
+    if N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == (128 if bits == 4 else 64):
+        f = ops.linear_w4_tiled if bits == 4 else ops.linear_w2_tiled
+        assert torch.equal(f(xt, ops.line_tile(q), G, (s, z)), y)
+
+
+def test_every_height_is_covered():
+    heights = {_lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, G, N, sqn=K * b // 8)[0] for M, N, K, b, G, _ in CASES}
+    assert heights == {3, 4, 5, 6, 7, 8}

@@ -1,0 +1,34 @@
+"""The register-B GEMM's plan at any tile height (csrc/gemm_rbm.hip): the row tiles cover the rows with
+no idle tile, no K range is empty, and the split-K planes fit the workspace the library asks for."""
+import pytest
+
+from infinitemodel_amd import _lib
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+@pytest.mark.parametrize("cus", [256, 80])
+def test_plans_cover_and_fit(bits, cus):
+    taken = 0
+    for N, K in [(4096, 14336), (28672, 4096), (6144, 4096), (4096, 4096), (2944, 768), (37, 64), (1000, 8192), (151936, 3584)]:
+        for M in list(range(65, 130)) + [200, 255, 256, 257, 384, 511, 512, 513, 600, 777, 1024, 1850, 2048, 4096, 8192]:
+            p = _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, 0 if bits == 8 else 64, N, sqn=K * bits // 8, cus=cus)
+            if M > 512:
+                assert p is not None
+            if p is None:
+                continue
+            taken += 1
+            ib, s = p[:2]
+            rt = -(-M // (32 * ib))
+            assert 3 <= ib <= 8 and (rt - 1) * 32 * ib < M
+            kps = -(-(K // 64) // s)
+            assert (s - 1) * kps < K // 64
+            if s > 1:
+                assert 4 * s * M * N <= 64 << 20
+                if cus == 256:      # the query's device default when no GPU is there
+                    assert _lib.lib().imq_linear_workspace_bytes(M, N, K) >= 4 * s * M * N
+    assert taken > 100
+
+
+def test_rows_up_to_64_and_odd_k_decline():
+    assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 64, 4096, 128, 4096, sqn=2048) is None
+    assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 600, 4096 + 32, 128, 4096, sqn=2064) is None
