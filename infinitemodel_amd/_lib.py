@@ -17,6 +17,7 @@ import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("IMQ_LIB_PATH") or os.path.join(HERE, "_lib", "libimq.so")
+FAST_PATH = os.path.join(os.path.dirname(LIB_PATH), "imq_fast.so")
 
 IMQ_DT_BF16, IMQ_DT_FP16, IMQ_DT_FP32, IMQ_DT_I32, IMQ_DT_I64 = 0, 1, 2, 3, 4
 IMQ_OK, IMQ_ERR_INVALID, IMQ_ERR_UNSUPPORTED, IMQ_ERR_ALIGN, IMQ_ERR_SCRATCH = 0, -1, -2, -3, -4
@@ -134,6 +135,29 @@ def lib():
             f.argtypes = args
         _LIB = L
         return _LIB
+
+
+_FAST_SYMBOLS = ("imq_linear_w4", "imq_linear_w4_tiled", "imq_linear_w2", "imq_linear_w2_tiled", "imq_linear_w8",
+                 "imq_linear_w8_tiled", "imq_linear_w4_workspace_bytes", "imq_linear_workspace_bytes",
+                 "imq_moe_experts_w4_ex", "imq_moe_workspace_bytes")
+
+
+def fast(scratch):
+    """The native host path (csrc/fastcall.cpp) bound to the loaded library, its workspaces taken from
+    ``scratch(device index, bytes) -> (pointer, bytes)``. Raises ImqUnavailable."""
+    import importlib.machinery
+    import importlib.util
+    L = lib()
+    if not os.path.exists(FAST_PATH):
+        raise ImqUnavailable(f"{FAST_PATH} not built (run `python -m infinitemodel_amd.build`)")
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("imq_fast", FAST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("imq_fast", loader))
+        loader.exec_module(mod)
+    except (ImportError, OSError) as exc:
+        raise ImqUnavailable(f"cannot load {FAST_PATH}: {exc}") from exc
+    mod.init({n: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST_SYMBOLS}, scratch)
+    return mod
 
 
 def call(name: str, *args) -> None:

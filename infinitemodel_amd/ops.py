@@ -11,6 +11,8 @@ raises ``ImqUnavailable``, a rejected call raises ``ImqError``.
 """
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from . import _lib
@@ -76,6 +78,44 @@ def _workspace(dev: torch.device, M: int, N: int, K: int):
     if ws is None:
         return 0, 0
     return ws.data_ptr(), ws.numel()
+
+
+def _scratch_ptr(index: int, need: int):
+    w = _scratch(torch.device("cuda", index), need)
+    return w.data_ptr(), w.numel()
+
+
+# The native host path (csrc/fastcall.cpp): ``_fast_linear(kind, x, q, sz, group, nd)`` and ``_fast_moe(...)``
+# return the result of a plain call and None for every other, which then takes the Python path below
+# with its conversions and checks. Bound on first use; without the module every call takes the Python path.
+_FAST_LOCK = threading.Lock()
+
+
+def _bind_fast() -> None:
+    global _fast_linear, _fast_moe
+    with _FAST_LOCK:
+        if _fast_linear is not _first_linear:
+            return
+        try:
+            m = _lib.fast(_scratch_ptr)
+            linear, moe = m.linear, m.moe
+        except _lib.ImqUnavailable as exc:
+            print(f"[imq] native host path unavailable ({exc}) -> Python host path", flush=True)
+            linear = moe = lambda *a: None      # noqa: E731
+        _fast_linear, _fast_moe = linear, moe
+
+
+def _first_linear(*a):
+    _bind_fast()
+    return _fast_linear(*a)
+
+
+def _first_moe(*a):
+    _bind_fast()
+    return _fast_moe(*a)
+
+
+_fast_linear, _fast_moe = _first_linear, _first_moe
 
 
 def _check_expert_ids(idx: torch.Tensor, E: int) -> None:
@@ -222,6 +262,8 @@ def _linear_g(fn: str, codes_per_byte: int, x, qweight, group_size: int, sz, out
 def linear_w4(x, qweight, group_size: int, sz, out=None):
     """``op(x[M,Kpad] bf16, qweight u8[N,Kpad/2], group, (scale, zero)) -> y[M,N] bf16``: the
     signature of the op returned by the reference's _w4a16_triton_op (worker_quant.py:1180-1217)."""
+    if out is None and (y := _fast_linear(4, x, qweight, sz, group_size, False)) is not None:
+        return y
     return _linear_g("imq_linear_w4", 2, x, qweight, group_size, sz, out)
 
 
@@ -229,6 +271,8 @@ def linear_w4_tiled(x, qweight_tiled, group_size: int, sz, out=None):
     """``linear_w4`` on int4 weights in the line-tiled layout (``line_tile``): the same results
     bit for bit. ``qweight_tiled`` is the dense u8 [N, Kpad/2] tiled array (N a multiple of 16,
     Kpad of 256, groups of 128); shapes no tiled-layout kernel takes raise ImqError."""
+    if out is None and (y := _fast_linear(20, x, qweight_tiled, sz, group_size, False)) is not None:
+        return y
     if group_size != 128:
         raise ValueError("line-tiled int4 weights take groups of 128")
     if not qweight_tiled.is_contiguous():
@@ -239,6 +283,8 @@ def linear_w4_tiled(x, qweight_tiled, group_size: int, sz, out=None):
 def linear_w2_tiled(x, qweight_tiled, group_size: int, sz, out=None):
     """``linear_w2`` on int2 weights in the line-tiled layout (``line_tile``): the dense u8
     [N, Kpad/4] tiled array (N a multiple of 16, Kpad of 512, groups of 64)."""
+    if out is None and (y := _fast_linear(18, x, qweight_tiled, sz, group_size, False)) is not None:
+        return y
     if group_size != 64:
         raise ValueError("line-tiled int2 weights take groups of 64")
     if not qweight_tiled.is_contiguous():
@@ -293,6 +339,8 @@ def line_untile(qweight_tiled, out=None):
 def linear_w8_tiled(x, qweight_tiled, scale, out=None):
     """``linear_w8`` on int8 weights in the line-tiled layout (``line_tile``): the dense int8 [N, K]
     tiled array (N a multiple of 16, K of 128); the same results bit for bit."""
+    if out is None and (y := _fast_linear(24, x, qweight_tiled, scale, 0, False)) is not None:
+        return y
     dev = _check_dev(x, qweight_tiled, scale)
     _check_packed(qweight_tiled, torch.int8)
     if not qweight_tiled.is_contiguous():
@@ -312,11 +360,15 @@ def linear_w8_tiled(x, qweight_tiled, scale, out=None):
 
 def linear_w2(x, qweight, group_size: int, sz, out=None):
     """int2 twin (worker_quant.py:1876-1910): qweight u8 [N, Kpad/4]."""
+    if out is None and (y := _fast_linear(2, x, qweight, sz, group_size, False)) is not None:
+        return y
     return _linear_g("imq_linear_w2", 4, x, qweight, group_size, sz, out)
 
 
 def linear_w8(x, qweight, scale, out=None):
     """``op(x, qweight int8[N,K], scale[N,1]) -> y bf16 [M,N]`` (worker_quant.py:1022-1048)."""
+    if out is None and (y := _fast_linear(8, x, qweight, scale, 0, False)) is not None:
+        return y
     dev = _check_dev(x, qweight, scale)
     _check_packed(qweight, torch.int8)
     x = _rows2d(x)
@@ -330,6 +382,18 @@ def linear_w8(x, qweight, scale, out=None):
         call("imq_linear_w8", _ptr(x), x.stride(0), M, K, _ptr(qweight), qweight.stride(0), _ptr(scale),
              scale.stride(0), dtype_code(scale.dtype), N, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
     return y
+
+
+# Group-wise ops a module may call through the native path itself (worker_quant's forward).
+for _op, _kind in ((linear_w4, 4), (linear_w4_tiled, 20), (linear_w2, 2), (linear_w2_tiled, 18)):
+    _op.fast_kind = _kind
+
+
+def linear_nd(op, x, qweight, group_size: int, sz):
+    """``op`` over the leading sizes of x (any rank, bf16, its last size the packed K) through the native
+    path, or None when the call is not a plain one or ``op`` not one of this module's."""
+    kind = getattr(op, "fast_kind", 0)
+    return _fast_linear(kind, x, qweight, sz, group_size, True) if kind else None
 
 
 # ---------------------------------------------------------------------------------------------
@@ -387,6 +451,10 @@ def moe_experts_w4(hidden, topk_idx, topk_w, gu, dn, group_size: int, workspace=
     Routing ids outside [0, E) raise ValueError, as the reference's eager loop does
     (``check_ids``: one device-to-host read per call, skipped under graph capture). Without a
     ``workspace`` the call uses the cached per-(device, stream) workspace."""
+    if not check_ids and workspace is None and act in _ACT:
+        y = _fast_moe(hidden, topk_idx, topk_w, gu, dn, group_size, _ACT[act], gu_bias, dn_bias, alpha, limit)
+        if y is not None:
+            return y
     gq, gs, gz, H = gu
     dq, ds, dz, I = dn
     dev = _check_dev(hidden, topk_idx, topk_w, gq, gs, gz, dq, ds, dz)

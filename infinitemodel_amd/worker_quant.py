@@ -340,6 +340,14 @@ def _dealias_rows(qw):
     return buf[:, :qw.shape[1]]
 
 
+def _linear_nd(op, x, packed, group_size: int, pair):
+    """A plain fused call through the native host path (ops.linear_nd), else None."""
+    if not getattr(op, "fast_kind", 0):
+        return None
+    from . import ops
+    return ops.linear_nd(op, x, packed, group_size, pair)
+
+
 # ---- group-wise int4 / int2 linear modules ---------------------------------------------------
 def _line_tiling_fits(mod, bits: int, in_pad: int) -> bool:
     """Whether a group-wise module's packed weight can take the line-tiled layout: rows a multiple
@@ -525,6 +533,12 @@ def _make_group_linear_cls(bits: int):
             return not (threshold and self.qweight is not None and _m_bucket(_rows(x)) >= threshold)
 
         def forward(self, x):
+            d = self.__dict__
+            fused = d.get("_fused")
+            if fused is not None and not d.get("_naive_m_min") and fused[3] == self.in_features:
+                y = _linear_nd(fused[2], x, fused[0], self.group_size, fused[1])
+                if y is not None:
+                    return y if self.bias is None else y + self.bias.to(y.dtype)
             if self._takes_fused(x):
                 packed, pair, op, in_pad = self._fused
                 xs = x.reshape(-1, self.in_features).to(torch.bfloat16)
