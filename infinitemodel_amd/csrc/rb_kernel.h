@@ -244,7 +244,10 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   // VALU instructions). gemm_rb keeps every offset below 2^31.
   constexpr bool BUF = MOE == 0;
   const uint16_t* xtile = a.x + (int64_t)m0 * a.sxm;
-  int xo[XC], xl[XC];
+  // a thread's chunks are 32 rows (4096 bytes of LDS) apart: the swizzle repeats every 16 rows
+  int xo[XC];
+  const int xl0 = 2 * rb_swz(tid >> 3, tid & 7);
+  static_assert(NTHR == 256, "chunk j of a thread: row tid / 8 + 32 j");
   // MoE forms: the block's routed rows RID[row] = perm[prow0 + row] (0 past cnt), staged in LDS by
   // plan_a for the row-sum staging and down's scatter. A wave's lanes of chunk j cover 8
   // consecutive rows, whose perm entries are one scalar load (the workspace keeps BM spare
@@ -275,7 +278,6 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
         r = MOE == 3 ? prow0 + (ok ? row : cnt - 1) : (ok ? pr / a.k : 0);
       }
       xo[j] = ((int)(r * a.sxm) + ch * 8) * (BUF ? 2 : 1);   // BUF: bytes
-      xl[j] = 2 * rb_swz(row, ch);                    // bytes
     }
   };
   // ---- weight load plan: columns n0 + 64 wave + 32 j + c (MOE 1: gate column tn 32 NW + 32 wave
@@ -509,7 +511,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   auto store_a = [&](auto setc, uint16_t* A) {
     constexpr int set = decltype(setc)::value;
 #pragma unroll
-    for (int j = 0; j < XC; ++j) *(u32x4_t*)((char*)A + xl[j]) = FOLD ? permute_x8(xr[set][j]) : xr[set][j];
+    for (int j = 0; j < XC; ++j) *(u32x4_t*)((char*)A + xl0 + 4096 * j) = FOLD ? permute_x8(xr[set][j]) : xr[set][j];
   };
 
   // acc: the running sums (FOLD: the current group's sums of x (128 + q)); tot: FOLD's total
@@ -592,69 +594,44 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
     scale_pair(bsc, sv, nz);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      // operands of the next slice (slice 0 of step kt+1 at s = 3) into the other register pair,
-      // while this slice's MFMAs read the pair filled one slice earlier
+      // the A fragments of the next slice (slice 0 of step kt+1 at s = 3) first, into the register pair
+      // the previous slice's MFMAs have read: a whole slice of MFMAs covers their LDS latency
       if (s < 3) {
-        if ((s & 1) == 0) {
+        if ((s & 1) == 0) read_frags(std::integral_constant<int, 1>{}, Ar, s + 1);
+        else read_frags(std::integral_constant<int, 0>{}, Ar, s + 1);
+      } else {
+        read_frags(std::integral_constant<int, 0>{}, Aw, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // the next slice's B operands, converted between this slice's MFMAs
+      if (s < 3) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) bq[1][j] = b_frag(bsc, s + 1, j, sv[j], nz[j]);
-          read_frags(std::integral_constant<int, 1>{}, Ar, s + 1);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 2; ++j) bq[0][j] = b_frag(bsc, s + 1, j, sv[j], nz[j]);
-          read_frags(std::integral_constant<int, 0>{}, Ar, s + 1);
-        }
+        for (int j = 0; j < 2; ++j) bq[(s + 1) & 1][j] = b_frag(bsc, s + 1, j, sv[j], nz[j]);
       } else {
         float sv2[2], nz2[2];
         scale_pair(std::integral_constant<int, as>{}, sv2, nz2);
 #pragma unroll
         for (int j = 0; j < 2; ++j) bq[0][j] = b_frag(std::integral_constant<int, as>{}, 0, j, sv2[j], nz2[j]);
-        read_frags(std::integral_constant<int, 0>{}, Aw, 0);
       }
-      if ((s & 1) == 0) {
-        // FOLD, first slice of a group (even step): fold the previous group's sums into the
-        // total with its scale, then start the group's sums from zero
-        constexpr bool group_start = FOLD && bs % 2 == 0;
 #pragma unroll
-        for (int i = 0; i < IB; ++i)
+      for (int i = 0; i < IB; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            if (group_start && s == 0) {
-              if constexpr (FOLD) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) tot[i][j][r] = fmaf(sfold[j], acc[i][j][r], tot[i][j][r]);
-              }
-              acc[i][j] = mfma32x32x16(af[0][i], bq[0][j], f32x16_t{});
-            } else {
-              acc[i][j] = mfma32x32x16(af[0][i], bq[0][j], acc[i][j]);
-            }
-          }
-        if (group_start && s == 0) {
-          sfold[0] = sv[0];
-          sfold[1] = sv[1];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < IB; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x16(af[1][i], bq[1][j], acc[i][j]);
-      }
+        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x16(af[s & 1][i], bq[s & 1][j], acc[i][j]);
       if (s == 0) store_a(std::integral_constant<int, as>{}, Aw);
+      // one MFMA, then a few VALU operations, repeated (and slice 0's LDS writes after its first MFMAs)
+#pragma unroll
+      for (int k = 0; k < 2 * IB; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
+        if (s == 0 && k >= IB) __builtin_amdgcn_sched_group_barrier(0x200, XC / IB, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
       if (s == 1) {
         lds_barrier();
         load_a(std::integral_constant<int, as>{}, kt + 1 + PD);
         __builtin_amdgcn_sched_barrier(0);
       }
-      // one MFMA, then a few VALU and one LDS read, repeated: keeps the dequant and the fragment
-      // reads between MFMAs instead of bunched before them
-#pragma unroll
-      for (int k = 0; k < 2 * IB; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
     }
-    __builtin_amdgcn_sched_barrier(0);
     load_b(bsc, kt + PD);
     load_s(bsc, kt + PD);
     __builtin_amdgcn_sched_barrier(0);
