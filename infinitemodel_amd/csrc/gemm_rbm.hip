@@ -21,9 +21,10 @@ double planes_us(int s, int64_t M, int64_t N) { return s > 1 ? 4.5 + 1e-6 * s * 
 
 // The tile plan, the cheapest by a model fitted to sweeps of heights and splits over 4096 x 4096 .. 28672 at
 // M 96 .. 2048 (it picks the measured best or one within 5%): a 64-code step of an ib x 32 row, 256-column
-// tile takes 0.55 + 0.17 ib us (int8 0.45 + 0.15 ib); heights up to 128 rows keep two workgroups on a CU,
-// whose steps then overlap to 0.89 of that each. Row blocks are spread evenly over the row tiles (777 rows:
-// 4 tiles of 7 blocks, not 4 of 8). Returns the modelled us.
+// tile takes 0.46 + 0.163 ib us (int8 0.32 + 0.145 ib); int4 / int2 steps 15% more once K is split more than
+// two ways (short ranges expose the load latency their unpack otherwise hides); heights up to 128 rows
+// keep two workgroups on a CU, whose steps then overlap to 0.89 of that each. Row blocks are spread
+// evenly over the row tiles (777 rows: 4 tiles of 7 blocks, not 4 of 8). Returns the modelled us.
 double rbm_plan(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes, RbmPlan* p) {
   const int KT = (int)(K / RB_BK);
   const int64_t blocks = imq_cdiv(M, 32), cols = imq_cdiv(N, 256);
@@ -33,11 +34,12 @@ double rbm_plan(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes,
     const int ib = (int)imq_cdiv(blocks, rt);
     if (ib < 3) break;
     if (rt > rt0 && ib == (int)imq_cdiv(blocks, rt - 1)) continue;   // the same height with idle tiles
-    const double t = bits == 8 ? 0.45 + 0.15 * ib : 0.55 + 0.17 * ib;
+    const double t1 = bits == 8 ? 0.32 + 0.145 * ib : 0.46 + 0.163 * ib;
     for (int s = 1; s <= (planes ? 8 : 1); ++s) {
       const int kps = (KT + s - 1) / s;
       const int64_t W = rt * cols * s;
       if (s > 1 && ((s - 1) * kps >= KT || kps < 8 || W > 2 * (int64_t)cus || 4ll * s * M * N > rbm_max_planes(M))) break;
+      const double t = bits != 8 && s > 2 ? 1.15 * t1 : t1;
       double us;
       if (W <= cus) us = kps * t;
       else if (ib <= 4) us = (double)((W + 2 * cus - 1) / (2 * cus)) * kps * 2 * 0.89 * t;
@@ -64,8 +66,8 @@ bool rbm_takes(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, bo
   if (M <= 64 || N <= 0 || K <= 0 || K % RB_BK != 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return false;
   if (bits != 8 && (G < 32 || (G & (G - 1)) != 0)) return false;
   const double us = rbm_plan(bits, M, N, K, cus, planes, p);
-  // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within 7% (its own spread)
-  return us > 0 && (M > 512 || us < 0.93 * lds_us(M, N, K, cus, planes));
+  // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within its own spread
+  return us > 0 && (M > 512 || us < 0.96 * lds_us(M, N, K, cus, planes));
 }
 
 }  // namespace
