@@ -72,18 +72,23 @@ constexpr int wk_rj(int ib, int jb) { return ib == 1 && jb > 1 ? 2 : 1; }
 
 // LDS bytes: the waves' activation steps (reused by the sums), then the scale / zero pairs of the
 // groups a range of kps K steps touches (one more when ranges start inside a group).
-inline size_t wk_lds_bytes(int bits, int ib, int jb, int kps, int gsh) {
+inline size_t wk_lds_bytes(int bits, int ib, int jb, int kps, int gsh, int waves = WK_WAVES) {
   const size_t groups = bits == 8 ? 0 : (size_t)((((int64_t)kps * RB_BK) >> gsh) + 2);
-  return (size_t)WK_WAVES * ib * wk_rj(ib, jb) * 4096 + groups * wk_szs(jb) * 4;
+  return (size_t)waves * ib * wk_rj(ib, jb) * 4096 + groups * wk_szs(jb) * 4;
 }
 
 // PA / PW: steps of activations / weights in flight per wave (PW a multiple of PA); MINW: waves per
 // SIMD the registers are bounded for.
-template <int BITS, int IB, int JB, bool TL, int PA, int PW, int MINW>
-__global__ __launch_bounds__(64 * WK_WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
+// FOLD (M <= 16, groups of 64 codes or more): the decode rows' arithmetic, no weight rounded: B holds the
+// codes themselves, a step's sums start from zero and are folded into the total with the step's scale, and
+// the zero point comes in through the rows' sums (an MFMA against ones): sum s (c - z) x = s (sum c x) -
+// z s (sum x).
+template <int BITS, int IB, int JB, bool TL, int PA, int PW, int MINW, int WAVES = WK_WAVES, bool FOLD = false>
+__global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
   static_assert(PW % PA == 0 && PW >= 2 && PW <= 4, "rings");
-  constexpr int BK = RB_BK, BN = 32 * JB, NTHR = 64 * WK_WAVES;
-  constexpr int XC = 4 * IB;                       // 16-byte activation loads per lane per step
+  static_assert(!FOLD || (IB == 1 && BITS != 8), "folded form: up to 16 rows of a group format");
+  constexpr int BK = RB_BK, BN = 32 * JB, NTHR = 64 * WAVES;
+  constexpr int XC = FOLD ? 2 : 4 * IB;            // 16-byte activation loads per lane per step (8 rows each)
   constexpr int SZS = wk_szs(JB), RJ = wk_rj(IB, JB);
   constexpr int QV = BITS == 8 ? 2 : 1, QB = 4 * BITS;
   using QT = std::conditional_t<BITS == 2, u32x2_t, u32x4_t>;
@@ -94,9 +99,9 @@ __global__ __launch_bounds__(64 * WK_WAVES, MINW) void gemm_wk_kernel(WkArgs a) 
   const int n0 = (blockIdx.x - split * a.tiles_n) * BN;
   const int kt0 = split * a.kps;
   const int KT = min(a.K / BK - kt0, a.kps);       // >= 1 (the plan leaves no empty range)
-  const int steps = KT > wave ? (KT - wave + WK_WAVES - 1) / WK_WAVES : 0;
+  const int steps = KT > wave ? (KT - wave + WAVES - 1) / WAVES : 0;
   char* const Aw = wk_lds + wave * (IB * RJ * 4096);   // this wave's activation step, [32 IB rows][64] bf16
-  uint32_t* const SZ = (uint32_t*)(wk_lds + WK_WAVES * IB * RJ * 4096);
+  uint32_t* const SZ = (uint32_t*)(wk_lds + WAVES * IB * RJ * 4096);
 
   // ---- load plan: offsets from the tile's first row, fixed for the whole loop; the step's part is
   // uniform. Rows past M repeat row M - 1, columns past N column N - 1 (never stored). --------------
@@ -124,7 +129,7 @@ __global__ __launch_bounds__(64 * WK_WAVES, MINW) void gemm_wk_kernel(WkArgs a) 
 
   u32x4_t xr[PA][XC];
   QT qr[PW][JB][QV];
-  auto kt_of = [&](int i) { return kt0 + min(wave, KT - 1) + WK_WAVES * max(min(i, steps - 1), 0); };
+  auto kt_of = [&](int i) { return kt0 + min(wave, KT - 1) + WAVES * max(min(i, steps - 1), 0); };
   auto load_a = [&](auto setc, int i) {
     const int kt = kt_of(i);
 #pragma unroll
@@ -215,8 +220,27 @@ __global__ __launch_bounds__(64 * WK_WAVES, MINW) void gemm_wk_kernel(WkArgs a) 
       }
     }
     load_a(setc, i + PA);
+    f32x16_t part[FOLD ? JB : 1], xs;                        // FOLD: the step's sums of c x and of x
+    if constexpr (FOLD) {
+      const uint32_t one2 = 0x3f803f80u;
+      const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, u32x4_t{one2, one2, one2, one2});
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+      for (int s = 0; s < 4; ++s) {
+        const bf16x8_t af = *(const bf16x8_t*)(Aw + aoff[s]);
+        xs = mfma32x32x16(af, ones, s == 0 ? f32x16_t{} : xs);
+#pragma unroll
+        for (int j = 0; j < JB; ++j) {
+          const u32x4_t d = codes8_bf16<BITS>(qr[set][j][0][BITS == 4 ? s : s >> 1], s & 1);
+          part[j] = mfma32x32x16(af, __builtin_bit_cast(bf16x8_t, d), s == 0 ? f32x16_t{} : part[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < JB; ++j)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) acc[0][j][r] = fmaf(nz[j], xs[r], fmaf(s_[j], part[j][r], acc[0][j][r]));   // rows < 16
+    }
+#pragma unroll
+    for (int s = 0; s < (FOLD ? 0 : 4); ++s) {
       bf16x8_t af[IB];
 #pragma unroll
       for (int b = 0; b < IB; ++b) af[b] = *(const bf16x8_t*)(Aw + aoff[s] + b * 4096);
@@ -267,7 +291,7 @@ __global__ __launch_bounds__(64 * WK_WAVES, MINW) void gemm_wk_kernel(WkArgs a) 
       const int u = q / (IB * 256), b = (q >> 8) % IB, r4 = (q >> 6) & 3, l = q & 63;
       f32x4_t v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int w = 0; w < WK_WAVES; ++w) v += *(const f32x4_t*)(wk_lds + w * (IB * RJ * 4096) + q * 16);
+      for (int w = 0; w < WAVES; ++w) v += *(const f32x4_t*)(wk_lds + w * (IB * RJ * 4096) + q * 16);
       const int n = n0 + 32 * (j + u) + (l & 31), m0 = 32 * b + 8 * r4 + 4 * (l >> 5);
       if (n >= a.N) continue;
       if (a.splits > 1) {
@@ -304,6 +328,29 @@ int wk_launch(const WkArgs& a, hipStream_t st) {
     }
   }
   kern<<<dim3((unsigned)(a.tiles_n * a.splits)), dim3(64 * WK_WAVES), lds, st>>>(a);
+  IMQ_LAUNCH_CHECK();
+  return IMQ_OK;
+}
+
+// The folded form: decode rows whose K no line or K-split kernel takes. us, generic kernel (one wave per row,
+// a code at a time) -> this: int2 12096 -> 1344 M = 1 / 7 / 16 113 / 221 / 385 -> 15, 3520 -> 2560 41 / 74 / 116 ->
+// 9; bound by its 24 K steps per wave in turn. One 32-column block per workgroup, 16 waves (decode shapes are short of workgroups,
+// not of columns), K unsplit.
+constexpr int WKD_WAVES = 16;
+template <int BITS>
+int wkd_launch(const WkArgs& a, hipStream_t st) {
+  const size_t lds = wk_lds_bytes(BITS, 1, 1, a.kps, a.gsh, WKD_WAVES);
+  auto kern = gemm_wk_kernel<BITS, 1, 1, false, 2, 2, 4, WKD_WAVES, true>;
+  if (lds > 65536) {
+    static int attr_set = 0;   // benign race: every caller sets the same value
+    if (!__atomic_load_n(&attr_set, __ATOMIC_ACQUIRE)) {
+      hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         device_info().max_lds);
+      if (e != hipSuccess) return (int)e;
+      __atomic_store_n(&attr_set, 1, __ATOMIC_RELEASE);
+    }
+  }
+  kern<<<dim3((unsigned)a.tiles_n), dim3(64 * WKD_WAVES), lds, st>>>(a);
   IMQ_LAUNCH_CHECK();
   return IMQ_OK;
 }

@@ -9,6 +9,8 @@ namespace imq {
 int wk_run4(const WkArgs& a, int jb, bool tiled, hipStream_t st);
 int wk_run2(const WkArgs& a, int jb, bool tiled, hipStream_t st);
 int wk_run8(const WkArgs& a, int jb, bool tiled, hipStream_t st);
+int wkd_run2(const WkArgs& a, hipStream_t st);
+int wkd_run4(const WkArgs& a, hipStream_t st);
 
 namespace {
 
@@ -98,6 +100,22 @@ int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, cons
     case IMQ_DT_FP32: return splitk_sum<8, IMQ_DT_FP32>(a.part, p.splits, a.M, a.N, sc, ssn, y, sym, st);
   }
   return IMQ_ERR_INVALID;
+}
+
+// Decode rows (M <= 16) the decode kernels do not take for their K: the folded form, row layout, K a multiple
+// of 64, groups of 2^k >= 64 codes, any dtypes and scale strides. IMQ_ERR_UNSUPPORTED: the generic kernel's.
+int gemm_wkd(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+             int64_t N, int64_t G, uint16_t* y, int64_t sym, hipStream_t st) {
+  if (M < 1 || M > 16 || K % RB_BK != 0 || G < RB_BK || (G & (G - 1)) != 0 || N > (1 << 30)) return IMQ_ERR_UNSUPPORTED;
+  const int qa = bits == 2 ? 8 : 16;               // a lane's load
+  if (((uintptr_t)x & 15) || (sxm & 7) || ((uintptr_t)q % qa) || sqn % qa) return IMQ_ERR_UNSUPPORTED;
+  if ((16 * sxm + K) * 2 > 0x7fffffff || 32 * sqn + K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
+  const int gsh = wk_gsh(bits, G), KT = (int)(K / RB_BK);
+  if (wk_lds_bytes(bits, 1, 1, KT, gsh, WKD_WAVES) > (size_t)device_info().max_lds) return IMQ_ERR_UNSUPPORTED;
+  const WkArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, sdt, zdt, (int)N, gsh, y, sym,
+                 (int)imq_cdiv(N, 32), 1, KT, nullptr};
+  return bits == 4 ? wkd_run4(a, st) : wkd_run2(a, st);
 }
 
 }  // namespace imq

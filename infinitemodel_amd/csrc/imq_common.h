@@ -119,15 +119,14 @@ IMQ_DEV float raw_to_bf16_f32(uint32_t r) {
   else return round_bf16_hw(__uint_as_float(r));
 }
 
-// 8 int4 (BITS 4: the nibbles of w) or int2 (BITS 2: the crumbs of 16-bit half `half` of w) codes -> 4
-// dwords of bf16 (c - z) s in K order: fma(c, s, -z s) is the exact product, rounded once by the
-// pack. A code 0..15 in a byte is the fp8 e4m3 value c 2^-9 (codes below 8 are its subnormals, 8..15
-// its first binade), so one v_cvt_scalef32_pk_f32_fp8 at scale 2^9 converts two codes exactly. That and
-// the packs run at 4 cycles per wave, plain fp32 and logic at 2: 54 cycles per 8 int4 codes
-// against 70 with v_cvt_f32_ubyteN (one code each), 55 against 96 for int2 with its bit-field extracts.
+// 8 int4 (BITS 4: the nibbles of w) or int2 (BITS 2: the crumbs of 16-bit half `half` of w) codes as exact
+// fp32 in K order, c[i] = code i. A code 0..15 in a byte is the fp8 e4m3 value c 2^-9 (codes below 8
+// are its subnormals, 8..15 its first binade), so one v_cvt_scalef32_pk_f32_fp8 at scale 2^9 converts two
+// codes exactly. That and the bf16 packs run at 4 cycles per wave, plain fp32 and logic at 2: with the
+// fma and packs of dequant8_bf16, 54 cycles per 8 int4 codes against 70 with v_cvt_f32_ubyteN (one code
+// each), 55 against 96 for int2 with its bit-field extracts.
 template <int BITS>
-IMQ_DEV u32x4_t dequant8_bf16(uint32_t w, int half, float s, float nzs) {
-  u32x4_t r;
+IMQ_DEV void codes8_f32(uint32_t w, int half, float* c) {
   auto pair = [&](uint32_t bytes, bool hi) -> f32x2_t {
     return hi ? __builtin_bit_cast(f32x2_t, __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)bytes, 512.f, true))
               : __builtin_bit_cast(f32x2_t, __builtin_amdgcn_cvt_scalef32_pk_f32_fp8((int)bytes, 512.f, false));
@@ -137,20 +136,42 @@ IMQ_DEV u32x4_t dequant8_bf16(uint32_t w, int half, float s, float nzs) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       const f32x2_t e = pair(even, p), o = pair(odd, p);
-      r[2 * p] = cvt_pk_bf16(fmaf(e[0], s, nzs), fmaf(o[0], s, nzs));
-      r[2 * p + 1] = cvt_pk_bf16(fmaf(e[1], s, nzs), fmaf(o[1], s, nzs));
+      c[4 * p] = e[0];
+      c[4 * p + 1] = o[0];
+      c[4 * p + 2] = e[1];
+      c[4 * p + 3] = o[1];
     }
   } else {
     // byte i of plane j holds code 4 i + j, the half's bytes codes j and 4 + j
-    f32x2_t c[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) c[j] = pair((w >> (2 * j)) & 0x03030303u, half != 0);
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      r[2 * p] = cvt_pk_bf16(fmaf(c[0][p], s, nzs), fmaf(c[1][p], s, nzs));
-      r[2 * p + 1] = cvt_pk_bf16(fmaf(c[2][p], s, nzs), fmaf(c[3][p], s, nzs));
+    for (int j = 0; j < 4; ++j) {
+      const f32x2_t v = pair((w >> (2 * j)) & 0x03030303u, half != 0);
+      c[j] = v[0];
+      c[4 + j] = v[1];
     }
   }
+}
+
+// Those codes -> 4 dwords of bf16 (c - z) s in K order: fma(c, s, -z s) is the exact product, rounded once by
+// the pack.
+template <int BITS>
+IMQ_DEV u32x4_t dequant8_bf16(uint32_t w, int half, float s, float nzs) {
+  float c[8];
+  codes8_f32<BITS>(w, half, c);
+  u32x4_t r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = cvt_pk_bf16(fmaf(c[2 * i], s, nzs), fmaf(c[2 * i + 1], s, nzs));
+  return r;
+}
+
+// Those codes themselves as bf16, exact.
+template <int BITS>
+IMQ_DEV u32x4_t codes8_bf16(uint32_t w, int half) {
+  float c[8];
+  codes8_f32<BITS>(w, half, c);
+  u32x4_t r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = cvt_pk_bf16(c[2 * i], c[2 * i + 1]);
   return r;
 }
 

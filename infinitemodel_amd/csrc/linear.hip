@@ -38,6 +38,15 @@ void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out);
 void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out);
 void rbm_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int64_t* out);
 void rb_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int64_t* out);
+int gemm_wkd(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+             int64_t N, int64_t G, uint16_t* y, int64_t sym, hipStream_t st);
+// Whether decode rows go to the folded short-batch form before the skinny kernels: K not whole line-steps (no
+// line or K-split kernel reads it), more than 8 rows, K long enough that a wave has several steps. us, skinny
+// -> folded: int4 2880 -> 5120 (K_pad 2944) M = 12 / 16 15.5 / 17.4 -> 13.5 / 13.7, int2 11008 -> 4096 M = 8 / 16
+// 17.8 / 31.7 -> 15.8 / 17.6, 3328 -> 4096 M = 16 11.3 -> 9.0; M = 4 11.7 -> 13.2 and short K (768 -> 16384
+// M = 16 10.7 -> 12.4) stay.
+bool folded_first(int bits, int64_t M, int64_t K) { return M > 8 && M <= 16 && K >= 2048 && K % (1024 / bits) != 0; }
 template <int BITS>
 int generic_gemv(const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
                  const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn,
@@ -141,6 +150,11 @@ extern "C" int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int
   const uint16_t* xb = (const uint16_t*)x;
   uint16_t* yb = (uint16_t*)y;
   const uint8_t* q = (const uint8_t*)qweight;
+  if (imq::folded_first(4, M, K_pad)) {
+    rc = imq::gemm_wkd(4, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                       z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
+    if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  }
   if (M <= 16) {
     rc = imq::skinny_w4(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype,
                         zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, workspace,
@@ -150,6 +164,9 @@ extern "C" int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int
                       s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride,
                       workspace, workspace_bytes, st);
   }
+  if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  rc = imq::gemm_wkd(4, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                     z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
   if (rc != IMQ_ERR_UNSUPPORTED) return rc;
   return imq::generic_gemv<4>(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g,
                               s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb,
@@ -306,6 +323,11 @@ extern "C" int imq_linear_w2(const void* x, int64_t x_row_stride, int64_t M, int
   const uint16_t* xb = (const uint16_t*)x;
   uint16_t* yb = (uint16_t*)y;
   const uint8_t* q = (const uint8_t*)qweight;
+  if (imq::folded_first(2, M, K_pad)) {
+    rc = imq::gemm_wkd(2, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                       z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
+    if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  }
   if (M <= 16) {
     rc = imq::skinny_w2(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype,
                         zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, workspace,
@@ -315,6 +337,9 @@ extern "C" int imq_linear_w2(const void* x, int64_t x_row_stride, int64_t M, int
                       s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride,
                       workspace, workspace_bytes, st);
   }
+  if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  rc = imq::gemm_wkd(2, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                     z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
   if (rc != IMQ_ERR_UNSUPPORTED) return rc;
   return imq::generic_gemv<2>(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g,
                               s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb,

@@ -102,3 +102,32 @@ def test_without_a_workspace_and_repeated(dev):
         yg.zero_()
         g.replay()
         assert torch.equal(yg, y) and torch.equal(ops.linear_w4(xt, q, 128, (s, z)), y)
+
+
+@pytest.mark.parametrize("M,N,K,bits,G,sdt,zdt", [
+    (1, 37, 64, 2, 64, "fp16", "fp16"), (3, 100, 192, 2, 64, "bf16", "fp32"), (16, 1344, 12096, 2, 64, "fp16", "fp16"),
+    (7, 2560, 3520, 2, 64, "bf16", "bf16"), (5, 33, 28736, 2, 64, "fp16", "fp16"), (2, 70, 1152, 2, 128, "fp32", "bf16"),
+    (1, 37, 448, 4, 64, "bf16", "bf16"), (16, 300, 1088, 4, 64, "fp16", "bf16"), (4, 96, 320, 4, 64, "bf16", "bf16"),
+    (9, 300, 2944, 4, 128, "bf16", "bf16"), (16, 130, 11008, 2, 64, "fp16", "fp16")])
+def test_decode_rows_of_odd_k_match_the_exact_product(dev, M, N, K, bits, G, sdt, zdt):
+    """Decode rows whose K no decode kernel takes: the folded form rounds no weight, so its results are
+    the exact (q - z) s product's to fp32 summation, strided operands included."""
+    import torch
+    from infinitemodel_amd import ops
+    r = C.rng(M + N + K)
+    codes = r.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    q = np.zeros((N, K * bits // 8), np.uint8)
+    for i in range(8 // bits):
+        q |= codes[:, i::8 // bits] << (bits * i)
+    s = oq.round_to(r.uniform(0.005, 0.05, (N, K // G)).astype(np.float32), sdt)
+    z = oq.round_to(r.uniform(0, (1 << bits) - 1, (N, K // G)).astype(np.float32), zdt)
+    x = C.bf16_normal(C.rng(M), (M, K))
+    op = ops.linear_w4 if bits == 4 else ops.linear_w2
+    st, zt = C.to_torch(s, sdt, dev), C.to_torch(z, zdt, dev)
+    y = op(C.to_torch(x, "bf16", dev), C.u8(q, dev), G, (st, zt))
+    _check(y, x, oq.dequant_exact(codes, s, z, G, K))
+    xw = torch.full((M, K + 16), float("nan"), dtype=torch.bfloat16, device=dev)
+    xw[:, 8:8 + K] = C.to_torch(x, "bf16", dev)
+    qw = torch.zeros(N, q.shape[1] + 16, dtype=torch.uint8, device=dev)
+    qw[:, :q.shape[1]] = C.u8(q, dev)
+    assert torch.equal(op(xw[:, 8:8 + K], qw[:, :q.shape[1]], G, (st.t().contiguous().t(), zt.t().contiguous().t())), y)
