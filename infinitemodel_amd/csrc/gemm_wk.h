@@ -1,4 +1,4 @@
-// The short-batch GEMM (16 < M <= 64): weights dequantized in registers, K split over the waves of a
+// The short-batch GEMM (16 < M <= 64, int8 from 5 rows): weights dequantized in registers, K split over the waves of a
 // workgroup. One translation unit per weight format (gemm_wk4.hip, gemm_wk2.hip, gemm_wk8.hip); plan and
 // dispatch in gemm_wk.hip.
 //

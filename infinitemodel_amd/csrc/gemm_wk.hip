@@ -51,13 +51,23 @@ bool wk_plan(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int 
   return p->splits != 0;
 }
 
+// The row counts the form takes. int4 / int2: 17 to 64 (decode rows round no weight). int8, whose integers
+// are exact in bf16: from 5, where the skinny kernel restages the activations for every 16 rows of
+// weights -- us, skinny -> this at M = 5 / 16: 4096 -> 4096 10.3 / 13.6 -> 8.8 / 8.7, 14336 -> 4096 25.9 / 37.8 ->
+// 18.0 / 18.3, 4096 -> 14336 18.2 / 25.2 -> 15.8 / 16.3; at a vocabulary's width the skinny kernel's
+// persistent tiles win up to 8 rows (3584 -> 152064 M = 8 100 against 116, M = 16 144 against 121).
+bool wk_rows(int bits, int64_t M, int64_t N) {
+  if (bits == 8 && M <= 16) return M > 8 || (M > 4 && N <= 65536);
+  return M > 16 && M <= 64;
+}
+
 }  // namespace
 
 // The short-batch GEMM's plan of an M x N x K call (int8 when G is 0) on a device of `cus` CUs, without a
 // device: out = {takes the call, 32-column blocks per workgroup, K ranges}.
 void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out) {
   WkPlan p{0, 0};
-  const bool takes = M > 16 && M <= 64 && K % RB_BK == 0 && wk_plan(bits, M, N, K, G, cus, max_lds, 8, &p);
+  const bool takes = wk_rows(bits, M, N) && K % RB_BK == 0 && wk_plan(bits, M, N, K, G, cus, max_lds, 8, &p);
   out[0] = takes ? 1 : 0;
   out[1] = p.jb;
   out[2] = p.splits;
@@ -71,13 +81,14 @@ int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
   return s > 1 ? s * M * N * 4 : 0;
 }
 
-// 16 < M <= 64, K a multiple of 64; groups and strides checked by the caller (gemm_wq_any). Scale and
+// The rows of wk_rows, K a multiple of 64; groups and strides checked by the caller (gemm_wq_any; int8 has none). Scale and
 // zero of any dtype. IMQ_ERR_UNSUPPORTED for offsets beyond 32 bits or tiles no LDS holds: the
 // LDS-dequant GEMM takes those. Without a large enough workspace K is not split.
 int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled) {
-  if (M <= 16 || M > 64) return IMQ_ERR_UNSUPPORTED;
+  if (!wk_rows(bits, M, N) || K <= 0 || K % RB_BK != 0) return IMQ_ERR_UNSUPPORTED;
+  if (((uintptr_t)x & 15) || (sxm & 7) || ((uintptr_t)q & 15) || (sqn & 15)) return IMQ_ERR_UNSUPPORTED;
   if ((64 * sxm + K) * 2 > 0x7fffffff || 128 * sqn + K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
   const DevInfo d = device_info();
   WkPlan p;

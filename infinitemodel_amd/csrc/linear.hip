@@ -47,6 +47,9 @@ int gemm_wkd(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, con
 // 17.8 / 31.7 -> 15.8 / 17.6, 3328 -> 4096 M = 16 11.3 -> 9.0; M = 4 11.7 -> 13.2 and short K (768 -> 16384
 // M = 16 10.7 -> 12.4) stay.
 bool folded_first(int bits, int64_t M, int64_t K) { return M > 8 && M <= 16 && K >= 2048 && K % (1024 / bits) != 0; }
+int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
+            const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
+            int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled);
 template <int BITS>
 int generic_gemv(const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
                  const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn,
@@ -227,6 +230,24 @@ extern "C" int imq_linear_w2_tiled(const void* x, int64_t x_row_stride, int64_t 
                             z_stride_n, z_stride_g, z_dtype, N, yb, y_row_stride, workspace, workspace_bytes, st);
 }
 
+namespace {
+
+// int8 decode rows: from 5 the short-batch GEMM where it takes them (wk_rows, gemm_wk.hip), else the
+// line and skinny kernels. Of the workspace at most imq_linear_workspace_bytes is used, so a larger buffer
+// kept for other calls changes no result.
+int decode_w8(const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const void* q, int64_t sqn, const void* sc, int64_t ssn,
+              int sdt, int64_t N, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled) {
+  if (M > 4) {
+    const int64_t own = imq_linear_workspace_bytes(M, N, K);
+    const int rc = imq::gemm_wk(8, x, sxm, M, K, (const uint8_t*)q, sqn, sc, ssn, 0, sdt, nullptr, 0, 0, sdt, N, 0, y,
+                                sym, ws, wsb < own ? wsb : own, st, tiled);
+    if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  }
+  return imq::skinny_w8(x, sxm, M, K, (const int8_t*)q, sqn, sc, ssn, sdt, N, y, sym, st, tiled);
+}
+
+}  // namespace
+
 // int8 weights in the line-tiled layout: the arguments and results of imq_linear_w8 (N a multiple of
 // 16, dense rows of K bytes, K a multiple of 128); the decode line and skinny kernels and both
 // prefill GEMMs read it, other calls return IMQ_ERR_UNSUPPORTED.
@@ -242,8 +263,8 @@ extern "C" int imq_linear_w8_tiled(const void* x, int64_t x_row_stride, int64_t 
   const uint16_t* xb = (const uint16_t*)x;
   uint16_t* yb = (uint16_t*)y;
   if (M <= 16)
-    return imq::skinny_w8(xb, x_row_stride, M, K, (const int8_t*)qweight, q_row_stride, scale, s_stride_n, s_dtype,
-                          N, yb, y_row_stride, st, true);
+    return decode_w8(xb, x_row_stride, M, K, qweight, q_row_stride, scale, s_stride_n, s_dtype, N, yb, y_row_stride,
+                     workspace, workspace_bytes, st, true);
   return imq::gemm_wq_tiled(8, xb, x_row_stride, M, K, (const uint8_t*)qweight, scale, s_stride_n, 0, s_dtype,
                             nullptr, 0, 0, s_dtype, N, yb, y_row_stride, workspace, workspace_bytes, st);
 }
@@ -358,8 +379,8 @@ extern "C" int imq_linear_w8(const void* x, int64_t x_row_stride, int64_t M, int
   uint16_t* yb = (uint16_t*)y;
   int rc;
   if (M <= 16) {
-    rc = imq::skinny_w8(xb, x_row_stride, M, K, (const int8_t*)qweight, q_row_stride, scale, s_stride_n,
-                        s_dtype, N, yb, y_row_stride, st, false);
+    rc = decode_w8(xb, x_row_stride, M, K, qweight, q_row_stride, scale, s_stride_n, s_dtype, N, yb, y_row_stride,
+                   workspace, workspace_bytes, st, false);
   } else {
     rc = imq::gemm_wq(8, xb, x_row_stride, M, K, (const uint8_t*)qweight, q_row_stride, scale, s_stride_n,
                       0, s_dtype, nullptr, 0, 0, s_dtype, N, 0, yb, y_row_stride, workspace, workspace_bytes, st);

@@ -64,7 +64,8 @@ def test_group_formats_match_the_oracle(dev, M, N, K, bits, G, sdt, zdt):
 
 
 @pytest.mark.parametrize("M,N,K,sdt", [(17, 40, 64, "bf16"), (33, 272, 1152, "fp16"), (64, 1008, 14336, "fp32"),
-                                       (32, 14336, 4096, "fp16")])
+                                       (32, 14336, 4096, "fp16"), (5, 48, 128, "bf16"), (16, 4096, 14336, "fp16"),
+                                       (8, 65552, 128, "bf16"), (9, 65552, 128, "bf16"), (12, 37, 192, "fp32")])
 def test_int8_matches_the_oracle(dev, M, N, K, sdt):
     import torch
     from infinitemodel_amd import ops

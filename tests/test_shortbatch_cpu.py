@@ -21,7 +21,7 @@ def _szs(jb):
 
 CASES = [(4, 17, 28672, 4096, 128), (4, 64, 28672, 4096, 128), (4, 32, 4096, 14336, 128), (4, 20, 37, 64, 64),
          (4, 33, 1008, 448, 32), (2, 64, 8192, 28672, 64), (2, 17, 96, 448, 64), (8, 40, 4096, 14336, 0),
-         (8, 17, 40, 64, 0), (4, 24, 256, 8192, 128), (4, 17, 151936, 3584, 128)]
+         (8, 17, 40, 64, 0), (8, 5, 4096, 14336, 0), (8, 16, 152064, 3584, 0), (4, 24, 256, 8192, 128), (4, 17, 151936, 3584, 128)]
 
 
 @pytest.mark.parametrize("bits,M,N,K,G", CASES)
@@ -93,3 +93,5 @@ def test_tiled_offsets_are_the_layout(bits, K):
 def test_small_devices_and_other_rows_decline():
     assert _plan(4, 16, 4096, 4096, 128) is None and _plan(4, 65, 4096, 4096, 128) is None
     assert _plan(4, 17, 4096, 4096 + 32, 128) is None
+    assert _plan(8, 4, 4096, 4096, 0) is None and _plan(8, 5, 4096, 4096, 0) is not None      # int8 from 5 rows
+    assert _plan(8, 8, 65552, 4096, 0) is None and _plan(8, 9, 65552, 4096, 0) is not None
