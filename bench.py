@@ -413,7 +413,8 @@ def bench_c3(args, dev):
     else:
         kern = ("w2_line_kernel" if M == 1 else
                 "w2_ksplit_kernel + splitk_rows_reduce_kernel" if M <= 16 and (M > 4 or layout == "line-tiled") else
-                "w2_skinny_kernel" if M <= 16 else "gemm_wq_kernel<2>")
+                "w2_skinny_kernel" if M <= 16 else "gemm_wk_kernel<2>" if M <= 64
+                else "gemm_rb_kernel<2> / gemm_wq_kernel<2>, by plan")
     roof = _hbm_roofline(f"{kern} ({entry}, M={M})", nbytes / len(sets), us, _traffic(f"c3_m{M}"))
     cfg = {"workload": f"C3 int2 g64 70B shapes 8192->28672 and 28672->8192, M={M}, 8 copies each", "M": M,
            "launches_per_step": len(sets), "distinct_bytes_per_step": nbytes,
@@ -574,11 +575,15 @@ def bench_c4(args, dev):
     tf_dense = sum(2.0 * M * N * K for N, K, _ in dense_sets) / (ms_dense * 1e-3)
     del dense_sets
     bits = 4 if args.quant == "int4" else 8
-    gemm = (f"gemm_rb_kernel<{bits}> + splitk_sum_kernel (register-B GEMM" if M > 512
-            else f"gemm_wq_kernel<{bits}> + splitk_sum_kernel (LDS-dequant GEMM")
+    from infinitemodel_amd import _lib
+    gemm = " / ".join(
+        f"gemm_wk_kernel<{bits}> (short-batch GEMM)" if M <= 64
+        else f"gemm_rb_kernel<{bits}> (register-B GEMM)" if _lib.launch_plan(
+            _lib.IMQ_PLAN_GEMM_RBM, M, K, 128 if bits == 4 else 0, N, sqn=K * bits // 8)
+        else f"gemm_wq_kernel<{bits}> (LDS-dequant GEMM)" for N, K in ((14336, 4096), (4096, 14336)))
     roof = {"bound": "mfma", "achieved": round(tf / 1e12, 2), "peak": BF16_PEAK / 1e12, "unit": "TFLOP/s",
             "frac": round(tf / BF16_PEAK, 4), "traffic": _traffic(f"c4_{args.quant}_m{M}"),
-            "kernel": f"{gemm}, imq_linear_{'w4' if bits == 4 else 'w8'} prefill)",
+            "kernel": f"{gemm}, + splitk_sum_kernel where K is split; imq_linear_{'w4' if bits == 4 else 'w8'} prefill",
             "avg_launch_us": round(ms * 1e3 / len(sets), 3), "flops_per_launch": flops / len(sets)}
     wbytes = sum(N * K * (0.53125 if args.quant == "int4" else 1.0) for N, K, _ in sets)
     cfg = {"workload": f"C4 prefill {args.quant} 4096->14336 and 14336->4096, M={M}", "M": M,
@@ -741,7 +746,8 @@ def bench_head(args, dev):
     ms = _time_steps(_graph_or_eager(step, not args.no_graph), args.steps, args.warmup)
     nbytes = N * K + N * 2 + M * K * 2 + M * N * 2
     entry = "imq_linear_w8_tiled" if layout == "line-tiled" else "imq_linear_w8"
-    roof = _hbm_roofline(f"{'w8_line_kernel' if M <= 4 else 'w8_skinny_kernel'} ({entry}, M={M})", nbytes,
+    kern = "w8_line_kernel" if M <= 4 else "w8_skinny_kernel" if M <= 8 else "gemm_wk_kernel<8>"
+    roof = _hbm_roofline(f"{kern} ({entry}, M={M})", nbytes,
                          ms * 1e3 / len(heads), _traffic(f"head_m{M}"))
     cfg = {"workload": f"int8 lm_head 3584 -> 152064 (Qwen2.5-7B), M={M}, {len(heads)} distinct copies per step",
            "M": M, "launches_per_step": len(heads), "packed_layout": layout,

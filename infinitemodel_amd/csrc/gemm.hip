@@ -1,4 +1,6 @@
-// Prefill-regime (M > 16) fused dequant GEMM for gfx950.
+// Prefill-regime (M > 16) fused dequant GEMM for gfx950, and the dispatch of those rows: the short-batch GEMM
+// up to 64 rows (gemm_wk.hip), above that the register-B GEMM where its plan is the faster (gemm_rbm.hip, and
+// gemm_rb.hip for other dtype pairs above 512 rows), this kernel for the rest.
 //
 // y[M, N] = x[M, K] . dequant(W[N, K])^T with bf16 activations, packed int4 / int2 (group-wise
 // asymmetric) or int8 (per-row symmetric) weights, fp32 accumulation and bf16 output: the

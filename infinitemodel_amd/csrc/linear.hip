@@ -1,6 +1,7 @@
 // C-ABI entry points of the fused dequant linear family (imq_linear_w4 / _w2 / _w8) and the
-// ABI metadata calls. Dispatch: decode rows (M <= 16) go to the MFMA skinny GEMV, prefill rows
-// to the LDS-dequant MFMA GEMM; shapes or alignments a fast kernel rejects fall back to the
+// ABI metadata calls. Dispatch: decode rows (M <= 16) go to the MFMA decode kernels (gemv.hip; int8 from 5
+// rows and int4 / int2 rows of no whole line-step to the short-batch forms, gemm_wk.hip), prefill rows to the
+// GEMMs (gemm.hip); shapes or alignments a fast kernel rejects fall back to the
 // generic dequantize-then-matmul kernel (never wrong, just slower).
 //
 // imq_linear_w4_noalloc is imq_linear_w4 with its workspace taken from a static per-device

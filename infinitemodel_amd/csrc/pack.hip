@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256) void pack_g_kernel(const void* __restrict__ W,
 // WPR waves per row (1 or 4), 8 columns per lane and pass: the row's |w| max, then the codes. The
 // first NV passes keep the row in registers, so rows up to 512 NV WPR columns are read once (longer
 // ones re-read their tail); divisions as in pack_g_kernel, one shared reciprocal per row. 4096 -> 14336 bf16:
-// 39 us, 4.5 TB/s (one wave per row with 2-byte loads and a division per element: 118 us).
+// 39 us, 4.5 TB/s (one wave per row with 2-byte loads and a division per element: 114 us).
 template <int DT, int WPR, int NV>
 __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W, int64_t sw, int64_t N,
                                                       int64_t K, int8_t* __restrict__ q, int64_t sq,
