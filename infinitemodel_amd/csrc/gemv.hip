@@ -1142,19 +1142,25 @@ __global__ __launch_bounds__(64 * NW) void w4_wsplit_kernel(SkinnyArgs a) {
 // ---------------------------------------------------------------------------------------------
 // int2 decode kernel (M <= 16). A K-step is one 64-code group: 16 bytes of each packed row.
 // Lane (row nl, quarter jl) works on dword jl = codes [16*jl, 16*jl+16) of each step, which
-// feeds two v_mfma_f32_16x16x32_bf16: MFMA h takes codes {8h..8h+7} of each
+// feeds two v_mfma_f32_16x16x32_bf16: MFMA h takes codes {4h..4h+3} and {4h+8..4h+11} of each
 // lane, so every MFMA's 32 K positions lie inside one group and the group's scale/zero apply to
-// its result exactly (y += s*acc - s*z*sum(x)). The codes arrive as 16-byte loads of four
+// its result exactly (y += s*acc - s*(128+z)*sum(x)). The codes arrive as 16-byte loads of four
 // whole steps (a 64-byte line per row) redistributed by a cross-lane 4x4 transpose. Activations
-// are staged in LDS in the matching order (permute_c8); K is staged in chunks when M * K_pad
+// are staged in LDS in the matching order (permute_x16); K is staged in chunks when M * K_pad
 // does not fit.
 // ---------------------------------------------------------------------------------------------
 constexpr int kStep2 = 64;
 
-// 8 elements of a 16-byte block in the order of unpack_crumb8_bf16: [0,2,1,3,4,6,5,7].
-IMQ_DEV u32x4_t permute_c8(const u32x4_t& v) {
-  return u32x4_t{perm_b32(v[1], v[0], 0x05040100u), perm_b32(v[1], v[0], 0x07060302u),
-                 perm_b32(v[3], v[2], 0x05040100u), perm_b32(v[3], v[2], 0x07060302u)};
+// Two 16-byte blocks lo (elements 0..7), hi (8..15) -> [0,8,1,9,2,10,3,11 | 4,12,5,13,6,14,7,15].
+IMQ_DEV void permute_x16(const u32x4_t& lo, const u32x4_t& hi, u32x4_t& o0, u32x4_t& o1) {
+  o0[0] = perm_b32(hi[0], lo[0], 0x05040100u);
+  o0[1] = perm_b32(hi[0], lo[0], 0x07060302u);
+  o0[2] = perm_b32(hi[1], lo[1], 0x05040100u);
+  o0[3] = perm_b32(hi[1], lo[1], 0x07060302u);
+  o1[0] = perm_b32(hi[2], lo[2], 0x05040100u);
+  o1[1] = perm_b32(hi[2], lo[2], 0x07060302u);
+  o1[2] = perm_b32(hi[3], lo[3], 0x05040100u);
+  o1[3] = perm_b32(hi[3], lo[3], 0x07060302u);
 }
 
 // 4x4 transpose of dwords across the four 16-lane rows: on entry register k of lane row j holds
@@ -1176,25 +1182,12 @@ IMQ_DEV void transpose4_lanerows(uint32_t (&d)[4]) {
   }
 }
 
-// 16 crumbs of one dword -> the 8 codes of MFMA half h as exact bf16, in the order
-// [c(8h), c(8h+2), c(8h+1), c(8h+3), c(8h+4), c(8h+6), c(8h+5), c(8h+7)]. A crumb alone in a nibble, read as
-// fp4 (e2m1), is code / 2, so one conversion at scale 2 gives two codes: 11 VALU
-// per 16 codes where shifting each crumb pair under the exponent of 128 took 15, and no bias to subtract. us, before -> now:
-// 8192 -> 28672 M = 1 / 2 / 8 / 16 19.7 / 21.2 / 28.7 / 32.5 -> 18.5 / 20.1 / 28.1 / 31.7; 28672 -> 8192 M = 1 / 8 23.6 / 29.6 -> 22.2 / 28.7.
-IMQ_DEV bf16x8_t unpack_crumb8_bf16(uint32_t w, int h) {
-  const uint32_t even = w & 0x33333333u, odd = (w >> 2) & 0x33333333u;
+// 16 crumbs of one dword -> the 8 bf16 (128 + code) of MFMA half h, in the order
+// [c(4h), c(4h+8), c(4h+1), c(4h+9), c(4h+2), c(4h+10), c(4h+3), c(4h+11)].
+IMQ_DEV bf16x8_t unpack_crumb8_bf16(uint32_t w, int h, uint32_t magic) {
   u32x4_t r;
-  if (h == 0) {
-    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(even, 2.f, 0));
-    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(odd, 2.f, 0));
-    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(even, 2.f, 1));
-    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(odd, 2.f, 1));
-  } else {
-    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(even, 2.f, 2));
-    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(odd, 2.f, 2));
-    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(even, 2.f, 3));
-    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(odd, 2.f, 3));
-  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) r[k] = ((w >> (2 * (4 * h + k))) & 0x00030003u) | magic;
   return __builtin_bit_cast(bf16x8_t, r);
 }
 
@@ -1242,14 +1235,17 @@ __global__ __launch_bounds__(64 * MAXW) void w2_skinny_kernel(SkinnyArgs a) {
       float sum = bf16x8_sum(lo) + bf16x8_sum(hi);
       sum = quad_sum4(sum);
       if (valid) {
-        *(u32x4_t*)(xl + m * xls + 16 * pr) = permute_c8(lo);
-        *(u32x4_t*)(xl + m * xls + 16 * pr + 8) = permute_c8(hi);
+        u32x4_t o0, o1;
+        permute_x16(lo, hi, o0, o1);
+        *(u32x4_t*)(xl + m * xls + 16 * pr) = o0;
+        *(u32x4_t*)(xl + m * xls + 16 * pr + 8) = o1;
         if ((pr & 3) == 0) xs[(pr >> 2) * 16 + m] = sum;
       }
     }
     lds_barrier();
   };
 
+  const uint32_t magic = magic_bf16_128x2();
   const uint16_t* xlane = xl + (nl < a.M ? nl : a.M - 1) * xls + 16 * jl;
   const float* xslane = xs + 4 * jl;
   int buf = 0;
@@ -1332,13 +1328,13 @@ __global__ __launch_bounds__(64 * MAXW) void w2_skinny_kernel(SkinnyArgs a) {
           const bf16x8_t b1 = *(const bf16x8_t*)(xlane + lb * kStep2 + 8);
           const float sca = va ? raw_to_bf16_f32<SDT>(s_raw(i)) : 0.f;
           const float scb = vb ? raw_to_bf16_f32<SDT>(s_raw(i + 1)) : 0.f;
-          const float cza = -raw_to_bf16_f32<ZDT>(z_raw(i)) * sca;
-          const float czb = -raw_to_bf16_f32<ZDT>(z_raw(i + 1)) * scb;
+          const float cza = -(128.f + raw_to_bf16_f32<ZDT>(z_raw(i))) * sca;
+          const float czb = -(128.f + raw_to_bf16_f32<ZDT>(z_raw(i + 1))) * scb;
           f32x4_t acca = {0.f, 0.f, 0.f, 0.f}, accb = {0.f, 0.f, 0.f, 0.f};
-          acca = mfma16x16x32(a0, unpack_crumb8_bf16(wv[i], 0), acca);
-          accb = mfma16x16x32(b0, unpack_crumb8_bf16(wv[i + 1], 0), accb);
-          acca = mfma16x16x32(a1, unpack_crumb8_bf16(wv[i], 1), acca);
-          accb = mfma16x16x32(b1, unpack_crumb8_bf16(wv[i + 1], 1), accb);
+          acca = mfma16x16x32(a0, unpack_crumb8_bf16(wv[i], 0, magic), acca);
+          accb = mfma16x16x32(b0, unpack_crumb8_bf16(wv[i + 1], 0, magic), accb);
+          acca = mfma16x16x32(a1, unpack_crumb8_bf16(wv[i], 1, magic), acca);
+          accb = mfma16x16x32(b1, unpack_crumb8_bf16(wv[i + 1], 1, magic), accb);
 #pragma unroll
           for (int q = 0; q < RC; ++q) {
             yacc[q] = fmaf(cza, xsa[q], yacc[q]);
@@ -1376,15 +1372,15 @@ __global__ __launch_bounds__(64 * MAXW) void w2_skinny_kernel(SkinnyArgs a) {
 //     gets group ar of row c (gA) and group 4 + ar of row c ^ 8 (gB), one group per dword set;
 //   * a 4x4 cross-lane transpose (transpose4_lanerows) turns that into dword ar of each of the
 //     four groups, so each MFMA pair's 64 K positions lie inside one group and the group's scale
-//     and zero apply to its accumulator exactly: y += s*acc - s*z*sum(x);
-//   * activations of the wave's K range are staged in the wave's LDS (permute_c8 order) with
+//     and zero apply to its accumulator exactly: y += s*acc - s*(128 + z)*sum(x);
+//   * activations of the wave's K range are staged in the wave's LDS (permute_x16 order) with
 //     per-group row sums; scale / zero words of the 16 rows likewise.
 // Rows c ^ 8 of gB are folded back with a row swap, partials reduce across waves in LDS.
 // ---------------------------------------------------------------------------------------------
 constexpr int kLine2 = 512;   // codes per int2 line-step (128 bytes of a row, 8 groups of 64)
 
 // Scale / zero of a wave's 16 rows over NGW groups, staged in LDS as float pairs
-// (s, -z * s) with the bf16 rounding of s and z applied once per (row, group) instead of
+// (s, -(128 + z) * s) with the bf16 rounding of s and z applied once per (row, group) instead of
 // in every lane that uses them; groups past K_pad are staged as (0, 0). Row stride 2 * NGW + 2
 // floats spreads the 16 rows over the LDS banks.
 IMQ_HOST_DEV constexpr int sz2_row(int ngw) { return 2 * ngw + 2; }
@@ -1436,7 +1432,7 @@ struct SzPairs {
           sc = g < gvalid ? sc : 0.f;
           f32x2_t v;
           v[0] = sc;
-          v[1] = -zr * sc;
+          v[1] = -(128.f + zr) * sc;
           *(f32x2_t*)(szf + r * sz2_row(NGW) + 2 * g) = v;
         }
       }
@@ -1469,7 +1465,7 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
   const int xrow = S2 * kLine2 + 8;
   const int wbytes = line2_wave_lds(M, S2);
   unsigned char* wl = smem + (size_t)wave * wbytes;
-  uint16_t* xw = (uint16_t*)wl;                       // [M][xrow], permute_c8 order
+  uint16_t* xw = (uint16_t*)wl;                       // [M][xrow], permute_x16 order
   float* xs = (float*)(wl + M * xrow * 2);           // [S2 * 8 groups][16 rows]
   float* szf = xs + NGW * 16;                         // [16 rows][sz2_row(NGW)]: (s, cz) pairs
   float* red = (float*)(smem + (size_t)W * wbytes);
@@ -1511,7 +1507,7 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
     wb[2 * i] = __builtin_nontemporal_load((const u32x4_t*)(q0 + lst * l));
     wb[2 * i + 1] = __builtin_nontemporal_load((const u32x4_t*)(q1 + lst * l));
   }
-  // 4) stage x (permute_c8) with per-group sums, and scale / zero words
+  // 4) stage x (permute_x16 per pair) with per-group sums, and scale / zero words
 #pragma unroll
   for (int u = 0; u < XU; ++u) {
     const int idx = lane + 64 * u;
@@ -1521,8 +1517,10 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
     // the 4 pairs of one group are 4 consecutive idx (XP is a multiple of 4)
     sum = quad_sum4(sum);
     if (ok) {
-      *(u32x4_t*)(xw + m * xrow + 16 * p) = permute_c8(xlo[u]);
-      *(u32x4_t*)(xw + m * xrow + 16 * p + 8) = permute_c8(xhi[u]);
+      u32x4_t o0, o1;
+      permute_x16(xlo[u], xhi[u], o0, o1);
+      *(u32x4_t*)(xw + m * xrow + 16 * p) = o0;
+      *(u32x4_t*)(xw + m * xrow + 16 * p + 8) = o1;
       if ((p & 3) == 0) xs[(p >> 2) * 16 + m] = sum;
     }
   }
@@ -1530,6 +1528,7 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
   // LDS is written and read by this wave only; its LDS operations execute in order
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
+  const uint32_t magic = magic_bf16_128x2();
   const uint16_t* xa = xw + (c < M ? c : M - 1) * xrow + 16 * ar;
   const float* sz_c = szf + c * sz2_row(NGW);
   const float* sz_x = szf + (c ^ 8) * sz2_row(NGW);
@@ -1564,14 +1563,14 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
       const bf16x8_t a1 = *(const bf16x8_t*)(xa + 64 * gA + 8);
       const bf16x8_t b0 = *(const bf16x8_t*)(xa + 64 * gB);
       const bf16x8_t b1 = *(const bf16x8_t*)(xa + 64 * gB + 8);
-      const f32x2_t pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -z * s)
+      const f32x2_t pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -(128 + z) * s)
       const f32x2_t pB = *(const f32x2_t*)(sz_x + 2 * gB);
       const float sA = pA[0], czA = pA[1], sB = pB[0], czB = pB[1];
       f32x4_t accA = {0.f, 0.f, 0.f, 0.f}, accB = {0.f, 0.f, 0.f, 0.f};
-      accA = mfma16x16x32(a0, unpack_crumb8_bf16(dA[k], 0), accA);
-      accB = mfma16x16x32(b0, unpack_crumb8_bf16(dB[k], 0), accB);
-      accA = mfma16x16x32(a1, unpack_crumb8_bf16(dA[k], 1), accA);
-      accB = mfma16x16x32(b1, unpack_crumb8_bf16(dB[k], 1), accB);
+      accA = mfma16x16x32(a0, unpack_crumb8_bf16(dA[k], 0, magic), accA);
+      accB = mfma16x16x32(b0, unpack_crumb8_bf16(dB[k], 0, magic), accB);
+      accA = mfma16x16x32(a1, unpack_crumb8_bf16(dA[k], 1, magic), accA);
+      accB = mfma16x16x32(b1, unpack_crumb8_bf16(dB[k], 1, magic), accB);
 #pragma unroll
       for (int r = 0; r < RC; ++r) {
         y0[r] = fmaf(czA, xsA[r], y0[r]);
@@ -1600,7 +1599,7 @@ __global__ __launch_bounds__(64 * MAXW) void w2_line_kernel(SkinnyArgs a) {
 // ---------------------------------------------------------------------------------------------
 // int2 decode kernel for 4 < M <= 16 (G = 64): the int4 K-split structure with the int2 line-step
 // of the int2 line kernel. A workgroup owns NW row tiles and one split of S2 line-steps (S2 * 512
-// codes); the activation chunk x[0:M, split] is staged once in LDS (permute_c8 order, per-group
+// codes); the activation chunk x[0:M, split] is staged once in LDS (permute_x16 order, per-group
 // row sums) and shared by the waves; wave w streams rows [16 w, 16 w + 16) of the tile over the
 // split with two full-line loads per line-step and the cross-lane group transpose; the fp32
 // partials go to part[split][m][n] and splitk_rows_reduce_kernel sums the splits in order.
@@ -1682,7 +1681,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(IMQ_W2K
     wb[2 * i] = __builtin_nontemporal_load((const u32x4_t*)(q0 + lst * l));
     wb[2 * i + 1] = __builtin_nontemporal_load((const u32x4_t*)(q1 + lst * l));
   }
-  // 4) stage x (permute_c8) with per-group sums, and this wave's scale / zero words
+  // 4) stage x (permute_x16 per pair) with per-group sums, and this wave's scale / zero words
 #pragma unroll
   for (int u = 0; u < XU; ++u) {
     const int idx = threadIdx.x + NT * u;
@@ -1692,14 +1691,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(IMQ_W2K
     // the 4 pairs of one group are 4 consecutive idx (XP and NT are multiples of 4)
     sum = quad_sum4(sum);
     if (ok) {
-      *(u32x4_t*)(xw + m * xrow + 16 * p) = permute_c8(xlo[u]);
-      *(u32x4_t*)(xw + m * xrow + 16 * p + 8) = permute_c8(xhi[u]);
+      u32x4_t o0, o1;
+      permute_x16(xlo[u], xhi[u], o0, o1);
+      *(u32x4_t*)(xw + m * xrow + 16 * p) = o0;
+      *(u32x4_t*)(xw + m * xrow + 16 * p + 8) = o1;
       if ((p & 3) == 0) xs[(p >> 2) * 16 + m] = sum;
     }
   }
   szp.store(lane, szf, (KL - ls0) * GPL);
   lds_barrier();   // x and its sums are shared by the waves; weights stay in flight
 
+  const uint32_t magic = magic_bf16_128x2();
   const uint16_t* xa = xw + (c < M ? c : M - 1) * xrow + 16 * ar;
   const float* sz_c = szf + c * sz2_row(NGW);
   const float* sz_x = szf + (c ^ 8) * sz2_row(NGW);
@@ -1723,7 +1725,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(IMQ_W2K
     o.a1 = *(const bf16x8_t*)(xa + 64 * gA + 8);
     o.b0 = *(const bf16x8_t*)(xa + 64 * gB);
     o.b1 = *(const bf16x8_t*)(xa + 64 * gB + 8);
-    o.pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -z * s)
+    o.pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -(128 + z) * s)
     o.pB = *(const f32x2_t*)(sz_x + 2 * gB);
   };
   Ops op[2];
@@ -1745,10 +1747,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(IMQ_W2K
       transpose4_lanerows(dB);    // dB[k]: dword ar of group 4 + k of row c ^ 8
     }
     const f32x4_t z4 = {0.f, 0.f, 0.f, 0.f};
-    acA[cur] = mfma16x16x32(op[cur].a0, unpack_crumb8_bf16(dA[k], 0), z4);
-    acB[cur] = mfma16x16x32(op[cur].b0, unpack_crumb8_bf16(dB[k], 0), z4);
-    acA[cur] = mfma16x16x32(op[cur].a1, unpack_crumb8_bf16(dA[k], 1), acA[cur]);
-    acB[cur] = mfma16x16x32(op[cur].b1, unpack_crumb8_bf16(dB[k], 1), acB[cur]);
+    acA[cur] = mfma16x16x32(op[cur].a0, unpack_crumb8_bf16(dA[k], 0, magic), z4);
+    acB[cur] = mfma16x16x32(op[cur].b0, unpack_crumb8_bf16(dB[k], 0, magic), z4);
+    acA[cur] = mfma16x16x32(op[cur].a1, unpack_crumb8_bf16(dA[k], 1, magic), acA[cur]);
+    acB[cur] = mfma16x16x32(op[cur].b1, unpack_crumb8_bf16(dB[k], 1, magic), acB[cur]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       y0[r] = fmaf(op[cur].pA[1], op[cur].xsA[r], y0[r]);
@@ -1794,14 +1796,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(IMQ_W2K
       const bf16x8_t a1 = *(const bf16x8_t*)(xa + 64 * gA + 8);
       const bf16x8_t b0 = *(const bf16x8_t*)(xa + 64 * gB);
       const bf16x8_t b1 = *(const bf16x8_t*)(xa + 64 * gB + 8);
-      const f32x2_t pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -z * s)
+      const f32x2_t pA = *(const f32x2_t*)(sz_c + 2 * gA);   // (s, -(128 + z) * s)
       const f32x2_t pB = *(const f32x2_t*)(sz_x + 2 * gB);
       const float sA = pA[0], czA = pA[1], sB = pB[0], czB = pB[1];
       f32x4_t accA = {0.f, 0.f, 0.f, 0.f}, accB = {0.f, 0.f, 0.f, 0.f};
-      accA = mfma16x16x32(a0, unpack_crumb8_bf16(dA[k], 0), accA);
-      accB = mfma16x16x32(b0, unpack_crumb8_bf16(dB[k], 0), accB);
-      accA = mfma16x16x32(a1, unpack_crumb8_bf16(dA[k], 1), accA);
-      accB = mfma16x16x32(b1, unpack_crumb8_bf16(dB[k], 1), accB);
+      accA = mfma16x16x32(a0, unpack_crumb8_bf16(dA[k], 0, magic), accA);
+      accB = mfma16x16x32(b0, unpack_crumb8_bf16(dB[k], 0, magic), accB);
+      accA = mfma16x16x32(a1, unpack_crumb8_bf16(dA[k], 1, magic), accA);
+      accB = mfma16x16x32(b1, unpack_crumb8_bf16(dB[k], 1, magic), accB);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         y0[r] = fmaf(czA, xsA[r], y0[r]);
