@@ -99,7 +99,8 @@ int imq_pack_w8(const void* W, int64_t w_row_stride, int w_dtype, int64_t N, int
  * workspace (optional, may be NULL): device memory of at least imq_linear_workspace_bytes(M, N,
  * K_pad) bytes, 16-byte aligned, contents need not be initialised. With it, prefill shapes whose
  * tiles do not fill the CUs split K across workgroups; a second launch sums the fp32 partials in
- * split order (deterministic). Calls that share a workspace must be ordered on one stream.
+ * split order (deterministic). Calls that share a workspace must be ordered on one stream, and be
+ * made one at a time: another thread's launches between the two of a call would overwrite its partials.
  * Without it (or when too small) K is not split. The bound covers the decode K-split kernels too
  * (4 < M <= 16; on line-tiled int2 weights also M 3..4 and the M <= 2 shapes too long in K for
  * the int2 line kernel). */

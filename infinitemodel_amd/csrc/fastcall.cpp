@@ -28,10 +28,11 @@ struct Api {
   decltype(&imq_moe_experts_w4_ex) moe = nullptr;
   decltype(&imq_moe_workspace_bytes) moe_ws = nullptr;
 } api;
-PyObject* scratch_fn = nullptr;   // ops._scratch_ptr(device index, bytes) -> (pointer, bytes)
+PyObject* scratch_fn = nullptr;   // ops._scratch_ptr(device index, bytes) -> (pointer, bytes, lock)
 
 struct Scratch {
   int64_t ptr = 0, bytes = 0;
+  PyObject* lock = nullptr;       // owned; one per (device, stream), ops.py's users hold the same
 };
 // The workspaces ops.py holds for the life of the process, one per (device, stream); read and written
 // with the GIL held.
@@ -46,14 +47,44 @@ bool scratch(int dev, void* stream, int64_t need, Scratch* out) {
     PyObject* r = PyObject_CallFunction(scratch_fn, "iL", dev, (long long)need);
     if (r == nullptr) return false;
     long long p = 0, b = 0;
-    const bool ok = PyArg_ParseTuple(r, "LL", &p, &b) != 0;
+    PyObject* lock = nullptr;
+    const bool ok = PyArg_ParseTuple(r, "LLO", &p, &b, &lock) != 0;
+    if (ok) {
+      if (s.lock == nullptr) s.lock = Py_NewRef(lock);   // the key's lock never changes
+      s.ptr = p;
+      s.bytes = b;
+    }
     Py_DECREF(r);
     if (!ok) return false;
-    s = Scratch{p, b};
   }
   *out = s;
   return true;
 }
+
+// Holds a workspace's lock while a call's launches go out: the GIL is released around them, and the kernel
+// that writes the partials and the one that sums them must not be parted by another thread's call on the
+// same stream. Taken and released with the GIL held (a waiting acquire lets go of it).
+class Held {
+ public:
+  // false: a Python error is set
+  bool take(const Scratch& s) {
+    if (s.lock == nullptr) return true;
+    PyObject* r = PyObject_CallMethod(s.lock, "acquire", nullptr);
+    if (r == nullptr) return false;
+    Py_DECREF(r);
+    lock_ = s.lock;
+    return true;
+  }
+  ~Held() {
+    if (lock_ == nullptr) return;
+    PyObject* r = PyObject_CallMethod(lock_, "release", nullptr);
+    if (r == nullptr) PyErr_Clear();
+    else Py_DECREF(r);
+  }
+
+ private:
+  PyObject* lock_ = nullptr;
+};
 
 int dtype_code(at::ScalarType t) {
   switch (t) {
@@ -164,6 +195,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t sqn = q->stride(0), s0 = s->stride(0);
     const int64_t s1 = bits == 8 ? 0 : s->stride(1), z0 = z ? z->stride(0) : 0, z1 = z ? z->stride(1) : 0;
     int rc;
+    Held held;
+    if (!held.take(ws)) return nullptr;
     Py_BEGIN_ALLOW_THREADS;
     if (bits == 8)
       rc = (tiled ? api.w8t : api.w8)(xp, sxm, M, K, qp, sqn, sp, s0, sdt, N, yp, N, (void*)ws.ptr, ws.bytes, stream);
@@ -246,6 +279,8 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const int64_t dq0 = dq.stride(0), dq1 = dq.stride(1), ds0 = ds.stride(0), ds1 = ds.stride(1);
     const int64_t b0 = b[0] ? b[0]->stride(0) : 0, b1 = b[1] ? b[1]->stride(0) : 0;
     int rc;
+    Held held;
+    if (!held.take(ws)) return nullptr;
     Py_BEGIN_ALLOW_THREADS;
     rc = api.moe(p[0], sx, T, H, k, p[1], idt, p[2], E, p[3], gq0, gq1, gK, p[4], p[5], gs0, gs1, I, p[6], dq0, dq1, dK, p[7],
                  p[8], ds0, ds1, sdt, group, p[9], b0, p[10], b1, bdt, act, alpha, limit, p[11], H, (void*)ws.ptr, ws.bytes,

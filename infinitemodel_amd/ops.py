@@ -48,41 +48,62 @@ def _rows2d(x: torch.Tensor) -> torch.Tensor:
 
 
 # Workspaces (split-K / K-split partials of the fused linears, MoE intermediates), one per
-# (device, stream): calls sharing one are ordered by that stream, and their contents need no
-# initialization. A workspace is never freed once handed out, because a HIP graph captured with it
-# keeps its address: when a call needs more, the old buffer is retired (kept alive for the life of
-# the process) and one at least twice its size takes its place, so at most log2(largest need)
-# buffers are ever retired per stream.
-_WS: dict = {}
+# (device, stream), their contents need no initialization. A call that uses one holds its lock from
+# its first launch to its last: the kernel that writes the partials and the launch that sums them are
+# two, and both host paths release the GIL between them, so without the lock two threads on one stream
+# could enqueue A's kernel, B's kernel, A's sum. A workspace is never freed once handed out, because a
+# HIP graph captured with it (and the native path's cached pointer) keeps its address: when a call needs
+# more, the old buffer is retired (kept alive for the life of the process) and one at least twice its
+# size takes its place, so at most log2(largest need) buffers are ever retired per stream.
+_WS: dict = {}                  # (device index, stream) -> (buffer, lock)
 _WS_RETIRED: list = []
+_WS_LOCK = threading.RLock()    # of the two containers; re-entrant, as an allocation may run finalizers
 
 
 def _scratch(dev: torch.device, need: int):
-    """The (device, current stream) workspace of at least ``need`` bytes, or None if need <= 0."""
-    if need <= 0:
-        return None
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    """The (device, current stream) workspace of at least ``need`` bytes and the lock its users hold."""
+    key = (dev.index, _stream(dev))
     ws = _WS.get(key)
-    if ws is None or ws.numel() < need:
-        size = need
-        if ws is not None:
-            _WS_RETIRED.append(ws)
-            size = max(need, 2 * ws.numel())
-        ws = torch.empty(size, dtype=torch.uint8, device=dev)
-        _WS[key] = ws
+    if ws is None or ws[0].numel() < need:
+        with _WS_LOCK:
+            ws = _WS.get(key)
+            if ws is None or ws[0].numel() < need:
+                size = need if ws is None else max(need, 2 * ws[0].numel())
+                buf = torch.empty(size, dtype=torch.uint8, device=dev)
+                ws = _WS.get(key)                # again: a finalizer may have come here meanwhile
+                if ws is not None:
+                    _WS_RETIRED.append(ws[0])
+                ws = _WS[key] = (buf, threading.RLock() if ws is None else ws[1])
     return ws
 
 
-def _workspace(dev: torch.device, M: int, N: int, K: int):
-    ws = _scratch(dev, int(_lib.lib().imq_linear_workspace_bytes(M, N, K)))
-    if ws is None:
-        return 0, 0
-    return ws.data_ptr(), ws.numel()
+class _Held:
+    """``with _Held(dev, need) as (pointer, bytes)``: the workspace for one call, locked (none for need <= 0)."""
+
+    __slots__ = ("ws",)
+
+    def __init__(self, dev: torch.device, need: int):
+        self.ws = _scratch(dev, need) if need > 0 else None
+
+    def __enter__(self):
+        if self.ws is None:
+            return 0, 0
+        self.ws[1].acquire()
+        return self.ws[0].data_ptr(), self.ws[0].numel()
+
+    def __exit__(self, *exc):
+        if self.ws is not None:
+            self.ws[1].release()
+
+
+def _workspace(dev: torch.device, M: int, N: int, K: int) -> _Held:
+    return _Held(dev, int(_lib.lib().imq_linear_workspace_bytes(M, N, K)))
 
 
 def _scratch_ptr(index: int, need: int):
-    w = _scratch(torch.device("cuda", index), need)
-    return w.data_ptr(), w.numel()
+    """The native path's view of a workspace: (pointer, bytes, lock)."""
+    buf, lock = _scratch(torch.device("cuda", index), need)
+    return buf.data_ptr(), buf.numel(), lock
 
 
 # The native host path (csrc/fastcall.cpp): ``_fast_linear(kind, x, q, sz, group, nd)`` and ``_fast_moe(...)``
@@ -246,16 +267,15 @@ def _linear_g(fn: str, codes_per_byte: int, x, qweight, group_size: int, sz, out
         if fn == "imq_linear_w4":
             # this call's own need (0 for the decode kernels that keep their partials in the
             # workgroup), not the shape-only bound over all formats
-            need = int(_lib.lib().imq_linear_w4_workspace_bytes(
+            held = _Held(dev, int(_lib.lib().imq_linear_w4_workspace_bytes(
                 M, Kpad, N, group_size, qweight.stride(0), x.stride(0), scale.stride(0), scale.stride(1),
-                dtype_code(scale.dtype), zero.stride(0), zero.stride(1), dtype_code(zero.dtype)))
-            w = _scratch(dev, need)
-            ws, wsb = (0, 0) if w is None else (w.data_ptr(), w.numel())
+                dtype_code(scale.dtype), zero.stride(0), zero.stride(1), dtype_code(zero.dtype))))
         else:
-            ws, wsb = _workspace(dev, M, N, Kpad)
-        call(fn, _ptr(x), x.stride(0), M, Kpad, _ptr(qweight), qweight.stride(0), _ptr(scale), scale.stride(0),
-             scale.stride(1), dtype_code(scale.dtype), _ptr(zero), zero.stride(0), zero.stride(1),
-             dtype_code(zero.dtype), N, group_size, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
+            held = _workspace(dev, M, N, Kpad)
+        with held as (ws, wsb):
+            call(fn, _ptr(x), x.stride(0), M, Kpad, _ptr(qweight), qweight.stride(0), _ptr(scale), scale.stride(0),
+                 scale.stride(1), dtype_code(scale.dtype), _ptr(zero), zero.stride(0), zero.stride(1),
+                 dtype_code(zero.dtype), N, group_size, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
     return y
 
 
@@ -352,9 +372,9 @@ def linear_w8_tiled(x, qweight_tiled, scale, out=None):
         raise ValueError(f"x has {K} columns, qweight {qweight_tiled.shape[1]}")
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     with torch.cuda.device(dev):
-        ws, wsb = _workspace(dev, M, N, K)
-        call("imq_linear_w8_tiled", _ptr(x), x.stride(0), M, K, _ptr(qweight_tiled), qweight_tiled.stride(0),
-             _ptr(scale), scale.stride(0), dtype_code(scale.dtype), N, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
+        with _workspace(dev, M, N, K) as (ws, wsb):
+            call("imq_linear_w8_tiled", _ptr(x), x.stride(0), M, K, _ptr(qweight_tiled), qweight_tiled.stride(0),
+                 _ptr(scale), scale.stride(0), dtype_code(scale.dtype), N, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
     return y
 
 
@@ -378,9 +398,9 @@ def linear_w8(x, qweight, scale, out=None):
         raise ValueError(f"x has {K} columns, qweight {qweight.shape[1]}")
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     with torch.cuda.device(dev):
-        ws, wsb = _workspace(dev, M, N, K)
-        call("imq_linear_w8", _ptr(x), x.stride(0), M, K, _ptr(qweight), qweight.stride(0), _ptr(scale),
-             scale.stride(0), dtype_code(scale.dtype), N, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
+        with _workspace(dev, M, N, K) as (ws, wsb):
+            call("imq_linear_w8", _ptr(x), x.stride(0), M, K, _ptr(qweight), qweight.stride(0), _ptr(scale),
+                 scale.stride(0), dtype_code(scale.dtype), N, _ptr(y), y.stride(0), ws, wsb, _stream(dev))
     return y
 
 
@@ -506,10 +526,11 @@ def moe_experts_w4(hidden, topk_idx, topk_w, gu, dn, group_size: int, workspace=
         _check_expert_ids(idx, E)
     w = topk_w.to(torch.bfloat16).contiguous()
     need = moe_workspace_bytes(T, k, E, H, I, group_size)
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = _scratch(dev, max(need, 1))
+    own = workspace is not None and workspace.numel() * workspace.element_size() >= need
     out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with torch.cuda.device(dev), _Held(dev, 0 if own else max(need, 1)) as (ws, wsb):
+        if own:
+            ws, wsb = _ptr(workspace), workspace.numel() * workspace.element_size()
         call("imq_moe_experts_w4_ex", _ptr(x), x.stride(0), T, H, k, _ptr(idx),
              _lib.IMQ_DT_I64 if idx.dtype == torch.int64 else _lib.IMQ_DT_I32, _ptr(w), E,
              _ptr(gq), gq.stride(0), gq.stride(1), gK, _ptr(gs), _ptr(gz), gs.stride(0), gs.stride(1), I,
@@ -518,6 +539,5 @@ def moe_experts_w4(hidden, topk_idx, topk_w, gu, dn, group_size: int, workspace=
              _ptr(gb) if gb is not None else None, gb.stride(0) if gb is not None else 0,
              _ptr(db) if db is not None else None, db.stride(0) if db is not None else 0,
              dtype_code(bdt) if bdt is not None else 0, _ACT[act], float(alpha), float(limit),
-             _ptr(out), out.stride(0), _ptr(workspace), workspace.numel() * workspace.element_size(),
-             _stream(dev))
+             _ptr(out), out.stride(0), ws, wsb, _stream(dev))
     return out

@@ -115,6 +115,41 @@ def test_streams_threads_and_capture(dev):
         assert torch.equal(y, want[i])
 
 
+@pytest.mark.parametrize("native", [True, False])
+def test_threads_that_share_a_stream(dev, monkeypatch, native):
+    """Calls that split K into the shared workspace, from several threads on torch's default stream: another thread's
+    kernel never comes between a call's partials and their sum, on either host path or between the two."""
+    import torch
+    from infinitemodel_amd import _lib, ops
+    N, K, M = 4096, 14336, 8
+    assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, 0, N, sqn=K)[1] > 1          # int8 splits K
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    x = [torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16) for _ in range(4)]
+    q8 = torch.randint(-127, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
+    q4 = torch.randint(0, 256, (N, K // 2), generator=g, device=dev, dtype=torch.uint8)
+    s8 = torch.full((N, 1), 1e-3, dtype=torch.bfloat16, device=dev)
+    s4 = torch.full((N, K // 128), 1e-2, dtype=torch.bfloat16, device=dev)
+    q2, s2 = q4[:, :K // 4].contiguous(), torch.full((N, K // 64), 1e-2, dtype=torch.bfloat16, device=dev)
+    if not native:
+        monkeypatch.setattr(ops, "_fast_linear", lambda *a: None)
+    out = [torch.empty(M, N, dtype=torch.bfloat16, device=dev) for _ in x]
+    ops_ = [lambda i: ops.linear_w8(x[i], q8, s8), lambda i: ops.linear_w4(x[i], q4, 128, (s4, s4)),
+            lambda i: ops.linear_w2(x[i], q2, 64, (s2, s2)), lambda i: ops.linear_w8(x[i], q8, s8, out=out[i])]
+    want = [[f(i).clone() for f in ops_] for i in range(4)]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        for _ in range(50):
+            ys = [f(i) for f in ops_]
+            bad.extend((i, j) for j, y in enumerate(ys) if not torch.equal(y, want[i][j]))
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [th.start() for th in ts]
+    [th.join() for th in ts]
+    assert not bad, bad[:8]
+
+
 @pytest.mark.parametrize("T,act", [(1, "silu_glu"), (5, "gptoss"), (40, "silu_glu")])
 def test_experts_same_bits_as_the_python_path(dev, monkeypatch, T, act):
     import torch
