@@ -126,7 +126,7 @@ bool rows_ok(const at::Tensor& x) {   // _rows2d would pass x through
 // linear(kind, x, q, sz, group, nd): kind = bits, + 16 for line-tiled weights; sz = (scale, zero), or the
 // scale for int8; nd: x of any rank, the result of x's leading sizes (a module's forward), else x
 // [M, K] -> y [M, N].
-PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* linear_call(PyObject* const* args, Py_ssize_t n) {
   if (n != 6) Py_RETURN_NONE;
   const long kind = PyLong_AsLong(args[0]), group = PyLong_AsLong(args[4]);
   const bool nd = args[5] == Py_True;
@@ -182,38 +182,34 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
                            : api.ws(M, N, K);
   Scratch ws;
   if (!scratch(dev, stream, need, &ws)) return nullptr;
-  try {
-    at::Tensor y;
-    if (nd && x->dim() != 2) {
-      c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
-      shape.back() = N;
-      y = at::empty(shape, x->options().requires_grad(false));
-    } else {
-      y = at::empty({M, N}, x->options().requires_grad(false));
-    }
-    void *xp = x->data_ptr(), *qp = q->data_ptr(), *sp = s->data_ptr(), *zp = z ? z->data_ptr() : nullptr, *yp = y.data_ptr();
-    const int64_t sqn = q->stride(0), s0 = s->stride(0);
-    const int64_t s1 = bits == 8 ? 0 : s->stride(1), z0 = z ? z->stride(0) : 0, z1 = z ? z->stride(1) : 0;
-    int rc;
-    Held held;
-    if (!held.take(ws)) return nullptr;
-    Py_BEGIN_ALLOW_THREADS;
-    if (bits == 8)
-      rc = (tiled ? api.w8t : api.w8)(xp, sxm, M, K, qp, sqn, sp, s0, sdt, N, yp, N, (void*)ws.ptr, ws.bytes, stream);
-    else
-      rc = (bits == 4 ? (tiled ? api.w4t : api.w4) : (tiled ? api.w2t : api.w2))(
-          xp, sxm, M, K, qp, sqn, sp, s0, s1, sdt, zp, z0, z1, zdt, N, group, yp, N, (void*)ws.ptr, ws.bytes, stream);
-    Py_END_ALLOW_THREADS;
-    if (rc != IMQ_OK) Py_RETURN_NONE;   // the Python path repeats the call and raises
-    return THPVariable_Wrap(std::move(y));
-  } catch (const std::exception&) {
-    Py_RETURN_NONE;                     // an allocation that failed fails again there, with torch's own error
+  at::Tensor y;
+  if (nd && x->dim() != 2) {
+    c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
+    shape.back() = N;
+    y = at::empty(shape, x->options().requires_grad(false));
+  } else {
+    y = at::empty({M, N}, x->options().requires_grad(false));
   }
+  void *xp = x->data_ptr(), *qp = q->data_ptr(), *sp = s->data_ptr(), *zp = z ? z->data_ptr() : nullptr, *yp = y.data_ptr();
+  const int64_t sqn = q->stride(0), s0 = s->stride(0);
+  const int64_t s1 = bits == 8 ? 0 : s->stride(1), z0 = z ? z->stride(0) : 0, z1 = z ? z->stride(1) : 0;
+  int rc;
+  Held held;
+  if (!held.take(ws)) return nullptr;
+  Py_BEGIN_ALLOW_THREADS;
+  if (bits == 8)
+    rc = (tiled ? api.w8t : api.w8)(xp, sxm, M, K, qp, sqn, sp, s0, sdt, N, yp, N, (void*)ws.ptr, ws.bytes, stream);
+  else
+    rc = (bits == 4 ? (tiled ? api.w4t : api.w4) : (tiled ? api.w2t : api.w2))(
+        xp, sxm, M, K, qp, sqn, sp, s0, s1, sdt, zp, z0, z1, zdt, N, group, yp, N, (void*)ws.ptr, ws.bytes, stream);
+  Py_END_ALLOW_THREADS;
+  if (rc != IMQ_OK) Py_RETURN_NONE;   // the Python path repeats the call and raises
+  return THPVariable_Wrap(std::move(y));
 }
 
 // moe(hidden, idx, w, gu, dn, group, act, gu_bias, dn_bias, alpha, limit): moe_experts_w4 without the id
 // check and with the cached workspace; gu / dn = (qweight, scale, zero, in_features).
-PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
+PyObject* moe_call(PyObject* const* args, Py_ssize_t n) {
   if (n != 11) Py_RETURN_NONE;
   const at::Tensor* x = plain(args[0], -1);
   if (x == nullptr || !plain_context()) Py_RETURN_NONE;
@@ -268,27 +264,35 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t need = api.moe_ws(T, k, E, H, I, group);
   Scratch ws;
   if (!scratch(dev, stream, need > 1 ? need : 1, &ws)) return nullptr;
+  at::Tensor out = at::empty({T, H}, x->options().requires_grad(false));
+  void* p[] = {x->data_ptr(), idx->data_ptr(), w->data_ptr(), gq.data_ptr(), gs.data_ptr(), t[0][2]->data_ptr(),
+               dq.data_ptr(), ds.data_ptr(), t[1][2]->data_ptr(), b[0] ? b[0]->data_ptr() : nullptr,
+               b[1] ? b[1]->data_ptr() : nullptr, out.data_ptr()};
+  const int idt = idx->scalar_type() == at::kLong ? IMQ_DT_I64 : IMQ_DT_I32;
+  const float alpha = (float)PyFloat_AS_DOUBLE(args[9]), limit = (float)PyFloat_AS_DOUBLE(args[10]);
+  const int64_t sx = x->stride(0), gq0 = gq.stride(0), gq1 = gq.stride(1), gs0 = gs.stride(0), gs1 = gs.stride(1);
+  const int64_t dq0 = dq.stride(0), dq1 = dq.stride(1), ds0 = ds.stride(0), ds1 = ds.stride(1);
+  const int64_t b0 = b[0] ? b[0]->stride(0) : 0, b1 = b[1] ? b[1]->stride(0) : 0;
+  int rc;
+  Held held;
+  if (!held.take(ws)) return nullptr;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = api.moe(p[0], sx, T, H, k, p[1], idt, p[2], E, p[3], gq0, gq1, gK, p[4], p[5], gs0, gs1, I, p[6], dq0, dq1, dK, p[7],
+               p[8], ds0, ds1, sdt, group, p[9], b0, p[10], b1, bdt, act, alpha, limit, p[11], H, (void*)ws.ptr, ws.bytes,
+               stream);
+  Py_END_ALLOW_THREADS;
+  if (rc != IMQ_OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(out));
+}
+
+// The two calls at the C boundary: what torch throws anywhere in them (a storage without an address, a device
+// error, an allocation that fails) must not leave it. The Python path repeats the call and raises torch's error.
+template <PyObject* (*F)(PyObject* const*, Py_ssize_t)>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
   try {
-    at::Tensor out = at::empty({T, H}, x->options().requires_grad(false));
-    void* p[] = {x->data_ptr(), idx->data_ptr(), w->data_ptr(), gq.data_ptr(), gs.data_ptr(), t[0][2]->data_ptr(),
-                 dq.data_ptr(), ds.data_ptr(), t[1][2]->data_ptr(), b[0] ? b[0]->data_ptr() : nullptr,
-                 b[1] ? b[1]->data_ptr() : nullptr, out.data_ptr()};
-    const int idt = idx->scalar_type() == at::kLong ? IMQ_DT_I64 : IMQ_DT_I32;
-    const float alpha = (float)PyFloat_AS_DOUBLE(args[9]), limit = (float)PyFloat_AS_DOUBLE(args[10]);
-    const int64_t sx = x->stride(0), gq0 = gq.stride(0), gq1 = gq.stride(1), gs0 = gs.stride(0), gs1 = gs.stride(1);
-    const int64_t dq0 = dq.stride(0), dq1 = dq.stride(1), ds0 = ds.stride(0), ds1 = ds.stride(1);
-    const int64_t b0 = b[0] ? b[0]->stride(0) : 0, b1 = b[1] ? b[1]->stride(0) : 0;
-    int rc;
-    Held held;
-    if (!held.take(ws)) return nullptr;
-    Py_BEGIN_ALLOW_THREADS;
-    rc = api.moe(p[0], sx, T, H, k, p[1], idt, p[2], E, p[3], gq0, gq1, gK, p[4], p[5], gs0, gs1, I, p[6], dq0, dq1, dK, p[7],
-                 p[8], ds0, ds1, sdt, group, p[9], b0, p[10], b1, bdt, act, alpha, limit, p[11], H, (void*)ws.ptr, ws.bytes,
-                 stream);
-    Py_END_ALLOW_THREADS;
-    if (rc != IMQ_OK) Py_RETURN_NONE;
-    return THPVariable_Wrap(std::move(out));
+    return F(args, n);
   } catch (const std::exception&) {
+    if (PyErr_Occurred()) return nullptr;
     Py_RETURN_NONE;
   }
 }
@@ -327,8 +331,8 @@ PyObject* init(PyObject*, PyObject* args) {
 }
 
 PyMethodDef methods[] = {
-    {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, "plain fused linear, or None"},
-    {"moe", (PyCFunction)(void (*)(void))moe, METH_FASTCALL, "plain fused experts, or None"},
+    {"linear", (PyCFunction)(void (*)(void))entry<linear_call>, METH_FASTCALL, "plain fused linear, or None"},
+    {"moe", (PyCFunction)(void (*)(void))entry<moe_call>, METH_FASTCALL, "plain fused experts, or None"},
     {"init", init, METH_VARARGS, "entry-point addresses and the workspace function"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "imq_fast", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -115,6 +115,30 @@ def test_streams_threads_and_capture(dev):
         assert torch.equal(y, want[i])
 
 
+def test_what_torch_throws_stays_inside_the_call(dev):
+    """An operand whose address torch refuses (as a fake tensor's): the native calls return None instead of ending the
+    process, and the Python path raises torch's error."""
+    import torch
+    from infinitemodel_amd import ops
+    q, sz = _case(dev, 4)
+    x = torch.randn(2, 1024, device=dev).to(torch.bfloat16)
+    y = ops.linear_w4(x, q, 128, sz)
+    for bad in ("x", "q"):
+        xb, qb = x.clone(), q.clone()
+        torch._C._set_throw_on_mutable_data_ptr(xb if bad == "x" else qb)
+        assert ops._fast_linear(4, xb, qb, sz, 128, False) is None
+        assert ops._fast_linear(4, xb.reshape(1, 2, 1024) if bad == "q" else xb, qb, sz, 128, True) is None
+        with pytest.raises(RuntimeError):
+            ops.linear_w4(xb, qb, 128, sz)
+    gu, dn = (torch.zeros(2, 64, 64, dtype=torch.uint8, device=dev), *[torch.ones(2, 64, 1, dtype=torch.bfloat16, device=dev)] * 2, 128), \
+        (torch.zeros(2, 128, 64, dtype=torch.uint8, device=dev), *[torch.ones(2, 128, 1, dtype=torch.bfloat16, device=dev)] * 2, 32)
+    h = torch.zeros(1, 128, dtype=torch.bfloat16, device=dev)
+    torch._C._set_throw_on_mutable_data_ptr(h)
+    idx, w = torch.zeros(1, 1, dtype=torch.int64, device=dev), torch.ones(1, 1, dtype=torch.bfloat16, device=dev)
+    assert ops._fast_moe(h, idx, w, gu, dn, 128, 0, None, None, 1.702, 7.0) is None
+    assert torch.equal(ops.linear_w4(x, q, 128, sz), y)
+
+
 @pytest.mark.parametrize("native", [True, False])
 def test_threads_that_share_a_stream(dev, monkeypatch, native):
     """Calls that split K into the shared workspace, from several threads on torch's default stream: another thread's
