@@ -103,7 +103,7 @@ int imq_pack_w8(const void* W, int64_t w_row_stride, int w_dtype, int64_t N, int
  * made one at a time: another thread's launches between the two of a call would overwrite its partials.
  * Without it (or when too small) K is not split. The bound covers the decode K-split kernels too
  * (4 < M <= 16; on line-tiled int2 weights also M 3..4 and the M <= 2 shapes too long in K for
- * the int2 line kernel). */
+ * the int2 line kernel) and the int8 short-batch plan of M 5..16. */
 int64_t imq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K_pad);
 
 /* Workspace bytes imq_linear_w4 uses for exactly this call (the same arguments as imq_linear_w4,

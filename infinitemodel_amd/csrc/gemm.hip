@@ -641,8 +641,6 @@ int gemm_bits(const GemmArgs& a, int sdt, int zdt, void* ws, int64_t wsb, hipStr
 
 }  // namespace
 
-// Workspace bytes a split-K launch of this shape may use (0: no launch splits K): the larger of
-// the register-B GEMM's plan (int4 / int8) and the LDS-dequant GEMM's (int2, other layouts).
 // The LDS-dequant GEMM's tile and split plan for an M x N x K call on a device of `cus` CUs,
 // without a device: out = {1, tile rows, tile columns, K splits}.
 void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out) {
@@ -655,9 +653,12 @@ void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out) {
   out[3] = s;
 }
 
+// Workspace bytes a split-K launch of this shape may use (0: no launch splits K): the largest need of the GEMMs'
+// plans over the formats and dtypes they take (up to 16 rows the int8 short-batch plan alone).
 int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  if (M <= 16 || N <= 0 || K % 64 != 0) return 0;
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
   const int cus = device_info().cus;
+  if (M <= 16) return wk_workspace_bytes(M, N, K, cus);
   const int64_t lds = use_big(M) ? split_bytes<CfgBig>(M, N, K, cus) : split_bytes<CfgSmall>(M, N, K, cus);
   const int64_t rb = rb_workspace_bytes(4, M, N, K, cus);
   const int64_t wk = wk_workspace_bytes(M, N, K, cus);

@@ -73,10 +73,15 @@ void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus
   out[2] = p.splits;
 }
 
-// Bytes of split-K planes a call of this shape may use: no plan has more than 8 ranges, nor more than two
-// workgroups per CU when it splits (of at least N / 128 column tiles).
+// Bytes of split-K planes a call of this shape may use. Past 16 rows: no plan has more than 8 ranges, nor more
+// than two workgroups per CU when it splits (of at least N / 128 column tiles). int8 rows 5 to 16: the plan's own.
 int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
-  if (M <= 16 || M > 64 || N <= 0 || K % RB_BK != 0) return 0;
+  if (M > 64 || N <= 0 || K <= 0 || K % RB_BK != 0) return 0;
+  if (M <= 16) {
+    WkPlan p;
+    if (!wk_rows(8, M, N) || !wk_plan(8, M, N, K, 0, cus, device_info().max_lds, 8, &p)) return 0;
+    return p.splits > 1 ? p.splits * M * N * 4 : 0;
+  }
   const int64_t s = std::min<int64_t>(8, 2 * (int64_t)cus / imq_cdiv(N, 128));
   return s > 1 ? s * M * N * 4 : 0;
 }

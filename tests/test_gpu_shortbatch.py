@@ -132,3 +132,27 @@ def test_decode_rows_of_odd_k_match_the_exact_product(dev, M, N, K, bits, G, sdt
     qw = torch.zeros(N, q.shape[1] + 16, dtype=torch.uint8, device=dev)
     qw[:, :q.shape[1]] = C.u8(q, dev)
     assert torch.equal(op(xw[:, 8:8 + K], qw[:, :q.shape[1]], G, (st.t().contiguous().t(), zt.t().contiguous().t())), y)
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 272, 6784), (8, 2688, 6784), (14, 100, 13696), (16, 512, 10368)])
+def test_int8_decode_rows_split_k_at_any_k(dev, M, N, K):
+    """int8 rows 5 to 16 whose plan splits a K that is no multiple of 256 (no other format's planes are of that
+    shape): the call gets its planes and matches the oracle, and a larger workspace changes nothing."""
+    import torch
+    from infinitemodel_amd import _lib, ops
+    plan = _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, 0, N, sqn=K)
+    need = int(_lib.lib().imq_linear_workspace_bytes(M, N, K))
+    assert plan[1] > 1 and need >= 4 * plan[1] * M * N
+    r = C.rng(N + K)
+    q = r.integers(-127, 128, (N, K), dtype=np.int8)
+    s = oq.round_to(r.uniform(1e-4, 1e-3, (N, 1)).astype(np.float32), "bf16")
+    x = C.bf16_normal(C.rng(M), (M, K))
+    qt, st, xt = torch.from_numpy(q).to(dev), C.to_torch(s, "bf16", dev), C.to_torch(x, "bf16", dev)
+    y = ops.linear_w8(xt, qt, st)
+    _check(y, x, q.astype(np.float64) * s)
+    for extra in (0, 4096):                                   # the planes lie in the workspace, nothing beyond the need
+        ws = torch.full((need + extra,), 0x5a, dtype=torch.uint8, device=dev)
+        y1 = torch.empty_like(y)
+        _lib.call("imq_linear_w8", xt.data_ptr(), K, M, K, qt.data_ptr(), K, st.data_ptr(), 1, 0, N, y1.data_ptr(), N,
+                  ws.data_ptr(), ws.numel(), torch.cuda.current_stream(dev).cuda_stream)
+        assert torch.equal(y1, y) and bool((ws[need:] == 0x5a).all()) and bool((ws != 0x5a).any())

@@ -95,3 +95,19 @@ def test_small_devices_and_other_rows_decline():
     assert _plan(4, 17, 4096, 4096 + 32, 128) is None
     assert _plan(8, 4, 4096, 4096, 0) is None and _plan(8, 5, 4096, 4096, 0) is not None      # int8 from 5 rows
     assert _plan(8, 8, 65552, 4096, 0) is None and _plan(8, 9, 65552, 4096, 0) is not None
+
+
+@pytest.mark.parametrize("bits", [2, 4, 8])
+def test_every_splitting_plan_fits_the_workspace_bound(bits):
+    """The bytes the library asks for hold every plan's planes at the library's own default of 256 CUs (int8 from 5
+    rows, K of any multiple of 64: with too few bytes the call would run unsplit)."""
+    split = 0
+    for K in (64, 1088, 1152, 2112, 3520, 4096, 6784, 8192, 10368, 13696, 14336, 28672):
+        for N in (37, 512, 1024, 2688, 4096, 6208, 14336, 65536):
+            for M in (5, 8, 9, 12, 14, 16, 17, 24, 32, 33, 48, 64):
+                p = _plan(bits, M, N, K, 0 if bits == 8 else 64)
+                if p is None or p[1] == 1:
+                    continue
+                split += 1
+                assert 4 * p[1] * M * N <= _lib.lib().imq_linear_workspace_bytes(M, N, K), (M, N, K, p)
+    assert split > (200 if bits == 8 else 100)
