@@ -205,9 +205,9 @@ __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W
       float t = FAST ? div_by(v, s, r) : v / s;
       if constexpr (DT == IMQ_DT_BF16) t = round_bf16_hw(t);
       else t = round_to<DT>(t);
-      // the conversion saturates and takes a NaN (0 / 0 at an fp16 zero row) to 0, as the host cast does
-      int ci = __float2int_rn(t);
-      ci = ci < -127 ? -127 : ci > 127 ? 127 : ci;
+      // clamped as a float (w / 0 is infinite, and a cast past int's range is undefined); a NaN (a NaN weight, or
+      // 0 / 0 at an fp16 zero row) becomes 0, as in the host cast
+      const int ci = t == t ? __float2int_rn(fminf(fmaxf(t, -127.f), 127.f)) : 0;
       d[e >> 2] |= ((uint32_t)ci & 0xffu) << (8 * (e & 3));
     }
     int8_t* dst = q + n * sq + k;

@@ -78,3 +78,29 @@ def test_packers_dispatch_to_the_device_and_match_the_oracle(dev):
     qo8, so8 = oq.pack_linear_int8(W.float().numpy(), "bf16")
     assert np.array_equal(q8.cpu().numpy(), qo8) and np.array_equal(s8.float().cpu().numpy(), so8)
     assert torch.equal(sc.pack_linear_int2(W.to(dev), 64)[0].cpu(), sc.pack_linear_int2(W, 64)[0])
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("K", [300, 4096, 6000, 20000])
+def test_int8_packer_at_scale_zero_and_non_finite_weights(dev, dt, K):
+    """Quotients outside the codes: an fp16 row whose scale rounds to 0 (w / 0 infinite, 0 / 0 NaN), infinite and NaN
+    weights. Infinities clamp to +-127, NaN becomes 0, and a row's scale is that of its largest non-NaN weight."""
+    import torch
+    from infinitemodel_amd import ops
+    W = (torch.randn(5, K, generator=torch.Generator().manual_seed(K)) * 0.02)
+    W[0] = 0.0
+    W[0, ::3], W[0, 1::3] = 2.0 ** -24, -2.0 ** -24          # the smallest fp16 subnormal: amax / 127 rounds to 0
+    W[1, 5], W[1, K - 1] = float("nan"), float("nan")
+    W[2, 7] = float("-inf")
+    W = W.to(_tdt(dt))
+    q, s = (t.cpu() for t in ops.pack_w8(W.to(dev)))
+    v = W.double()                                           # on the host: torch's GPU divides by a scalar's reciprocal
+    amax = torch.where(v.isnan(), torch.zeros_like(v), v).abs().amax(1, keepdim=True)
+    want_s = torch.maximum((amax.float() / 127).to(W.dtype), torch.tensor(1e-8).to(W.dtype))
+    assert torch.equal(s, want_s)
+    quot = (W.float() / s.float()).to(W.dtype).float()
+    want = torch.where(quot.isnan(), torch.zeros_like(quot), quot.round().clamp(-127, 127)).to(torch.int8)
+    assert torch.equal(q, want)
+    if dt == "fp16":
+        assert float(s[0]) == 0 and set(q[0].unique().tolist()) == {-127, 0, 127}
+    assert set(q[2].unique().tolist()) == {0} and float(s[2]) == float("inf")
