@@ -92,13 +92,6 @@ constexpr int RB_BK = 64;
 #ifndef RB_VALU_PER_MFMA_8
 #define RB_VALU_PER_MFMA_8 3
 #endif
-#ifndef RB_VALU_PER_MFMA_FOLD
-#define RB_VALU_PER_MFMA_FOLD 4
-#endif
-// FOLD: 1 unpacks a step's four B slices at its top (step_fold), 0 one slice ahead (step)
-#ifndef RB_FOLD_EARLY_UNPACK
-#define RB_FOLD_EARLY_UNPACK 1
-#endif
 
 // Bias element i as the raw aligned dword holding it (which lies in the element's page), read
 // without a branch so it can go out with the first loads (a null bias reads `fb`'s first word);
@@ -323,8 +316,6 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   // of two strided global loads per column block -- those loads touch a separate cache line per
   // lane and, issued every step, kept the texture unit busier than the weight stream itself.
   uint32_t* SZ = (uint32_t*)(lds + 3 * A_EL);
-  // FOLD's step unpacks all of a step's weights at its top (step_fold); else one slice ahead
-  constexpr bool EARLY = FOLD && RB_FOLD_EARLY_UNPACK;
   // The MoE forms' staging into LDS (the caller places the barrier after it): the block rows'
   // group sums (FOLD, needs the row plan), and the scale / zero pairs -- with 16-byte aligned
   // scale rows (unit group stride) one 16-byte load covers 16 / sizeof(scale) groups of a column
@@ -438,8 +429,8 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
       sz_scalar();
     }
   };
-  if constexpr (!EARLY) plan_a();
-  if constexpr (MOE != 0 && !EARLY) {
+  if constexpr (!FOLD) plan_a();
+  if constexpr (MOE != 0 && !FOLD) {
     lds_barrier();     // RID, read by the row-sum staging
     stage_moe();
     __syncthreads();   // the prologue's weight-set loads read pairs other threads staged
@@ -571,8 +562,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
     return __builtin_bit_cast(bf16x8_t, d);
   };
 
-  constexpr int VPM = FOLD ? RB_VALU_PER_MFMA_FOLD : BITS == 8 ? RB_VALU_PER_MFMA_8 : BITS == 4 ? RB_VALU_PER_MFMA_4
-                                                                                             : RB_VALU_PER_MFMA_2;
+  constexpr int VPM = BITS == 8 ? RB_VALU_PER_MFMA_8 : BITS == 4 ? RB_VALU_PER_MFMA_4 : RB_VALU_PER_MFMA_2;
   // LDS: three buffers of BM x 64 activations; step kt reads buffer kt % 3 and writes A(kt+1) into
   // buffer (kt+1) % 3, whose last reads (steps kt-2 and the slice-0 prefetch at the end of kt-3)
   // all precede the barrier of step kt-1 -- so one barrier per step suffices, placed after
@@ -586,6 +576,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   //   slice 1: then wait for the LDS writes, barrier, and load A(kt+1+PD) into the freed A set;
   //   after slice 3: load B(kt+PD) into the freed B set.
   auto step = [&](int kt, int rb, int wb, auto bsc) {
+    static_assert(!FOLD || sizeof(bsc) == 0, "the folded form's step is step_fold: this one folds no group");
     constexpr int bs = decltype(bsc)::value;     // kt % PD
     constexpr int as = (bs + 1) % PD;            // A(kt+1) and B(kt+1) live in set (kt+1) % PD
     const uint16_t* Ar = lds + rb * A_EL;
@@ -707,7 +698,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   // outstanding at the top of step kt) so the waits the compiler places at the loop head match
   // the loop's: A(0) is loaded first, then A(1), B(0), ..., with A(0) written to buffer 0 just
   // before A(PD) takes its register set.
-  if constexpr (EARLY) {
+  if constexpr (FOLD) {
     // the fold step's steady state has B(kt), A(kt+1), B(kt+1), A(kt+2) outstanding at the top
     // of step kt
     static_assert(PD == 2, "the fold step keeps two register sets");
@@ -771,7 +762,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void gemm_rb_kernel(RbArgs a) {
   int kt = 0;
   auto run_step = [&](auto uc) {
     const int wb = rb == 2 ? 0 : rb + 1;
-    if constexpr (EARLY) step_fold(kt + decltype(uc)::value, rb, wb, uc);
+    if constexpr (FOLD) step_fold(kt + decltype(uc)::value, rb, wb, uc);
     else step(kt + decltype(uc)::value, rb, wb, uc);
     rb = wb;
   };

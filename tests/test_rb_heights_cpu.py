@@ -32,3 +32,12 @@ def test_plans_cover_and_fit(bits, cus):
 def test_rows_up_to_64_and_odd_k_decline():
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 64, 4096, 128, 4096, sqn=2048) is None
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 600, 4096 + 32, 128, 4096, sqn=2064) is None
+
+
+def test_no_build_switch_picks_the_step():
+    """The folded form's step and the dequantizing one are not interchangeable (only step_fold folds a group's sums), so
+    what a build may override in the kernel's header are the scheduler's VALU counts alone."""
+    import os
+    import re
+    src = open(os.path.join(os.path.dirname(_lib.__file__), "csrc", "rb_kernel.h")).read()
+    assert set(re.findall(r"#\s*if(?:ndef|def)?\s+(\w+)", src)) == {"RB_VALU_PER_MFMA_2", "RB_VALU_PER_MFMA_4", "RB_VALU_PER_MFMA_8"}
