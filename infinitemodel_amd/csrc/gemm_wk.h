@@ -77,15 +77,16 @@ inline size_t wk_lds_bytes(int bits, int ib, int jb, int kps, int gsh, int waves
   return (size_t)waves * ib * wk_rj(ib, jb) * 4096 + groups * wk_szs(jb) * 4;
 }
 
-// PA / PW: steps of activations / weights in flight per wave (PW a multiple of PA); MINW: waves per
-// SIMD the registers are bounded for.
+// PA: steps of activations in flight per wave (1 or 2; of weights two); MINW: waves per SIMD the registers are
+// bounded for.
 // FOLD (M <= 16, groups of 64 codes or more): the decode rows' arithmetic, no weight rounded: B holds the
 // codes themselves, a step's sums start from zero and are folded into the total with the step's scale, and
 // the zero point comes in through the rows' sums (an MFMA against ones): sum s (c - z) x = s (sum c x) -
 // z s (sum x).
-template <int BITS, int IB, int JB, bool TL, int PA, int PW, int MINW, int WAVES = WK_WAVES, bool FOLD = false>
+template <int BITS, int IB, int JB, bool TL, int PA, int MINW, int WAVES = WK_WAVES, bool FOLD = false>
 __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
-  static_assert(PW % PA == 0 && PW >= 2 && PW <= 4, "rings");
+  constexpr int PW = 2;
+  static_assert(PW % PA == 0, "rings");
   static_assert(!FOLD || (IB == 1 && BITS != 8), "folded form: up to 16 rows of a group format");
   constexpr int BK = RB_BK, BN = 32 * JB, NTHR = 64 * WAVES;
   constexpr int XC = FOLD ? 2 : 4 * IB;            // 16-byte activation loads per lane per step (8 rows each)
@@ -164,8 +165,6 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
   };
   fill(std::integral_constant<int, 0>{});
   fill(std::integral_constant<int, 1>{});
-  if constexpr (PW > 2) fill(std::integral_constant<int, 2>{});
-  if constexpr (PW > 3) fill(std::integral_constant<int, 3>{});
   const int g_lo = (kt0 * BK) >> a.gsh;
   if constexpr (BITS != 8) {
     constexpr int TPC = NTHR / BN, SB = 8;
@@ -263,14 +262,8 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
   for (; i + PW <= steps; i += PW) {
     step(std::integral_constant<int, 0>{}, i);
     step(std::integral_constant<int, 1>{}, i + 1);
-    if constexpr (PW > 2) step(std::integral_constant<int, 2>{}, i + 2);
-    if constexpr (PW > 3) step(std::integral_constant<int, 3>{}, i + 3);
   }
   if (i < steps) step(std::integral_constant<int, 0>{}, i);
-  if constexpr (PW > 2)
-    if (i + 1 < steps) step(std::integral_constant<int, 1>{}, i + 1);
-  if constexpr (PW > 3)
-    if (i + 2 < steps) step(std::integral_constant<int, 2>{}, i + 2);
 
   // ---- the waves' sums, RJ 32-column blocks at a time: a wave writes them where its activations were,
   // 16 bytes (4 rows) per lane; a thread adds the 8 waves' quads in wave order ----------------------
@@ -315,9 +308,9 @@ int wk_launch(const WkArgs& a, hipStream_t st) {
   // accumulators allow it: deeper rings at two waves per SIMD measured slower (4096 -> 28672 int4 at
   // M = 32, 64 columns: 22.3 us at 2 / 2 / 4, 28.6 at 4 / 4 / 2), a step's own chain (LDS, unpack,
   // MFMA) being as long as its loads.
-  constexpr int PA = IB == 1 && JB == 2 ? 2 : 1, PW = 2, MINW = IB == 1 && JB <= 2 ? 4 : 2;
+  constexpr int PA = IB == 1 && JB == 2 ? 2 : 1, MINW = IB == 1 && JB <= 2 ? 4 : 2;
   const size_t lds = wk_lds_bytes(BITS, IB, JB, a.kps, a.gsh);
-  auto kern = gemm_wk_kernel<BITS, IB, JB, TL, PA, PW, MINW>;
+  auto kern = gemm_wk_kernel<BITS, IB, JB, TL, PA, MINW>;
   if (lds > 65536) {
     static int attr_set = 0;   // benign race: every caller sets the same value
     if (!__atomic_load_n(&attr_set, __ATOMIC_ACQUIRE)) {
@@ -340,7 +333,7 @@ constexpr int WKD_WAVES = 16;
 template <int BITS>
 int wkd_launch(const WkArgs& a, hipStream_t st) {
   const size_t lds = wk_lds_bytes(BITS, 1, 1, a.kps, a.gsh, WKD_WAVES);
-  auto kern = gemm_wk_kernel<BITS, 1, 1, false, 2, 2, 4, WKD_WAVES, true>;
+  auto kern = gemm_wk_kernel<BITS, 1, 1, false, 2, 4, WKD_WAVES, true>;
   if (lds > 65536) {
     static int attr_set = 0;   // benign race: every caller sets the same value
     if (!__atomic_load_n(&attr_set, __ATOMIC_ACQUIRE)) {
