@@ -77,6 +77,66 @@ inline size_t wk_lds_bytes(int bits, int ib, int jb, int kps, int gsh, int waves
   return (size_t)waves * ib * wk_rj(ib, jb) * 4096 + groups * wk_szs(jb) * 4;
 }
 
+// The outputs of a wave's 32 columns whose folded sum is not finite, again, weight by weight as the generic kernel
+// sums them (generic_gemv, gemv.hip): s sum(c x) - z s sum(x) is infinity less infinity for an infinite
+// activation, whose own product (c - z) s x has a sign. Lane (column n, half h) holds rows m8 + 4 h + e; bit e of
+// `bad` asks for one. Only K steps with an infinite or NaN activation decide, found by the wave together; a row
+// without any (a finite sum that overflowed) takes every step. Reached by non-finite sums only.
+template <int BITS>
+IMQ_DEV void wk_exact(const WkArgs& a, int m8, int n, int h, int lane, uint32_t bad) {
+  const uint8_t* q = a.q + (int64_t)n * a.sqn;
+  const int KT = a.K / RB_BK;
+#pragma unroll 1
+  for (int r = 0; r < 8; ++r) {
+    const bool mine = (r >> 2) == h && ((bad >> (r & 3)) & 1u) != 0;
+    if (__ballot(mine) == 0) continue;
+    const uint16_t* x = a.x + (int64_t)(m8 + r) * a.sxm;
+    float acc = 0.f;
+    bool found = false, live = true;
+#pragma unroll 1
+    for (int pass = 0; pass < 2 && !found; ++pass) {
+#pragma unroll 1
+      for (int k0 = 0; k0 < KT && live; k0 += 64) {
+        bool odd = false;
+        if (k0 + lane < KT) {
+#pragma unroll
+          for (int c8 = 0; c8 < RB_BK / 8; ++c8) {
+            const u32x4_t xv = *(const u32x4_t*)(x + (k0 + lane) * RB_BK + 8 * c8);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              const uint32_t xd = xv[d];
+              odd |= (xd & 0x7f80u) == 0x7f80u || (xd & 0x7f800000u) == 0x7f800000u;
+            }
+          }
+        }
+        uint64_t steps = __ballot(odd);
+        found |= steps != 0;
+        if (pass == 1) steps = __ballot(k0 + lane < KT);
+#pragma unroll 1
+        for (; steps != 0 && live; steps &= steps - 1) {
+          const int k = (k0 + __builtin_ctzll(steps)) * RB_BK;
+          const int64_t g = k >> a.gsh;
+          const float s = round_bf16(wk_f32(wk_raw(a.sc, a.sdt, n * a.ssn + g * a.ssg), a.sdt));
+          const float z = round_bf16(wk_f32(wk_raw(a.zr, a.zdt, n * a.szn + g * a.szg), a.zdt));
+#pragma unroll
+          for (int c8 = 0; c8 < RB_BK / 8; ++c8) {
+            const u32x4_t xv = *(const u32x4_t*)(x + k + 8 * c8);
+            const uint32_t w = BITS == 4 ? *(const uint32_t*)(q + (k + 8 * c8) / 2) : *(const uint16_t*)(q + (k + 8 * c8) / 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              const uint32_t xd = xv[i >> 1];
+              const float c = (float)((w >> (BITS * i)) & ((1u << BITS) - 1u));
+              acc = fmaf(bf16_bits_to_f32((i & 1) ? xd >> 16 : xd & 0xffffu), (c - z) * s, acc);
+            }
+          }
+          live = __ballot(mine && acc == acc) != 0;   // a NaN stays one
+        }
+      }
+    }
+    if (mine) a.y[(int64_t)(m8 + r) * a.sym + n] = (uint16_t)cvt_pk_bf16(acc, 0.f);
+  }
+}
+
 // PA: steps of activations in flight per wave (1 or 2; of weights two); MINW: waves per SIMD the registers are
 // bounded for.
 // FOLD (M <= 16, groups of 64 codes or more): the decode rows' arithmetic, no weight rounded: B holds the
@@ -265,6 +325,7 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
   }
   if (i < steps) step(std::integral_constant<int, 0>{}, i);
 
+  uint32_t bad = 0;                                          // FOLD: the thread's outputs that are not finite
   // ---- the waves' sums, RJ 32-column blocks at a time: a wave writes them where its activations were,
   // 16 bytes (4 rows) per lane; a thread adds the 8 waves' quads in wave order ----------------------
 #pragma unroll
@@ -296,9 +357,16 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
         if constexpr (BITS == 8) s8 = wk_f32(wk_raw(a.sc, a.sdt, (int64_t)n * a.ssn), a.sdt);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (m0 + e < a.M) a.y[(int64_t)(m0 + e) * a.sym + n] = (uint16_t)cvt_pk_bf16(v[e] * s8, 0.f);
+          if (m0 + e < a.M) {
+            a.y[(int64_t)(m0 + e) * a.sym + n] = (uint16_t)cvt_pk_bf16(v[e] * s8, 0.f);
+            if constexpr (FOLD) bad |= __builtin_isfinite(v[e]) ? 0u : 1u << e;
+          }
       }
     }
+  }
+  if constexpr (FOLD) {                                      // one pass: wave w's lanes hold rows 8 w + 4 h + e of column c
+    static_assert(JB == 1 && RJ == 1, "one quad per thread");
+    if (__ballot(bad != 0) != 0) wk_exact<BITS>(a, 8 * wave, min(n0 + c, a.N - 1), h, lane, bad);
   }
 }
 

@@ -156,3 +156,46 @@ def test_int8_decode_rows_split_k_at_any_k(dev, M, N, K):
         _lib.call("imq_linear_w8", xt.data_ptr(), K, M, K, qt.data_ptr(), K, st.data_ptr(), 1, 0, N, y1.data_ptr(), N,
                   ws.data_ptr(), ws.numel(), torch.cuda.current_stream(dev).cuda_stream)
         assert torch.equal(y1, y) and bool((ws[need:] == 0x5a).all()) and bool((ws != 0x5a).any())
+
+
+@pytest.mark.parametrize("M,N,K,bits,G", [(6, 37, 320, 4, 64), (6, 70, 192, 2, 64), (6, 33, 1152, 2, 128), (12, 100, 2944, 4, 128)])
+def test_non_finite_activations_at_odd_k(dev, M, N, K, bits, G):
+    """Decode rows of odd K with infinite and NaN activations: an output is the sum of its own products (q - z) s x, so
+    one infinity gives an infinity of that product's sign (NaN at a zero weight), opposite ones and NaN give NaN, and
+    the other rows are what they are without them."""
+    import torch
+    from infinitemodel_amd import ops
+    r = C.rng(K)
+    codes = r.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    q = np.zeros((N, K * bits // 8), np.uint8)
+    for i in range(8 // bits):
+        q |= codes[:, i::8 // bits] << (bits * i)
+    s = oq.round_to(r.uniform(0.005, 0.05, (N, K // G)).astype(np.float32), "bf16")
+    z = r.integers(0, 1 << bits, (N, K // G)).astype(np.float32)          # whole zero points: zero weights come up
+    x = C.bf16_normal(C.rng(M), (M, K))
+    clean, inf = x.copy(), np.float32("inf")
+    x[1, K - 3], x[2, 5], x[3, 70] = inf, -inf, np.nan
+    x[4, 1], x[4, K // 2] = inf, -inf
+    x[5] = np.nan
+    w = oq.dequant_exact(codes, s, z, G, K).astype(np.float64)
+    assert (w[:, K - 3] == 0).any() or (w[:, 5] == 0).any()
+    with np.errstate(invalid="ignore"):
+        want = (x.astype(np.float64)[:, None, :] * w[None]).sum(-1)
+    op = ops.linear_w4 if bits == 4 else ops.linear_w2
+    args = (C.u8(q, dev), G, (C.to_torch(s, "bf16", dev), C.to_torch(z, "bf16", dev)))
+    y, y0 = op(C.to_torch(x, "bf16", dev), *args), op(C.to_torch(clean, "bf16", dev), *args)
+    got = C.t2np(y)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    at = np.isinf(want)
+    assert np.array_equal(np.isinf(got), at) and np.array_equal(np.sign(got[at]), np.sign(want[at]))
+    rest = [i for i in range(M) if i not in (1, 2, 3, 4, 5)]
+    assert torch.equal(y[rest], y0[rest]) and bool(torch.isfinite(y0).all())
+    # finite activations whose sum of codes overflows, their own products not: the exact sum, all its steps
+    big = np.zeros((M, K), np.float32)
+    big[M - 1, ::K // 8] = 2.0 ** 127                        # times a code of 2 or more: past fp32's range
+    sx = oq.round_to(np.full((N, K // G), 2.0 ** -7, np.float32), "bf16")
+    got = C.t2np(op(C.to_torch(big, "bf16", dev), args[0], G, (C.to_torch(sx, "bf16", dev), args[2][1])))
+    want = big.astype(np.float64) @ oq.dequant_exact(codes, sx, z, G, K).astype(np.float64).T
+    assert np.isfinite(want).all()
+    assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max()
