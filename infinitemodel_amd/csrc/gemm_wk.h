@@ -81,9 +81,13 @@ inline size_t wk_lds_bytes(int bits, int ib, int jb, int kps, int gsh, int waves
 // sums them (generic_gemv, gemv.hip): s sum(c x) - z s sum(x) is infinity less infinity for an infinite
 // activation, whose own product (c - z) s x has a sign. Lane (column n, half h) holds rows m8 + 4 h + e; bit e of
 // `bad` asks for one. Only K steps with an infinite or NaN activation decide, found by the wave together; a row
-// without any (a finite sum that overflowed) takes every step. Reached by non-finite sums only.
+// without any (a finite sum that overflowed) takes every step. Reached by non-finite sums only, and a call of its
+// own on the kernel's arguments in memory, so that it takes no registers from the loop.
+typedef const __attribute__((address_space(4))) WkArgs* WkKernarg;
 template <int BITS>
-IMQ_DEV void wk_exact(const WkArgs& a, int m8, int n, int h, int lane, uint32_t bad) {
+__device__ __attribute__((noinline)) void wk_exact(WkKernarg ap, int m8, int n, uint32_t bad) {
+  const WkArgs a = *(const WkArgs*)ap;
+  const int lane = threadIdx.x & 63, h = lane >> 5;
   const uint8_t* q = a.q + (int64_t)n * a.sqn;
   const int KT = a.K / RB_BK;
 #pragma unroll 1
@@ -99,7 +103,7 @@ IMQ_DEV void wk_exact(const WkArgs& a, int m8, int n, int h, int lane, uint32_t 
       for (int k0 = 0; k0 < KT && live; k0 += 64) {
         bool odd = false;
         if (k0 + lane < KT) {
-#pragma unroll
+#pragma unroll 1
           for (int c8 = 0; c8 < RB_BK / 8; ++c8) {
             const u32x4_t xv = *(const u32x4_t*)(x + (k0 + lane) * RB_BK + 8 * c8);
 #pragma unroll
@@ -118,7 +122,7 @@ IMQ_DEV void wk_exact(const WkArgs& a, int m8, int n, int h, int lane, uint32_t 
           const int64_t g = k >> a.gsh;
           const float s = round_bf16(wk_f32(wk_raw(a.sc, a.sdt, n * a.ssn + g * a.ssg), a.sdt));
           const float z = round_bf16(wk_f32(wk_raw(a.zr, a.zdt, n * a.szn + g * a.szg), a.zdt));
-#pragma unroll
+#pragma unroll 1
           for (int c8 = 0; c8 < RB_BK / 8; ++c8) {
             const u32x4_t xv = *(const u32x4_t*)(x + k + 8 * c8);
             const uint32_t w = BITS == 4 ? *(const uint32_t*)(q + (k + 8 * c8) / 2) : *(const uint16_t*)(q + (k + 8 * c8) / 4);
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void gemm_wk_kernel(WkArgs a) {
   }
   if constexpr (FOLD) {                                      // one pass: wave w's lanes hold rows 8 w + 4 h + e of column c
     static_assert(JB == 1 && RJ == 1, "one quad per thread");
-    if (__ballot(bad != 0) != 0) wk_exact<BITS>(a, 8 * wave, min(n0 + c, a.N - 1), h, lane, bad);
+    if (__ballot(bad != 0) != 0) wk_exact<BITS>((WkKernarg)__builtin_amdgcn_kernarg_segment_ptr(), 8 * wave, min(n0 + c, a.N - 1), bad);
   }
 }
 
@@ -401,7 +405,9 @@ constexpr int WKD_WAVES = 16;
 template <int BITS>
 int wkd_launch(const WkArgs& a, hipStream_t st) {
   const size_t lds = wk_lds_bytes(BITS, 1, 1, a.kps, a.gsh, WKD_WAVES);
-  auto kern = gemm_wk_kernel<BITS, 1, 1, false, 2, 4, WKD_WAVES, true>;
+  // int2 fits the registers of five waves per SIMD: the next workgroup's 16 waves start once the waves without outputs
+  // have ended (at four, 64 -> 152064 M = 4 94 us against 82)
+  auto kern = gemm_wk_kernel<BITS, 1, 1, false, 2, BITS == 2 ? 5 : 4, WKD_WAVES, true>;
   if (lds > 65536) {
     static int attr_set = 0;   // benign race: every caller sets the same value
     if (!__atomic_load_n(&attr_set, __ATOMIC_ACQUIRE)) {
