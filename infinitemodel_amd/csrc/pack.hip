@@ -154,6 +154,13 @@ __global__ __launch_bounds__(256) void pack_g_kernel(const void* __restrict__ W,
   }
 }
 
+// v_cvt_i32_f32: truncates, saturates out-of-range values, NaN -> 0.
+IMQ_DEV int cvt_i32(float f) {
+  int i;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(f));
+  return i;
+}
+
 // WPR waves per row (1 or 4), 8 columns per lane and pass: the row's |w| max, then the codes. The
 // first NV passes keep the row in registers, so rows up to 512 NV WPR columns are read once (longer
 // ones re-read their tail); divisions as in pack_g_kernel, one shared reciprocal per row. 4096 -> 14336 bf16:
@@ -205,9 +212,11 @@ __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W
       float t = FAST ? div_by(v, s, r) : v / s;
       if constexpr (DT == IMQ_DT_BF16) t = round_bf16_hw(t);
       else t = round_to<DT>(t);
-      // clamped as a float (w / 0 is infinite, and a cast past int's range is undefined); a NaN (a NaN weight, or
-      // 0 / 0 at an fp16 zero row) becomes 0, as in the host cast
-      const int ci = t == t ? __float2int_rn(fminf(fmaxf(t, -127.f), 127.f)) : 0;
+      // the instruction itself, whose results are defined where a C++ cast's are not: w / 0 saturates, and a NaN (a
+      // NaN weight, or 0 / 0 at an fp16 zero row) becomes 0, as in the host cast. (A float clamp and a compare
+      // before a cast: 4096 x 4096 15.8 us against 14.0.)
+      int ci = cvt_i32(rintf(t));
+      ci = ci < -127 ? -127 : ci > 127 ? 127 : ci;
       d[e >> 2] |= ((uint32_t)ci & 0xffu) << (8 * (e & 3));
     }
     int8_t* dst = q + n * sq + k;
