@@ -161,21 +161,21 @@ IMQ_DEV int cvt_i32(float f) {
   return i;
 }
 
-// WPR waves per row (1 or 4), 8 columns per lane and pass: the row's |w| max, then the codes. The
-// first NV passes keep the row in registers, so rows up to 512 NV WPR columns are read once (longer
-// ones re-read their tail); divisions as in pack_g_kernel, one shared reciprocal per row. 4096 -> 14336 bf16:
-// 39 us, 4.5 TB/s (one wave per row with 2-byte loads and a division per element: 114 us).
-template <int DT, int WPR, int NV>
+// LPR lanes per row (8 to 64 of a wave, or the workgroup's 256), 8 columns per lane and pass: the row's |w| max,
+// then the codes. The first NV passes keep the row in registers, so rows up to 8 LPR NV columns are read once
+// (longer ones re-read their tail); divisions as in pack_g_kernel, one shared reciprocal per row. 4096 -> 14336
+// bf16: 39 us, 4.5 TB/s (one wave per row with 2-byte loads and a division per element: 114 us).
+template <int DT, int LPR, int NV>
 __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W, int64_t sw, int64_t N,
                                                       int64_t K, int8_t* __restrict__ q, int64_t sq,
                                                       void* __restrict__ sc, int64_t ssn, bool wvec, bool qvec) {
-  constexpr int64_t STEP = 512 * WPR;                  // columns of a pass
+  constexpr int64_t STEP = 8 * LPR;                    // columns of a pass
   __shared__ float part[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t n0 = WPR == 1 ? (int64_t)blockIdx.x * 4 + wave : blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rl = threadIdx.x % LPR;
+  const int64_t n0 = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
   const bool live = n0 < N;
   const int64_t n = live ? n0 : N - 1;
-  const int64_t row = n * sw, kl = 8 * (WPR == 1 ? lane : (int)threadIdx.x);
+  const int64_t row = n * sw, kl = 8 * rl;
   Raw8<DT> raw[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) load8_row<DT>(raw[i], W, row, kl + i * STEP, K, wvec);
@@ -191,8 +191,8 @@ __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(get8<DT>(t, e)));
   }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-  if constexpr (WPR == 4) {
+  for (int off = (LPR < 64 ? LPR : 64) / 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
+  if constexpr (LPR == 256) {
     if (lane == 0) part[wave] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
@@ -239,7 +239,7 @@ __global__ __launch_bounds__(256) void pack_w8_kernel(const void* __restrict__ W
   };
   if (fast) codes(std::true_type{});
   else codes(std::false_type{});
-  if (live && lane == 0 && (WPR == 1 || wave == 0)) store_from_f32<DT>(sc, n * ssn, s);
+  if (live && rl == 0) store_from_f32<DT>(sc, n * ssn, s);
 }
 
 bool dt_ok(int d) { return d == IMQ_DT_BF16 || d == IMQ_DT_FP16 || d == IMQ_DT_FP32; }
@@ -282,8 +282,9 @@ int launch_g(const void* W, int64_t sw, int64_t N, int64_t in_f, int64_t G, uint
   return IMQ_ERR_UNSUPPORTED;
 }
 
-// A wave per row while the row fits one wave's registers (4096 columns), else four; NV passes cover
-// the row where they can.
+// As many lanes as a short row has 8-column pieces (64 columns x 100000 rows: 25 us with a wave of 2-byte loads per
+// row, 40 with a wave of 16-byte loads, 8 of its lanes reading, 7 with 8 rows per wave), a wave per row
+// while the row fits its registers (4096 columns), else four; NV passes cover the row where they can.
 template <int DT>
 int launch_w8(const void* W, int64_t sw, int64_t N, int64_t K, int8_t* q, int64_t sq, void* sc, int64_t ssn,
               hipStream_t st) {
@@ -293,16 +294,21 @@ int launch_w8(const void* W, int64_t sw, int64_t N, int64_t K, int8_t* q, int64_
   const int64_t step = 1 << 22;                        // rows a launch: its threads stay below 2^31
   for (int64_t n = 0; n < N; n += step) {
     const int64_t rows = std::min(step, N - n);
-    const dim3 g((unsigned)(K <= 4096 ? (rows + 3) / 4 : rows)), b(256);
+    const int lpr = K <= 64 ? 8 : K <= 128 ? 16 : K <= 256 ? 32 : K <= 4096 ? 64 : 256;
+    const dim3 g((unsigned)((rows * lpr + 255) / 256)), b(256);
     const void* Wn = (const char*)W + n * sw * ES;
     void* scn = (char*)sc + n * ssn * ES;
     int8_t* qn = q + n * sq;
-#define IMQ_P8(W_, V_) pack_w8_kernel<DT, W_, V_><<<g, b, 0, st>>>(Wn, sw, rows, K, qn, sq, scn, ssn, wvec, qvec)
-    if (K <= 1024) IMQ_P8(1, 2);
-    else if (K <= 2048) IMQ_P8(1, 4);
-    else if (K <= 4096) IMQ_P8(1, 8);
-    else if (K <= 8192) IMQ_P8(4, 4);
-    else IMQ_P8(4, 8);
+#define IMQ_P8(L_, V_) pack_w8_kernel<DT, L_, V_><<<g, b, 0, st>>>(Wn, sw, rows, K, qn, sq, scn, ssn, wvec, qvec)
+    if (lpr == 8) IMQ_P8(8, 1);
+    else if (lpr == 16) IMQ_P8(16, 1);
+    else if (lpr == 32) IMQ_P8(32, 1);
+    else if (K <= 512) IMQ_P8(64, 1);
+    else if (K <= 1024) IMQ_P8(64, 2);
+    else if (K <= 2048) IMQ_P8(64, 4);
+    else if (K <= 4096) IMQ_P8(64, 8);
+    else if (K <= 8192) IMQ_P8(256, 4);
+    else IMQ_P8(256, 8);
 #undef IMQ_P8
     IMQ_LAUNCH_CHECK();
   }

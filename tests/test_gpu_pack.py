@@ -104,3 +104,16 @@ def test_int8_packer_at_scale_zero_and_non_finite_weights(dev, dt, K):
     if dt == "fp16":
         assert float(s[0]) == 0 and set(q[0].unique().tolist()) == {-127, 0, 127}
     assert set(q[2].unique().tolist()) == {0} and float(s[2]) == float("inf")
+
+
+@pytest.mark.parametrize("dt", DTS)
+@pytest.mark.parametrize("N,K", [(1, 1), (9, 64), (33, 65), (17, 128), (300, 100), (5, 129), (40, 250), (7, 256), (6, 257), (21, 512), (6, 513)])
+def test_int8_packer_short_rows(dev, dt, N, K):
+    """Rows of 8, 16, 32 and 64 lanes, several to a wave: each row's scale and codes are its own (special rows beside
+    ordinary ones), up to the last column and row."""
+    from infinitemodel_amd import ops, shard_compile as sc
+    W = _weights(N, K, dt, seed=N * K)
+    qh, sh = sc.pack_linear_int8(W)
+    qd, sd = ops.pack_w8(W.to(dev))
+    assert np.array_equal(qd.cpu().numpy(), qh.numpy())
+    assert np.array_equal(_bits(sd), _bits(sh))
