@@ -653,6 +653,18 @@ void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out) {
   out[3] = s;
 }
 
+// us of a call of this kernel where the K ranges are short, so that a tile's fixed cost (its first loads, its
+// epilogue) counts: fitted to graph replays of the kernel alone over K 64 .. 28672 x N 384 .. 131072 x M 17 .. 2048
+// (4 to 8% rms). The other GEMMs weigh their own plans against it (gemm_wk.hip, gemm_rbm.hip).
+double gemm_lds_us(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes) {
+  int64_t out[5] = {};
+  gemm_plan_query(M, N, K, cus, out);
+  const int64_t s = planes ? out[3] : 1, kps = imq_cdiv(K / 64, s), W = imq_cdiv(M, out[1]) * imq_cdiv(N, out[2]) * s;
+  const double sum = s > 1 ? 1.3 + 1.2e-6 * s * M * N : 0;
+  if (out[1] == CfgBig::BM) return 1 + (double)imq_cdiv(W, cus) * (5.5 + kps * (bits == 8 ? 0.88 : 0.93)) + sum;
+  return 2.9 + (W <= cus ? 1.0 : 1.42 * imq_cdiv(W, 2 * cus)) * (1.65 + kps * (bits == 8 ? 0.65 : 0.76)) + 0.5e-6 * M * N + sum;
+}
+
 // Workspace bytes a split-K launch of this shape may use (0: no launch splits K): the largest need of the GEMMs'
 // plans over the formats and dtypes they take (up to 16 rows the int8 short-batch plan alone).
 int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {

@@ -8,6 +8,7 @@ int rbm_run4(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStrea
 int rbm_run2(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStream_t st);
 int rbm_run8(const RbArgs& a, RbmPlan p, int sdt, bool tiled, void* ws, hipStream_t st);
 void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out);
+double gemm_lds_us(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes);
 
 namespace {
 
@@ -62,12 +63,36 @@ double lds_us(int64_t M, int64_t N, int64_t K, int cus, bool planes) {
   return 3 + (double)imq_cdiv(W, cus) * imq_cdiv(K / RB_BK, s) * (out[1] == 256 ? 1.1 : 0.87) + planes_us((int)s, M, N);
 }
 
+// A plan's us where its K ranges are short: the fixed cost of a tile grows with its height (the epilogue), fitted to
+// graph replays at every height and M 65 .. 512 (7.5% rms; rbm_plan and lds_us are fitted to long ranges, where
+// they are nearer).
+double short_us(int bits, int64_t M, int64_t N, int64_t K, int cus, const RbmPlan& p) {
+  const int64_t kps = imq_cdiv(K / RB_BK, p.splits), W = imq_cdiv(M, 32 * p.ib) * imq_cdiv(N, 256) * p.splits;
+  const double t = 0.6 + 1.88 * p.ib + kps * (bits == 8 ? 0.21 + 0.146 * p.ib : 0.447 + 0.127 * p.ib);
+  const double rounds = W <= cus ? 1 : p.ib <= 4 ? 1.72 * imq_cdiv(W, 2 * cus) : (double)imq_cdiv(W, cus);
+  return 0.8 + rounds * t + (p.splits > 1 ? 1 + 1.15e-6 * p.splits * M * N : 0);
+}
+
+// Whether this GEMM takes a call, the LDS-dequant GEMM the rest. us, LDS-dequant against this kernel, where each side
+// of a line was wrong before it: 200 rows, 64 -> 152064 int4 31 / 39 and 448 -> 100000 int4 at 512 rows 87 / 106; int8
+// at 96 rows, 1024 -> 4096 13.0 / 13.9 (8 steps a range); int2 at 1024 rows, 64 -> 152064 117 / 162.
 bool rbm_takes(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, bool planes, RbmPlan* p) {
   if (M <= 64 || N <= 0 || K <= 0 || K % RB_BK != 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return false;
   if (bits != 8 && (G < 32 || (G & (G - 1)) != 0)) return false;
   const double us = rbm_plan(bits, M, N, K, cus, planes, p);
-  // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within its own spread
-  return us > 0 && (M > 512 || us < 0.96 * lds_us(M, N, K, cus, planes));
+  if (us <= 0) return false;
+  if (M > 512) {
+    // int2 of short K and tiles for more than half of 256 CUs: the fixed cost decides. int4 and int8 have had a
+    // register-B form above 512 rows throughout, and smaller grids differ by a microsecond at most.
+    if (bits != 2 || K > 512 || imq_cdiv(M, 32 * p->ib) * imq_cdiv(N, 256) <= 128) return true;
+    return short_us(bits, M, N, K, cus, *p) < gemm_lds_us(bits, M, N, K, cus, planes);
+  }
+  // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within its own spread, and short ranges where
+  // its fixed cost is the smaller (by more than the two fits' spread where K is only short for its splits: at 12%
+  // modelled, 4 to 13% measured; below that the two are within 5% of each other)
+  if (us >= 0.96 * lds_us(M, N, K, cus, planes)) return false;
+  if (imq_cdiv(K / RB_BK, p->splits) > 12) return true;
+  return short_us(bits, M, N, K, cus, *p) < (K <= 512 ? 1.0 : 1.12) * gemm_lds_us(bits, M, N, K, cus, planes);
 }
 
 }  // namespace

@@ -11,6 +11,7 @@ int wk_run2(const WkArgs& a, int jb, bool tiled, hipStream_t st);
 int wk_run8(const WkArgs& a, int jb, bool tiled, hipStream_t st);
 int wkd_run2(const WkArgs& a, hipStream_t st);
 int wkd_run4(const WkArgs& a, hipStream_t st);
+double gemm_lds_us(int bits, int64_t M, int64_t N, int64_t K, int cus, bool planes);
 
 namespace {
 
@@ -55,10 +56,34 @@ bool wk_plan(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int 
 // are exact in bf16: from 5, where the skinny kernel restages the activations for every 16 rows of
 // weights -- us, skinny -> this at M = 5 / 16: 4096 -> 4096 10.3 / 13.6 -> 8.8 / 8.7, 14336 -> 4096 25.9 / 37.8 ->
 // 18.0 / 18.3, 4096 -> 14336 18.2 / 25.2 -> 15.8 / 16.3; at a vocabulary's width the skinny kernel's
-// persistent tiles win up to 8 rows (3584 -> 152064 M = 8 100 against 116, M = 16 144 against 121).
-bool wk_rows(int bits, int64_t M, int64_t N) {
-  if (bits == 8 && M <= 16) return M > 8 || (M > 4 && N <= 65536);
+// persistent tiles win up to 8 rows (3584 -> 152064 M = 8 100 against 116, M = 16 144 against 121), and at a short K,
+// where this form's sum over its waves costs more than the whole call, while rows times K stay small (64 -> 65536
+// M = 8 / 16 5.8 / 7.1 against 9.1 / 9.0, 192 -> 65536 M = 8 7.7 against 9.0, 256 -> 65536 M = 16 13 against 8).
+bool wk_rows(int bits, int64_t M, int64_t N, int64_t K) {
+  if (bits == 8 && M <= 16) return M > 4 && (M > 8 || N <= 65536) && (N <= 16384 || M * K > 1536);
   return M > 16 && M <= 64;
+}
+
+// Whether the plan is worth taking past 16 rows. Where the workgroups outnumber the CUs each pays its fixed cost
+// (staging, the sum over its waves) in turn, and at a short K the LDS-dequant GEMM's tiles, half as many with
+// stores as wide, are faster: us, LDS-dequant against this, 64 -> 131072 int4 M = 17 / 64 11 / 25 and 14 / 48, 512 -> 65536
+// int4 M = 64 21 / 26, 768 -> 65536 int8 M = 64 19 / 24, but 768 -> 65536 int4 M = 17 21 / 16 and 2048 -> 65536 int4 M = 64
+// 51 / 42. This form's us is a fit to graph replays of such calls (3 to 12% rms), c + rounds (f + step per K step of a
+// wave + per K / 512), with a margin where the fit runs high; from three steps a wave it has been the faster at every
+// width, and grids within the CUs differ by 2 us at most, at K = 64.
+bool wk_worth(int bits, int64_t M, int64_t N, int64_t K, int cus, const WkPlan& p) {
+  const int64_t W = imq_cdiv(N, 32 * p.jb);
+  if (M <= 16 || p.splits > 1 || W <= cus || K > 2 * WK_WAVES * RB_BK) return true;
+  struct Cost { double c, f, step, per; };
+  const bool one = p.jb == 1;
+  const Cost k = bits == 8 ? (M > 32 ? (one ? Cost{5.3, 0.33, 0, 1.13} : Cost{3.9, 2.85, 0.1, 1.3})
+                                     : (one ? Cost{3.4, 0.3, 0.2, 0.4} : Cost{3.1, 0.6, 0.9, 0.35}))
+                 : M > 32  ? (one ? Cost{6.9, 0.36, 0.3, 0.45} : Cost{6.0, 4.5, 0.2, 0.74})
+                 : one     ? Cost{3.2, 2.2, 0.75, 0}
+                 : bits == 4 ? (p.jb == 2 ? Cost{5.1, 1.95, 0.2, 0.55} : Cost{7.3, 3.3, 0.47, 1.56})
+                             : (p.jb == 2 ? Cost{2.9, 3.3, 0.7, 0.46} : Cost{6.3, 1.76, 0, 1.94});
+  const double steps = (double)imq_cdiv(K / RB_BK, WK_WAVES), us = k.c + (double)W / cus * (k.f + k.step * steps + k.per * K / 512);
+  return us < (bits == 4 && M <= 32 ? 1.1 : bits == 8 || M <= 32 ? 1.0 : 1.05) * gemm_lds_us(bits, M, N, K, cus, true);
 }
 
 }  // namespace
@@ -67,10 +92,11 @@ bool wk_rows(int bits, int64_t M, int64_t N) {
 // device: out = {takes the call, 32-column blocks per workgroup, K ranges}.
 void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out) {
   WkPlan p{0, 0};
-  const bool takes = wk_rows(bits, M, N) && K % RB_BK == 0 && wk_plan(bits, M, N, K, G, cus, max_lds, 8, &p);
+  const bool takes = wk_rows(bits, M, N, K) && K % RB_BK == 0 && wk_plan(bits, M, N, K, G, cus, max_lds, 8, &p) &&
+                     wk_worth(bits, M, N, K, cus, p);
   out[0] = takes ? 1 : 0;
-  out[1] = p.jb;
-  out[2] = p.splits;
+  out[1] = takes ? p.jb : 0;
+  out[2] = takes ? p.splits : 0;
 }
 
 // Bytes of split-K planes a call of this shape may use. Past 16 rows: no plan has more than 8 ranges, nor more
@@ -79,7 +105,7 @@ int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
   if (M > 64 || N <= 0 || K <= 0 || K % RB_BK != 0) return 0;
   if (M <= 16) {
     WkPlan p;
-    if (!wk_rows(8, M, N) || !wk_plan(8, M, N, K, 0, cus, device_info().max_lds, 8, &p)) return 0;
+    if (!wk_rows(8, M, N, K) || !wk_plan(8, M, N, K, 0, cus, device_info().max_lds, 8, &p)) return 0;
     return p.splits > 1 ? p.splits * M * N * 4 : 0;
   }
   const int64_t s = std::min<int64_t>(8, 2 * (int64_t)cus / imq_cdiv(N, 128));
@@ -92,12 +118,13 @@ int64_t wk_workspace_bytes(int64_t M, int64_t N, int64_t K, int cus) {
 int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled) {
-  if (!wk_rows(bits, M, N) || K <= 0 || K % RB_BK != 0) return IMQ_ERR_UNSUPPORTED;
+  if (!wk_rows(bits, M, N, K) || K <= 0 || K % RB_BK != 0) return IMQ_ERR_UNSUPPORTED;
   if (((uintptr_t)x & 15) || (sxm & 7) || ((uintptr_t)q & 15) || (sqn & 15)) return IMQ_ERR_UNSUPPORTED;
   if ((64 * sxm + K) * 2 > 0x7fffffff || 128 * sqn + K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
   const DevInfo d = device_info();
   WkPlan p;
   if (!wk_plan(bits, M, N, K, G, d.cus, d.max_lds, 8, &p)) return IMQ_ERR_UNSUPPORTED;
+  if (!wk_worth(bits, M, N, K, d.cus, p)) return IMQ_ERR_UNSUPPORTED;
   if (p.splits > 1 && (!ws || wsb < (int64_t)p.splits * M * N * 4 || ((uintptr_t)ws & 15)))
     if (!wk_plan(bits, M, N, K, G, d.cus, d.max_lds, 1, &p)) return IMQ_ERR_UNSUPPORTED;
   const int KT = (int)(K / RB_BK), kps = (KT + p.splits - 1) / p.splits;

@@ -199,3 +199,22 @@ def test_non_finite_activations_at_odd_k(dev, M, N, K, bits, G):
     want = big.astype(np.float64) @ oq.dequant_exact(codes, sx, z, G, K).astype(np.float64).T
     assert np.isfinite(want).all()
     assert np.abs(got - want).max() <= 2.0 ** -8 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("M,N,K,bits,G", [(17, 33000, 64, 4, 64), (64, 20000, 64, 4, 32), (33, 33008, 512, 2, 64), (24, 131072, 64, 2, 64),
+                                          (64, 33000, 192, 8, 0), (8, 16400, 192, 8, 0), (16, 16400, 64, 8, 0)])
+def test_short_k_and_wide_n_are_other_kernels_calls(dev, M, N, K, bits, G):
+    """Row counts of the short-batch GEMM whose plan it declines (workgroups for more than the CUs, few K steps each): the
+    LDS-dequant GEMM's (int8 decode rows: the skinny kernel's), against the oracle."""
+    import torch
+    from infinitemodel_amd import _lib, ops
+    assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, G, N, sqn=K * bits // 8) is None
+    x = C.bf16_normal(C.rng(M), (M, K))
+    xt = C.to_torch(x, "bf16", dev)
+    if bits == 8:
+        r = C.rng(N + K)
+        q = r.integers(-127, 128, (N, K), dtype=np.int8)
+        s = oq.round_to(r.uniform(1e-4, 1e-3, (N, 1)).astype(np.float32), "bf16")
+        return _check(ops.linear_w8(xt, torch.from_numpy(q).to(dev), C.to_torch(s, "bf16", dev)), x, q.astype(np.float64) * s)
+    q, s, z, w = _group_case(dev, bits, N, K, G, "bf16", "bf16", seed=M + N + K)
+    _check((ops.linear_w4 if bits == 4 else ops.linear_w2)(xt, q, G, (s, z)), x, w)

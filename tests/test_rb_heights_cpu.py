@@ -29,6 +29,21 @@ def test_plans_cover_and_fit(bits, cus):
     assert taken > 100
 
 
+def test_short_k_ranges_decline():
+    """Few K steps a range and tiles past the CUs, or (up to 512 rows) a tile's fixed cost alone: the LDS-dequant GEMM's,
+    measured. int4 and int8 stay above 512 rows, and a model's prefill shapes keep their plans."""
+    plan = lambda b, M, N, K: _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, 0 if b == 8 else 64, N, sqn=K * b // 8)   # noqa: E731
+    for M, N, K in ((200, 152064, 64), (512, 100000, 448), (256, 152064, 256)):
+        assert all(plan(b, M, N, K) is None for b in (2, 4)), (M, N, K)
+    assert plan(8, 96, 4096, 1024) is None and plan(8, 128, 2560, 2944) is None and plan(8, 150, 1008, 1024) is not None
+    assert plan(2, 1024, 152064, 64) is None and plan(2, 1024, 40000, 512) is None and plan(2, 1024, 40000, 2048) is not None
+    assert plan(4, 1024, 152064, 64) is not None and plan(8, 1024, 152064, 64) is not None
+    for b in (2, 4, 8):
+        for M, N, K in ((300, 28672, 4096), (384, 28672, 4096), (777, 28672, 8192), (2048, 4096, 14336)):
+            assert plan(b, M, N, K) is not None, (b, M, N, K)
+    assert plan(4, 200, 28672, 4096)[:2] == (7, 2) and plan(8, 512, 14336, 4096)[:2] == (4, 1) and plan(8, 512, 4096, 14336)[:2] == (4, 4)
+
+
 def test_rows_up_to_64_and_odd_k_decline():
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 64, 4096, 128, 4096, sqn=2048) is None
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 600, 4096 + 32, 128, 4096, sqn=2064) is None

@@ -111,3 +111,17 @@ def test_every_splitting_plan_fits_the_workspace_bound(bits):
                 split += 1
                 assert 4 * p[1] * M * N <= _lib.lib().imq_linear_workspace_bytes(M, N, K), (M, N, K, p)
     assert split > (200 if bits == 8 else 100)
+
+
+def test_short_k_and_wide_n_decline():
+    """Where the workgroups outnumber the CUs and each has few K steps, the LDS-dequant GEMM (int8 decode rows: the skinny
+    kernel) measured faster; at a model's widths the form keeps its rows."""
+    for bits in (2, 4, 8):
+        G = 0 if bits == 8 else 64
+        for M in (17, 33, 64):
+            assert _plan(bits, M, 131072, 64, G) is None and _plan(bits, M, 4096, 64, G) is not None
+            for N, K in ((4096, 4096), (6144, 4096), (28672, 4096), (4096, 14336), (14336, 4096), (8192, 28672), (152064, 3584), (9728, 896)):
+                assert _plan(bits, M, N, K, G) is not None, (bits, M, N, K)
+        assert _plan(bits, 64, 65536, 512, G) is None and _plan(bits, 64, 65536, 2048, G) is not None
+    assert _plan(8, 8, 65536, 192, 0) is None and _plan(8, 9, 65536, 192, 0) is not None
+    assert _plan(8, 16, 20000, 64, 0) is None and _plan(8, 16, 16384, 64, 0) is not None
