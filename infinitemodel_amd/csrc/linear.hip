@@ -43,11 +43,26 @@ int gemm_wkd(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, con
              const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
              int64_t N, int64_t G, uint16_t* y, int64_t sym, hipStream_t st);
 // Whether decode rows go to the folded short-batch form before the skinny kernels: K not whole line-steps (no
-// line or K-split kernel reads it), more than 8 rows, K long enough that a wave has several steps. us, skinny
-// -> folded: int4 2880 -> 5120 (K_pad 2944) M = 12 / 16 15.5 / 17.4 -> 13.5 / 13.7, int2 11008 -> 4096 M = 8 / 16
-// 17.8 / 31.7 -> 15.8 / 17.6, 3328 -> 4096 M = 16 11.3 -> 9.0; M = 4 11.7 -> 13.2 and short K (768 -> 16384
-// M = 16 10.7 -> 12.4) stay.
-bool folded_first(int bits, int64_t M, int64_t K) { return M > 8 && M <= 16 && K >= 2048 && K % (1024 / bits) != 0; }
+// line or K-split kernel reads it), and
+//   * many activations, as the skinny kernels' time steps up with what they stage: int4 from 72 K elements, where they
+//     no longer fit the LDS and are staged in chunks, int2 from 33 K; or
+//   * more than 8 rows of a longer K over at most one 32-column workgroup per CU (int4: over more than half the CUs;
+//     below that its skinny kernel is not short of tiles either).
+// us, cold weights, skinny -> folded: int4 6272 -> 9728 M = 10 / 12 21 / 41 -> 23.5 / 24, 11136 -> 5120 M = 6 / 7 29 / 41 -> 18 / 18,
+// 2944 -> 5120 M = 8 / 9 / 16 9.3 / 9.7 / 11.4 -> 8.6 / 8.5 / 8.7, 2944 -> 2560 M = 9 / 16 6.8 / 9.0 -> 8.5 / 8.8, 2944 -> 9728 M = 9 /
+// 16 12 / 14 -> 16 / 18; int2 3328 -> 9728 M = 9 / 12 15 / 20 -> 15 / 15, 11008 -> 5120 M = 8 / 16 43 / 65 -> 15 / 17, 2304 -> 1024
+// M = 9 / 14 7.8 / 9.4 -> 7.6 / 7.6, 2304 -> 18944 M = 12 / 16 19 / 26 -> 20 / 20.
+bool folded_first(int bits, int64_t M, int64_t N, int64_t K) {
+  if (M <= 4 || M > 16 || K % (1024 / bits) == 0) return false;
+  if (M * K >= (bits == 4 ? 72 << 10 : 33 << 10)) return true;
+  const int64_t tiles = imq_cdiv(N, 32), cus = device_info().cus;
+  return M > 8 && K >= 2048 && tiles <= cus && (bits == 2 || 2 * tiles > cus);
+}
+// Whether the generic kernel (one wave per row) is the faster for rows no decode kernel takes: few rows of a short K,
+// less than the folded form's staging and sum over 16 waves. us, generic against folded: 64 -> 1024 M = 1 / 16 3.9 / 5.3
+// against 6.7 / 7.0, 128 -> 1024 M = 8 / 16 5.8 / 7.2 against 6.9 / 7.0, 320 -> 1024 M = 1 / 4 5.4 / 6.8 against 6.2 / 6.3,
+// 64 -> 4096 M = 1 6.7 against 6.2.
+bool generic_first(int64_t M, int64_t N, int64_t K) { return N <= 2048 && K * (M + 4) <= 2048; }
 int gemm_wk(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, int64_t sqn,
             const void* sc, int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt,
             int64_t N, int64_t G, uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st, bool tiled);
@@ -154,7 +169,7 @@ extern "C" int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int
   const uint16_t* xb = (const uint16_t*)x;
   uint16_t* yb = (uint16_t*)y;
   const uint8_t* q = (const uint8_t*)qweight;
-  if (imq::folded_first(4, M, K_pad)) {
+  if (imq::folded_first(4, M, N, K_pad)) {
     rc = imq::gemm_wkd(4, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
                        z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
     if (rc != IMQ_ERR_UNSUPPORTED) return rc;
@@ -169,9 +184,11 @@ extern "C" int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int
                       workspace, workspace_bytes, st);
   }
   if (rc != IMQ_ERR_UNSUPPORTED) return rc;
-  rc = imq::gemm_wkd(4, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
-                     z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
-  if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  if (!imq::generic_first(M, N, K_pad)) {
+    rc = imq::gemm_wkd(4, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                       z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
+    if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  }
   return imq::generic_gemv<4>(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g,
                               s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb,
                               y_row_stride, st);
@@ -345,7 +362,7 @@ extern "C" int imq_linear_w2(const void* x, int64_t x_row_stride, int64_t M, int
   const uint16_t* xb = (const uint16_t*)x;
   uint16_t* yb = (uint16_t*)y;
   const uint8_t* q = (const uint8_t*)qweight;
-  if (imq::folded_first(2, M, K_pad)) {
+  if (imq::folded_first(2, M, N, K_pad)) {
     rc = imq::gemm_wkd(2, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
                        z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
     if (rc != IMQ_ERR_UNSUPPORTED) return rc;
@@ -360,9 +377,11 @@ extern "C" int imq_linear_w2(const void* x, int64_t x_row_stride, int64_t M, int
                       workspace, workspace_bytes, st);
   }
   if (rc != IMQ_ERR_UNSUPPORTED) return rc;
-  rc = imq::gemm_wkd(2, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
-                     z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
-  if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  if (!imq::generic_first(M, N, K_pad)) {
+    rc = imq::gemm_wkd(2, xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g, s_dtype, zero,
+                       z_stride_n, z_stride_g, z_dtype, N, group_size, yb, y_row_stride, st);
+    if (rc != IMQ_ERR_UNSUPPORTED) return rc;
+  }
   return imq::generic_gemv<2>(xb, x_row_stride, M, K_pad, q, q_row_stride, scale, s_stride_n, s_stride_g,
                               s_dtype, zero, z_stride_n, z_stride_g, z_dtype, N, group_size, yb,
                               y_row_stride, st);

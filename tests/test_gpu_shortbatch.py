@@ -158,7 +158,7 @@ def test_int8_decode_rows_split_k_at_any_k(dev, M, N, K):
         assert torch.equal(y1, y) and bool((ws[need:] == 0x5a).all()) and bool((ws != 0x5a).any())
 
 
-@pytest.mark.parametrize("M,N,K,bits,G", [(6, 37, 320, 4, 64), (6, 70, 192, 2, 64), (6, 33, 1152, 2, 128), (12, 100, 2944, 4, 128)])
+@pytest.mark.parametrize("M,N,K,bits,G", [(6, 37, 320, 4, 64), (8, 70, 192, 2, 64), (6, 33, 1152, 2, 128), (12, 100, 6272, 4, 128)])
 def test_non_finite_activations_at_odd_k(dev, M, N, K, bits, G):
     """Decode rows of odd K with infinite and NaN activations: an output is the sum of its own products (q - z) s x, so
     one infinity gives an infinity of that product's sign (NaN at a zero weight), opposite ones and NaN give NaN, and
@@ -218,3 +218,22 @@ def test_short_k_and_wide_n_are_other_kernels_calls(dev, M, N, K, bits, G):
         return _check(ops.linear_w8(xt, torch.from_numpy(q).to(dev), C.to_torch(s, "bf16", dev)), x, q.astype(np.float64) * s)
     q, s, z, w = _group_case(dev, bits, N, K, G, "bf16", "bf16", seed=M + N + K)
     _check((ops.linear_w4 if bits == 4 else ops.linear_w2)(xt, q, G, (s, z)), x, w)
+
+
+@pytest.mark.parametrize("M,N,K,bits,G", [(1, 40, 64, 4, 64), (16, 2048, 64, 2, 64), (12, 33, 128, 2, 64), (13, 33, 128, 2, 64), (2, 100, 320, 4, 64),
+                                          (7, 64, 11136, 4, 128), (6, 64, 11136, 4, 128), (16, 33, 2304, 2, 64), (9, 4128, 2944, 4, 128), (9, 4096, 2944, 4, 128), (5, 48, 6912, 2, 64), (4, 33, 12096, 2, 64)])
+def test_decode_rows_on_both_sides_of_the_folded_forms_lines(dev, M, N, K, bits, G):
+    """Decode rows of odd K at the lines between the generic, skinny and folded kernels: no weight is rounded on any
+    side, so each matches the exact product."""
+    from infinitemodel_amd import ops
+    r = C.rng(M + N + K)
+    codes = r.integers(0, 1 << bits, (N, K), dtype=np.uint8)
+    q = np.zeros((N, K * bits // 8), np.uint8)
+    for i in range(8 // bits):
+        q |= codes[:, i::8 // bits] << (bits * i)
+    s = oq.round_to(r.uniform(0.005, 0.05, (N, K // G)).astype(np.float32), "bf16")
+    z = oq.round_to(r.uniform(0, (1 << bits) - 1, (N, K // G)).astype(np.float32), "bf16")
+    x = C.bf16_normal(C.rng(M), (M, K))
+    y = (ops.linear_w4 if bits == 4 else ops.linear_w2)(C.to_torch(x, "bf16", dev), C.u8(q, dev), G,
+                                                       (C.to_torch(s, "bf16", dev), C.to_torch(z, "bf16", dev)))
+    _check(y, x, oq.dequant_exact(codes, s, z, G, K))
