@@ -666,13 +666,14 @@ double gemm_lds_us(int bits, int64_t M, int64_t N, int64_t K, int cus, bool plan
 }
 
 // Workspace bytes a split-K launch of this shape may use (0: no launch splits K): the largest need of the GEMMs'
-// plans over the formats and dtypes they take (up to 16 rows the int8 short-batch plan alone).
-int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+// plans over the formats and dtypes they take (up to 16 rows the int8 short-batch plan alone); pair16: of scale and zero
+// in one 16-bit dtype, which gemm_rb does not take.
+int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool pair16) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
   const int cus = device_info().cus;
   if (M <= 16) return wk_workspace_bytes(M, N, K, cus);
   const int64_t lds = use_big(M) ? split_bytes<CfgBig>(M, N, K, cus) : split_bytes<CfgSmall>(M, N, K, cus);
-  const int64_t rb = rb_workspace_bytes(4, M, N, K, cus);
+  const int64_t rb = pair16 ? 0 : rb_workspace_bytes(4, M, N, K, cus);
   const int64_t wk = wk_workspace_bytes(M, N, K, cus);
   const int64_t rbm = rbm_workspace_bytes(M, N, K, cus);
   return std::max(std::max(lds, rb), std::max(wk, rbm));

@@ -33,7 +33,7 @@ int gemm_wq(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, cons
 int gemm_wq_tiled(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, const uint8_t* q, const void* sc,
                   int64_t ssn, int64_t ssg, int sdt, const void* zr, int64_t szn, int64_t szg, int zdt, int64_t N,
                   uint16_t* y, int64_t sym, void* ws, int64_t wsb, hipStream_t st);
-int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool pair16);
 int decode_plan_query(int kind, const int64_t* in, int64_t* out);
 void gemm_plan_query(int64_t M, int64_t N, int64_t K, int cus, int64_t* out);
 void wk_plan_query(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, int max_lds, int64_t* out);
@@ -94,7 +94,7 @@ extern "C" int imq_abi_version(void) { return IMQ_ABI_VERSION; }
 
 extern "C" int64_t imq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K_pad) {
   if (M < 0 || N < 0 || K_pad <= 0) return -1;
-  const int64_t g = imq::gemm_workspace_bytes(M, N, K_pad);
+  const int64_t g = imq::gemm_workspace_bytes(M, N, K_pad, false);
   const int64_t d = imq::ksplit_workspace_bytes(M, N, K_pad);
   const int64_t d2 = imq::ksplit2_workspace_bytes(M, N, K_pad);
   const int64_t gd = g > d ? g : d;
@@ -107,7 +107,7 @@ extern "C" int64_t imq_linear_w4_workspace_bytes(int64_t M, int64_t K_pad, int64
                                                  int64_t z_stride_g, int z_dtype) {
   if (M < 0 || N < 0 || K_pad <= 0 || group_size <= 0 || K_pad % group_size) return -1;
   if (M == 0 || N == 0) return 0;
-  if (M > 16) return imq::gemm_workspace_bytes(M, N, K_pad);
+  if (M > 16) return imq::gemm_workspace_bytes(M, N, K_pad, s_dtype == z_dtype && s_dtype != IMQ_DT_FP32);
   return imq::w4_decode_workspace_bytes(M, K_pad, group_size, N, q_row_stride, x_row_stride, s_stride_n, s_stride_g,
                                         z_stride_n, z_stride_g, s_dtype, z_dtype);
 }
@@ -123,7 +123,7 @@ extern "C" int imq_launch_plan(int kind, const int64_t* in, int64_t* out) {
     return IMQ_OK;
   }
   if (kind == IMQ_PLAN_GEMM_RB) {
-    if (cus <= 0) return IMQ_OK;
+    if (cus <= 0 || in[7] == IMQ_DT_BF16 || in[7] == IMQ_DT_FP16) return IMQ_OK;   // gemm_rbm's
     imq::rb_plan_query(G == 0 ? 8 : 4, M, N, K, G == 0 ? 128 : G, cus, out);
     return IMQ_OK;
   }
