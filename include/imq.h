@@ -318,8 +318,9 @@ int imq_gptq_int2_solve(float* W, int64_t ldw, int64_t out, int64_t in_f, const 
  *     IMQ_PLAN_W8_LINE    int8 line kernel: p1 line-steps per wave, p2 waves
  *     IMQ_PLAN_GEMM       LDS-dequant GEMM: p1 tile rows, p2 tile columns, p3 K splits
  *     IMQ_PLAN_GEMM_RB    register-B GEMM of fp32 scale and zero (M > 512; int4 with group_size, int8 when it
- *                         is 0): p1 32-row blocks per wave, p2 K splits. Mixed dtypes have the same plan;
- *                         bf16 and fp16 alike are IMQ_PLAN_GEMM_RBM's
+ *                         is 0) or of mixed dtypes: p1 32-row blocks per wave, p2 K splits. The plan of the
+ *                         shape, whatever s_dtype says: calls of bf16 or fp16 scale and zero alike are
+ *                         IMQ_PLAN_GEMM_RBM's
  *     IMQ_PLAN_GEMM_WK    short-batch GEMM (16 < M <= 64, int8 from 5; the format by q_row_stride, dense rows):
  *                         p1 32-column blocks per workgroup, p2 K ranges
  *     IMQ_PLAN_GEMM_RBM   register-B GEMM at any tile height (M > 64, bf16 / fp16 scale and zero

@@ -123,7 +123,7 @@ extern "C" int imq_launch_plan(int kind, const int64_t* in, int64_t* out) {
     return IMQ_OK;
   }
   if (kind == IMQ_PLAN_GEMM_RB) {
-    if (cus <= 0 || in[7] == IMQ_DT_BF16 || in[7] == IMQ_DT_FP16) return IMQ_OK;   // gemm_rbm's
+    if (cus <= 0) return IMQ_OK;
     imq::rb_plan_query(G == 0 ? 8 : 4, M, N, K, G == 0 ? 128 : G, cus, out);
     return IMQ_OK;
   }
