@@ -135,8 +135,8 @@ int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int64_t K_pad,
  * dense: N * row_bytes bytes). imq_linear_w4_tiled / imq_linear_w2_tiled take the arguments of
  * imq_linear_w4 / imq_linear_w2 and give the same results, with qweight tiled (q_row_stride =
  * row_bytes; int4 groups of 128, int2 groups of 64); the decode line / wave-split / K-split kernels
- * and the prefill GEMMs read the layout, and a call none of them takes returns
- * IMQ_ERR_UNSUPPORTED. They serve the reference operators of imq_linear_w4 / _w2
+ * and the prefill GEMMs read the layout, and a call none of them takes (past 16 rows also one whose
+ * scale and zero differ in dtype) returns IMQ_ERR_UNSUPPORTED. They serve the reference operators of imq_linear_w4 / _w2
  * (_w4a16_triton_op, worker_quant.py:1079-1225; _w2a16_triton_op, 1775-1918) for modules whose
  * weights were tiled once at load. */
 int imq_line_tile(const void* q_rows, int64_t q_row_stride, int64_t N, int64_t row_bytes, void* q_tiled,

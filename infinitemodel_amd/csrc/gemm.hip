@@ -760,6 +760,7 @@ int gemm_wq_any(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, 
                 bool tiled) {
   if (M <= 0 || N <= 0) return IMQ_OK;
   if (K % 64 != 0 || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff) return IMQ_ERR_UNSUPPORTED;
+  if (tiled && bits != 8 && sdt != zdt) return IMQ_ERR_UNSUPPORTED;   // line-tiled weights: scale and zero of one dtype
   int gsh = 0;
   if (bits != 8) {
     if (G < 32 || (G & (G - 1)) != 0) return IMQ_ERR_UNSUPPORTED;   // power-of-two groups >= 32
@@ -784,8 +785,7 @@ int gemm_wq_any(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, 
   }
   GemmArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, (int)N, gsh, y, sym, 0, 0, 1, 0,
              nullptr};
-  if (tiled) {   // line-tiled weights: scale and zero of one dtype (int8: the scale's)
-    if (sdt != zdt && bits != 8) return IMQ_ERR_UNSUPPORTED;
+  if (tiled) {
     if (bits == 8) {
       switch (sdt) {
         case IMQ_DT_BF16: return launch_gemm<8, IMQ_DT_BF16, IMQ_DT_BF16, true>(a, ws, wsb, st);

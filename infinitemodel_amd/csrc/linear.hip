@@ -197,8 +197,8 @@ extern "C" int imq_linear_w4(const void* x, int64_t x_row_stride, int64_t M, int
 // int4 weights in the line-tiled layout: the arguments and results of imq_linear_w4. The layout
 // permutes 16-byte pieces within each 16-row tile (N a multiple of 16, dense rows of K_pad / 2
 // bytes, K_pad a multiple of 256, groups of 128); the kernels that read it are the decode line,
-// wave-split and K-split kernels and the two prefill GEMMs. A call none of them takes returns
-// IMQ_ERR_UNSUPPORTED: no row-layout kernel may read these bytes.
+// wave-split and K-split kernels and the prefill GEMMs. A call none of them takes (past 16 rows also one whose scale
+// and zero differ in dtype) returns IMQ_ERR_UNSUPPORTED: no row-layout kernel may read these bytes.
 extern "C" int imq_linear_w4_tiled(const void* x, int64_t x_row_stride, int64_t M, int64_t K_pad,
                                    const void* qweight, int64_t q_row_stride, const void* scale,
                                    int64_t s_stride_n, int64_t s_stride_g, int s_dtype, const void* zero,
@@ -224,7 +224,7 @@ extern "C" int imq_linear_w4_tiled(const void* x, int64_t x_row_stride, int64_t 
 
 // int2 weights in the line-tiled layout: the arguments and results of imq_linear_w2 (N a multiple of
 // 16, dense rows of K_pad / 4 bytes, K_pad a multiple of 512, groups of 64); the decode line and
-// K-split kernels and the LDS-dequant GEMM read it, other calls return IMQ_ERR_UNSUPPORTED.
+// K-split kernels and the prefill GEMMs read it, other calls return IMQ_ERR_UNSUPPORTED.
 extern "C" int imq_linear_w2_tiled(const void* x, int64_t x_row_stride, int64_t M, int64_t K_pad,
                                    const void* qweight, int64_t q_row_stride, const void* scale,
                                    int64_t s_stride_n, int64_t s_stride_g, int s_dtype, const void* zero,

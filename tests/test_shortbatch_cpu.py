@@ -1,6 +1,8 @@
 """The short-batch GEMM's plan and address arithmetic (csrc/gemm_wk.h), restated: every K step is taken by
 one wave of one range, every operand read lies inside its buffer, the line-tiled offsets are the
 layout's definition, the staged scale groups cover the steps that use them, and the LDS regions fit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -125,3 +127,15 @@ def test_short_k_and_wide_n_decline():
         assert _plan(bits, 64, 65536, 512, G) is None and _plan(bits, 64, 65536, 2048, G) is not None
     assert _plan(8, 8, 65536, 192, 0) is None and _plan(8, 9, 65536, 192, 0) is not None
     assert _plan(8, 16, 20000, 64, 0) is None and _plan(8, 16, 16384, 64, 0) is not None
+
+
+@pytest.mark.parametrize("bits,M", [(4, 17), (4, 32), (4, 64), (4, 200), (4, 1024), (2, 17), (2, 64), (2, 1024)])
+@pytest.mark.parametrize("dts", [(0, 1), (0, 2), (1, 0), (2, 0)])
+def test_line_tiled_weights_of_mixed_dtypes_are_refused(bits, M, dts):
+    """Past 16 rows a line-tiled call's scale and zero have one dtype, whichever GEMM would take its row count. Refused
+    before any launch: the pointers are never read."""
+    L, K, N, G = _lib.lib(), 1024, 64, 128 if bits == 4 else 64
+    p = ctypes.c_void_p(1 << 20)
+    rc = (L.imq_linear_w4_tiled if bits == 4 else L.imq_linear_w2_tiled)(
+        p, K, M, K, p, K * bits // 8, p, K // G, 1, dts[0], p, K // G, 1, dts[1], N, G, p, N, None, 0, None)
+    assert rc == _lib.IMQ_ERR_UNSUPPORTED
