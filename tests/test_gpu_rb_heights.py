@@ -17,6 +17,20 @@ CASES = [(513, 1008, 1024, 4, 128, "bf16"), (777, 8200, 256, 4, 64, "fp16"), (10
          (1010, 14336, 256, 4, 256, "fp16"), (601, 1000, 256, 2, 64, "fp16"), (777, 2000, 2048, 2, 64, "bf16"),
          (1010, 8200, 512, 2, 32, "fp16"), (601, 16400, 512, 2, 64, "bf16"), (150, 1008, 1024, 8, 0, "fp16"),
          (1010, 14336, 256, 8, 0, "bf16")]
+# the heights those leave out of a format or a layout
+CASES += [(150, 16, 1024, 4, 128, "fp16"), (1537, 4000, 256, 4, 128, "fp16"), (1537, 5008, 256, 4, 128, "bf16"),
+          (777, 1500, 4096, 4, 64, "fp16"), (1010, 10000, 256, 4, 128, "fp16"), (1010, 11008, 256, 4, 128, "fp16"),
+          (700, 16400, 256, 4, 128, "bf16"),
+          (150, 16, 1024, 2, 64, "bf16"), (777, 8208, 512, 2, 64, "fp16"), (1537, 5008, 512, 2, 64, "bf16"),
+          (1010, 10000, 512, 2, 64, "fp16"), (1010, 11008, 512, 2, 64, "fp16"), (700, 16400, 1024, 2, 64, "bf16"),
+          (200, 8208, 4096, 2, 64, "bf16"),
+          (150, 16, 256, 8, 0, "bf16"), (1537, 4000, 256, 8, 0, "fp16"), (1537, 5008, 256, 8, 0, "bf16"),
+          (300, 8208, 2048, 8, 0, "fp16"), (1010, 10000, 256, 8, 0, "fp16"), (1010, 11008, 256, 8, 0, "bf16"),
+          (700, 16400, 256, 8, 0, "fp16")]
+
+
+def _tiles(N, K, bits, G):
+    return N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == {4: 128, 2: 64, 8: 0}[bits]
 
 
 @pytest.mark.parametrize("M,N,K,bits,G,dt", CASES)
@@ -34,13 +48,13 @@ def test_tile_heights(dev, M, N, K, bits, G, dt):
         qt, st = torch.from_numpy(q).to(dev), C.to_torch(s, dt, dev)
         y = ops.linear_w8(xt, qt, st)
         _check(y, x, q.astype(np.float64) * s)
-        if N % 16 == 0 and K % 128 == 0:
+        if _tiles(N, K, bits, G):
             assert torch.equal(ops.linear_w8_tiled(xt, ops.line_tile(qt), st), y)
         return
     q, s, z, w = _group_case(dev, bits, N, K, G, dt, dt, seed=N + K)
     y = (ops.linear_w4 if bits == 4 else ops.linear_w2)(xt, q, G, (s, z))
     _check(y, x, w)
-    if N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == (128 if bits == 4 else 64):
+    if _tiles(N, K, bits, G):
         f = ops.linear_w4_tiled if bits == 4 else ops.linear_w2_tiled
         assert torch.equal(f(xt, ops.line_tile(q), G, (s, z)), y)
 
@@ -48,3 +62,8 @@ def test_tile_heights(dev, M, N, K, bits, G, dt):
 def test_every_height_is_covered():
     heights = {_lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, G, N, sqn=K * b // 8)[0] for M, N, K, b, G, _ in CASES}
     assert heights == {3, 4, 5, 6, 7, 8}
+    for bits in (4, 2, 8):                                     # of each format, in each layout
+        of = lambda cases: {_lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, G, N, sqn=K * b // 8)[0]   # noqa: E731
+                            for M, N, K, b, G, _ in cases if b == bits}
+        assert of(CASES) == {3, 4, 5, 6, 7, 8}, bits
+        assert of([c for c in CASES if _tiles(c[1], c[2], c[3], c[4])]) == {3, 4, 5, 6, 7, 8}, bits

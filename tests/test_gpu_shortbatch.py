@@ -38,7 +38,26 @@ CASES = [
     (64, 2944, 768, 4, 128, "fp32", "fp32"), (48, 4096, 4096, 4, 128, "bf16", "bf16"), (31, 257, 14336, 4, 256, "fp16", "fp16"),
     (20, 30000, 512, 4, 128, "bf16", "bf16"), (17, 96, 448, 2, 64, "fp16", "fp16"), (64, 1000, 8192, 2, 64, "fp16", "fp16"),
     (32, 16400, 1024, 2, 32, "bf16", "fp16"), (40, 300, 28672, 2, 128, "fp32", "bf16"),
+    # each form on line-tiled weights too
+    (17, 48, 512, 4, 128, "fp16", "fp16"), (32, 14336, 512, 4, 128, "bf16", "bf16"), (21, 2000, 8192, 4, 128, "fp16", "fp16"),
+    (17, 48, 512, 2, 64, "bf16", "bf16"), (30, 48, 4096, 2, 64, "fp16", "fp16"), (32, 14336, 512, 2, 64, "fp32", "fp32"),
+    (18, 30000, 512, 2, 64, "bf16", "bf16"), (33, 48, 512, 2, 64, "fp16", "fp16"), (64, 2000, 8192, 2, 64, "bf16", "bf16"),
 ]
+
+
+def test_every_form_is_covered():
+    """int4 and int2: one or two blocks of 32 rows with each count of column blocks, in both layouts."""
+    from infinitemodel_amd import _lib
+    want = {(1, 1), (1, 2), (1, 4), (2, 1), (2, 2)}
+    for b in (4, 2):
+        of = lambda M, N, K, G: (-(-M // 32), _lib.launch_plan(_lib.IMQ_PLAN_GEMM_WK, M, K, G, N, sqn=K * b // 8)[0])   # noqa: E731
+        mine = [c for c in CASES if c[3] == b]
+        assert {of(M, N, K, G) for M, N, K, _, G, _, _ in mine} == want
+        assert {of(M, N, K, G) for M, N, K, _, G, s, z in mine if s == z and _tiles(N, K, b, G)} == want
+
+
+def _tiles(N, K, bits, G):
+    return N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == (128 if bits == 4 else 64)
 
 
 @pytest.mark.parametrize("M,N,K,bits,G,sdt,zdt", CASES)
@@ -58,7 +77,7 @@ def test_group_formats_match_the_oracle(dev, M, N, K, bits, G, sdt, zdt):
     out = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device=dev)
     op(xw[:, 8:8 + K], qw[:, :q.shape[1]], G, (s.t().contiguous().t(), z.t().contiguous().t()), out=out[:, :N])
     assert torch.equal(out[:, :N], y) and bool((out[:, N:] == 7).all())
-    if N % 16 == 0 and (K * bits // 8) % 128 == 0 and G == (128 if bits == 4 else 64) and sdt == zdt:
+    if _tiles(N, K, bits, G) and sdt == zdt:
         tiled = ops.linear_w4_tiled if bits == 4 else ops.linear_w2_tiled
         assert torch.equal(tiled(C.to_torch(x, "bf16", dev), ops.line_tile(q), G, (s, z)), y)
 
