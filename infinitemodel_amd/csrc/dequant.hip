@@ -43,7 +43,11 @@ IMQ_DEV void dequant_values(const float* c, float s, float z, uint32_t* o) {
       o[i] = __float_as_uint(a * s);
       o[i + 1] = __float_as_uint(b * s);
     } else {
-      o[i / 2] = pack2<ODT, HW>(a * s, b * s);
+      a *= s;
+      b *= s;
+      // fp16: a product and its conversion would become one v_fma_mixlo_f16 that adds +0, and a zero its sign
+      if constexpr (ODT == IMQ_DT_FP16) asm("" : "+v"(a), "+v"(b));
+      o[i / 2] = pack2<ODT, HW>(a, b);
     }
   }
 }

@@ -90,3 +90,24 @@ def test_int8_packer_and_dequant_edges(dev, dt, N, K, wide):
         odd = torch.zeros(N, K + 3, dtype=torch.int8, device=dev)[:, 1:1 + K]
         odd.copy_(qd)
         assert _same(ops.dequant_w8(odd, sd, _tdt(odt)), ref), odt
+
+
+@pytest.mark.parametrize("sdt", DTS)
+def test_zero_products_keep_their_sign(dev, sdt):
+    """Scales of zero (an fp16 group whose step underflows) and of either sign: a zero product has the sign of its
+    factors, as torch's has, in every dtype written."""
+    import torch
+    from infinitemodel_amd import ops, worker_quant as wq
+    g = torch.Generator().manual_seed(5)
+    N, K = 24, 264
+    s = torch.tensor([0.0, -0.0, 0.01, -0.01]).repeat(N // 4)[:, None].to(_tdt(sdt))
+    q8 = torch.randint(-3, 4, (N, K), generator=g).to(torch.int8)
+    for odt in DTS:
+        assert _same(ops.dequant_w8(q8.to(dev), s.to(dev), _tdt(odt)), q8.to(_tdt(odt)) * s), odt
+    for bits, G, f in ((4, 64, ops.dequant_w4), (2, 64, ops.dequant_w2)):
+        Kp = 320
+        q = torch.randint(0, 256, (N, Kp * bits // 8), generator=g, dtype=torch.uint8)
+        sg, z = s.expand(N, Kp // G).contiguous(), torch.randint(0, 4, (N, Kp // G), generator=g).to(_tdt(sdt))
+        for odt in DTS:
+            ref = wq._dequant_g_torch(q, sg, z, K, G, _tdt(odt), bits)
+            assert _same(f(q.to(dev), sg.to(dev), z.to(dev), K, G, _tdt(odt)), ref), (bits, odt)
