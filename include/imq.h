@@ -324,7 +324,8 @@ int imq_gptq_int2_solve(float* W, int64_t ldw, int64_t out, int64_t in_f, const 
  *     IMQ_PLAN_GEMM_WK    short-batch GEMM (16 < M <= 64, int8 from 5; the format by q_row_stride, dense rows):
  *                         p1 32-column blocks per workgroup, p2 K ranges
  *     IMQ_PLAN_GEMM_RBM   register-B GEMM at any tile height (M > 64, bf16 / fp16 scale and zero
- *                         alike; the format by q_row_stride, dense rows): p1 32-row blocks, p2 K splits
+ *                         alike; the format by q_row_stride, dense rows): p1 32-row blocks (int4 and int2 in
+ *                         rows may run taller ones where the tiles outnumber the CUs), p2 K splits
  * Returns IMQ_OK, or IMQ_ERR_INVALID for an unknown kind or a null pointer. */
 #define IMQ_PLAN_W4_LINE 1
 #define IMQ_PLAN_W4_KSPLIT 2

@@ -73,6 +73,30 @@ double short_us(int bits, int64_t M, int64_t N, int64_t K, int cus, const RbmPla
   return 0.8 + rounds * t + (p.splits > 1 ? 1 + 1.15e-6 * p.splits * M * N : 0);
 }
 
+// The tile height a row-layout int4 or int2 call runs at, its splits kept (so its sums are the line-tiled call's bit
+// for bit). A K step of such a weight is 32 or 16 bytes of each row, so a 128-byte line is read over 4 or 8 steps, and two
+// workgroups to a CU drift apart by more steps than the L2 holds: up to 400 workgroups 1.22 times rbm_plan's estimate,
+// up to 512 1.55, past that 1.35 (means of 180 calls; line-tiled 1.0 to 1.1). us at 241 rows, three 96-row tiles against
+// one of 256: int4 11648 -> 21440 360 / 181, 6848 -> 36480 345 / 200.
+int rows_height(int64_t M, int64_t N, int cus, const RbmPlan& p) {
+  const int64_t blocks = imq_cdiv(M, 32), cols = imq_cdiv(N, 256), rt0 = imq_cdiv(blocks, 8);
+  if (p.ib > 4 || imq_cdiv(blocks, p.ib) * cols * p.splits <= cus) return p.ib;
+  double best = 0;
+  int height = p.ib;
+  for (int64_t rt = rt0; rt <= 3 * rt0; ++rt) {
+    const int ib = (int)imq_cdiv(blocks, rt);
+    if (ib < 3) break;
+    const int64_t W = imq_cdiv(blocks, ib) * cols * p.splits;
+    const double pair = 2 * 0.89 * (5 * W <= 8 * cus ? 1.22 : W <= 2 * cus ? 1.55 : 1.35);
+    const double us = (0.46 + 0.163 * ib) * (W <= cus ? 1 : ib <= 4 ? pair * imq_cdiv(W, 2 * cus) : (double)imq_cdiv(W, cus));
+    if (best == 0 || us < best) {
+      best = us;
+      height = ib;
+    }
+  }
+  return height;
+}
+
 // Whether this GEMM takes a call, the LDS-dequant GEMM the rest. us, LDS-dequant against this kernel, where each side
 // of a line was wrong before it: 200 rows, 64 -> 152064 int4 31 / 39 and 448 -> 100000 int4 at 512 rows 87 / 106; int8
 // at 96 rows, 1024 -> 4096 13.0 / 13.9 (8 steps a range); int2 at 1024 rows, 64 -> 152064 117 / 162.
@@ -137,6 +161,7 @@ int gemm_rbm(int bits, const uint16_t* x, int64_t sxm, int64_t M, int64_t K, con
   if (p.splits > 1 && (!ws || wsb < 4 * p.splits * M * N || ((uintptr_t)ws & 15)))
     if (!rbm_takes(bits, M, N, K, G, cus, false, &p)) return IMQ_ERR_UNSUPPORTED;
   RbArgs a{x, sxm, (int)M, (int)K, q, sqn, sc, ssn, ssg, zr, szn, szg, (int)N, gsh, y, sym, 0, 0, 1, 0, nullptr};
+  if (bits != 8 && !tiled) p.ib = rows_height(M, N, cus, p);
   if (bits == 4) return rbm_run4(a, p, sdt, tiled, ws, st);
   if (bits == 2) return rbm_run2(a, p, sdt, tiled, ws, st);
   return rbm_run8(a, p, sdt, tiled, ws, st);

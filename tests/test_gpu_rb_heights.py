@@ -67,3 +67,26 @@ def test_every_height_is_covered():
                             for M, N, K, b, G, _ in cases if b == bits}
         assert of(CASES) == {3, 4, 5, 6, 7, 8}, bits
         assert of([c for c in CASES if _tiles(c[1], c[2], c[3], c[4])]) == {3, 4, 5, 6, 7, 8}, bits
+
+
+@pytest.mark.parametrize("M,N,K,bits,G", [(241, 36480, 768, 4, 128), (241, 21440, 11776, 4, 128), (228, 38656, 1024, 2, 64)])
+def test_rows_past_the_cus_run_taller_tiles(dev, M, N, K, bits, G):
+    """Row-layout int4 and int2 calls whose short tiles outnumber the CUs run at another height than line-tiled ones, with
+    the same splits: the same bits."""
+    import torch
+    from infinitemodel_amd import ops
+    plan = _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, G, N, sqn=K * bits // 8)
+    assert plan is not None and plan[0] <= 4 and -(-M // (32 * plan[0])) * -(-N // 256) * plan[1] > 256
+    g = torch.Generator(device=dev).manual_seed(M)
+    q = torch.randint(0, 256, (N, K * bits // 8), dtype=torch.uint8, device=dev, generator=g)
+    s = (torch.rand(N, K // G, device=dev, generator=g) * 0.02 + 0.001).to(torch.bfloat16)
+    z = torch.randint(0, 1 << bits, (N, K // G), device=dev, generator=g).to(torch.bfloat16)
+    x = torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16)
+    op, tiled, deq = (ops.linear_w4, ops.linear_w4_tiled, ops.dequant_w4) if bits == 4 else (ops.linear_w2, ops.linear_w2_tiled, ops.dequant_w2)
+    y = op(x, q, G, (s, z))
+    assert torch.equal(tiled(x, ops.line_tile(q), G, (s, z)), y)
+    rows = torch.cat([torch.arange(64), torch.arange(N - 64, N)]).to(dev)
+    w = deq(q[rows].contiguous(), s[rows].contiguous(), z[rows].contiguous(), K, G, torch.bfloat16)
+    ref = x.cpu().double() @ w.cpu().double().T
+    err = (y[:, rows].cpu().double() - ref).abs().max() / ref.pow(2).mean().sqrt()
+    assert err < 2.0 ** -8 * 5       # the output's own rounding, half a unit of 2^-8 at values up to 5 to 6 standard deviations
