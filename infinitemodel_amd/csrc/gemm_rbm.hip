@@ -105,18 +105,24 @@ bool rbm_takes(int bits, int64_t M, int64_t N, int64_t K, int64_t G, int cus, bo
   if (bits != 8 && (G < 32 || (G & (G - 1)) != 0)) return false;
   const double us = rbm_plan(bits, M, N, K, cus, planes, p);
   if (us <= 0) return false;
+  const double ratio = short_us(bits, M, N, K, cus, *p) / gemm_lds_us(bits, M, N, K, cus, planes);
   if (M > 512) {
-    // int2 of short K and tiles for more than half of 256 CUs: the fixed cost decides. int4 and int8 have had a
-    // register-B form above 512 rows throughout, and smaller grids differ by a microsecond at most.
-    if (bits != 2 || K > 512 || imq_cdiv(M, 32 * p->ib) * imq_cdiv(N, 256) <= 128) return true;
-    return short_us(bits, M, N, K, cus, *p) < gemm_lds_us(bits, M, N, K, cus, planes);
+    // int2 of short K and tiles for more than half of 256 CUs, or of few columns and K up to 4096: the fixed cost
+    // decides (2048 -> 1024 at 985 rows 19.6 / 23.7). int4 and int8 have had a register-B form above 512 rows
+    // throughout, and smaller grids differ by a microsecond at most.
+    if (bits != 2) return true;
+    if (K <= 512) return imq_cdiv(M, 32 * p->ib) * imq_cdiv(N, 256) <= 128 || ratio < 1.0;
+    return K > 4096 || N > 1024 || ratio < 0.95;
   }
   // up to 512 rows the LDS-dequant GEMM keeps the calls the model puts within its own spread, and short ranges where
   // its fixed cost is the smaller (by more than the two fits' spread where K is only short for its splits: at 12%
   // modelled, 4 to 13% measured; below that the two are within 5% of each other)
   if (us >= 0.96 * lds_us(M, N, K, cus, planes)) return false;
+  // int8 of K up to 320, or of one 128-row tile and K up to 1024, where both are within the fits' spread: the LDS-dequant
+  // GEMM unless 5% is modelled (192 -> 12352 at 132 rows 8.9 / 10.1, 896 -> 256 at 79 rows 13.7 / 14.9)
+  if (bits == 8 && (K <= 320 || (M <= 128 && K <= 1024))) return ratio < 0.95;
   if (imq_cdiv(K / RB_BK, p->splits) > 12) return true;
-  return short_us(bits, M, N, K, cus, *p) < (K <= 512 ? 1.0 : 1.12) * gemm_lds_us(bits, M, N, K, cus, planes);
+  return ratio < (K <= 512 ? 1.0 : 1.12);
 }
 
 }  // namespace

@@ -24,7 +24,7 @@ CASES += [(150, 16, 1024, 4, 128, "fp16"), (1537, 4000, 256, 4, 128, "fp16"), (1
           (150, 16, 1024, 2, 64, "bf16"), (777, 8208, 512, 2, 64, "fp16"), (1537, 5008, 512, 2, 64, "bf16"),
           (1010, 10000, 512, 2, 64, "fp16"), (1010, 11008, 512, 2, 64, "fp16"), (700, 16400, 1024, 2, 64, "bf16"),
           (200, 8208, 4096, 2, 64, "bf16"),
-          (150, 16, 256, 8, 0, "bf16"), (1537, 4000, 256, 8, 0, "fp16"), (1537, 5008, 256, 8, 0, "bf16"),
+          (150, 16, 384, 8, 0, "bf16"), (1537, 4000, 256, 8, 0, "fp16"), (1537, 5008, 256, 8, 0, "bf16"),
           (300, 8208, 2048, 8, 0, "fp16"), (1010, 10000, 256, 8, 0, "fp16"), (1010, 11008, 256, 8, 0, "bf16"),
           (700, 16400, 256, 8, 0, "fp16")]
 

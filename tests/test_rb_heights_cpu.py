@@ -44,6 +44,15 @@ def test_short_k_ranges_decline():
     assert plan(4, 200, 28672, 4096)[:2] == (7, 2) and plan(8, 512, 14336, 4096)[:2] == (4, 1) and plan(8, 512, 4096, 14336)[:2] == (4, 4)
 
 
+def test_few_columns_of_int2_and_short_k_of_int8_decline():
+    """Where the LDS-dequant GEMM measured faster; int4 of those columns, int2 of longer K and int8 past them stay."""
+    plan = lambda b, M, N, K: _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, M, K, 0 if b == 8 else 64, N, sqn=K * b // 8)   # noqa: E731
+    assert all(plan(2, M, 1024, 2048) is None and plan(4, M, 1024, 2048) is not None for M in (872, 985, 1170))
+    assert plan(2, 985, 1024, 8192) is not None and plan(2, 985, 2048, 4096) is not None
+    assert plan(8, 132, 12352, 192) is None and plan(8, 79, 256, 896) is None
+    assert plan(8, 256, 14336, 640) is not None and plan(8, 200, 14336, 1024) is not None
+
+
 def test_rows_up_to_64_and_odd_k_decline():
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 64, 4096, 128, 4096, sqn=2048) is None
     assert _lib.launch_plan(_lib.IMQ_PLAN_GEMM_RBM, 600, 4096 + 32, 128, 4096, sqn=2064) is None
