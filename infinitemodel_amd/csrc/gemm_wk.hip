@@ -71,8 +71,12 @@ bool wk_rows(int bits, int64_t M, int64_t N, int64_t K) {
 // 51 / 42. This form's us is a fit to graph replays of such calls (3 to 12% rms), c + rounds (f + step per K step of a
 // wave + per K / 512), with a margin where the fit runs high; from three steps a wave it has been the faster at every
 // width, and grids within the CUs differ by 2 us at most, at K = 64.
+// int8 rows 5 to 8: two-block workgroups that just outnumber the CUs run a second round nearly empty, and the skinny
+// kernel's persistent tiles are the faster while it can stage the rows: 3584 -> 18944 M = 6 / 8 18.4 / 19.5 against 21.5 / 21.8,
+// 6144 -> 16896 M = 7 39.7 against 44.0; from 1.4 rounds on 3392 -> 23393 M = 7 26.0 against 25.0.
 bool wk_worth(int bits, int64_t M, int64_t N, int64_t K, int cus, const WkPlan& p) {
   const int64_t W = imq_cdiv(N, 32 * p.jb);
+  if (M <= 8) return !(p.jb == 2 && p.splits == 1 && W > cus && 5 * W <= 7 * cus && K >= 1024 && M * K <= 48 << 10);
   if (M <= 16 || p.splits > 1 || W <= cus || K > 2 * WK_WAVES * RB_BK) return true;
   struct Cost { double c, f, step, per; };
   const bool one = p.jb == 1;

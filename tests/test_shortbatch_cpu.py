@@ -129,6 +129,14 @@ def test_short_k_and_wide_n_decline():
     assert _plan(8, 16, 20000, 64, 0) is None and _plan(8, 16, 16384, 64, 0) is not None
 
 
+def test_int8_rows_5_to_8_just_past_the_cus_decline():
+    """A second, nearly empty round of workgroups: the skinny kernel's, while it can stage the rows."""
+    for M in (5, 6, 8):
+        assert _plan(8, M, 18944, 3584, 0) is None and _plan(8, M, 16384, 3584, 0) is not None
+        assert _plan(8, M, 28672, 4096, 0) is not None and _plan(8, M, 18944, 14336, 0) is not None
+    assert _plan(8, 9, 18944, 3584, 0) is not None and _plan(8, 8, 18944, 512, 0) is not None
+
+
 @pytest.mark.parametrize("bits,M", [(4, 17), (4, 32), (4, 64), (4, 200), (4, 1024), (2, 17), (2, 64), (2, 1024)])
 @pytest.mark.parametrize("dts", [(0, 1), (0, 2), (1, 0), (2, 0)])
 def test_line_tiled_weights_of_mixed_dtypes_are_refused(bits, M, dts):
