@@ -399,7 +399,7 @@ int wk_launch(const WkArgs& a, hipStream_t st) {
 
 // The folded form: decode rows whose K no line or K-split kernel takes. us, generic kernel (one wave per row,
 // a code at a time) -> this: int2 12096 -> 1344 M = 1 / 7 / 16 113 / 221 / 385 -> 15, 3520 -> 2560 41 / 74 / 116 ->
-// 9; bound by its 24 K steps per wave in turn. One 32-column block per workgroup, 16 waves (decode shapes are short of workgroups,
+// 9; bound by its 12 K steps per wave in turn. One 32-column block per workgroup, 16 waves (decode shapes are short of workgroups,
 // not of columns), K unsplit.
 constexpr int WKD_WAVES = 16;
 template <int BITS>
