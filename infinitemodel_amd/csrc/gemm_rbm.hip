@@ -75,7 +75,8 @@ double short_us(int bits, int64_t M, int64_t N, int64_t K, int cus, const RbmPla
 
 // The tile height a row-layout int4 or int2 call runs at, its splits kept (so its sums are the line-tiled call's bit
 // for bit). A K step of such a weight is 32 or 16 bytes of each row, so a 128-byte line is read over 4 or 8 steps, and two
-// workgroups to a CU drift apart by more steps than the L2 holds: up to 400 workgroups 1.22 times rbm_plan's estimate,
+// workgroups to a CU lose it from the L2 between them (fetched, 11776 -> 21440 at 241 rows in 96-row tiles: 516 MB in rows,
+// 234 MB line-tiled, 89 MB in rows at 256-row tiles): up to 400 workgroups 1.22 times rbm_plan's estimate,
 // up to 512 1.55, past that 1.35 (means of 180 calls; line-tiled 1.0 to 1.1). us at 241 rows, three 96-row tiles against
 // one of 256: int4 11648 -> 21440 360 / 181, 6848 -> 36480 345 / 200.
 int rows_height(int64_t M, int64_t N, int cus, const RbmPlan& p) {
